@@ -10,12 +10,14 @@
 // scalar (the solver's residue) per iteration to evaluate the stopping rule.
 #include <algorithm>
 #include <cmath>
+#include <future>
 #include <vector>
 
 #include "blas1.hpp"
 #include "krylov.hpp"
 #include "segments.hpp"
 #include "spmv.hpp"
+#include "tri_strips.hpp"
 
 using namespace tnlmi;
 
@@ -54,6 +56,10 @@ struct tnlmi_preconditioner
    DeviceArray< int32_t > lridx, uridx;
    DeviceArray< double > lrval, urval, bpos;
    DeviceArray< double > xpos;  // the sync-free solve's results in position order (+ kLvThreads spare slots)
+   // the solves as a pipeline of row strips, where that is the faster form
+   // (tri_strips_build decides); mid: the upper solve's positions to the lower's
+   TriStrips lstrips, ustrips;
+   DeviceArray< int32_t > mid;
    tnlmi_matrix M{};                   // explicit: x = M b
 };
 
@@ -557,6 +563,19 @@ void upload_vec( DeviceArray< T >& d, const std::vector< T >& h, hipStream_t s )
       TNLMI_HIP( hipMemcpyAsync( d.ptr, h.data(), sizeof( T ) * h.size(), hipMemcpyHostToDevice, s ) );
 }
 
+// out[p] = pos[row[p]] (-1 where row[p] is)
+__global__ void compose_map_k( int64_t n, const int32_t* __restrict__ row, const int32_t* __restrict__ pos,
+                               int32_t* __restrict__ out )
+{
+   const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+   if( p < n )
+      out[ p ] = row[ p ] >= 0 ? pos[ row[ p ] ] : -1;
+}
+void compose_map( int64_t n, const int32_t* row, const int32_t* pos, int32_t* out, hipStream_t s )
+{
+   hipLaunchKernelGGL( compose_map_k, dim3( (unsigned) ceil_div( n, 256 ) ), dim3( 256 ), 0, s, n, row, pos, out );
+}
+
 // ILU0.hpp:12-96 (IKJ on A's pattern) on the host, as the reference does;
 // the triangular solves run on the GPU by levels.
 void ilu0_build( tnlmi_preconditioner& P, const tnlmi_matrix& A, hipStream_t s )
@@ -669,6 +688,33 @@ void ilu0_build( tnlmi_preconditioner& P, const tnlmi_matrix& A, hipStream_t s )
    };
    plan_runs( P.llev, P.lruns );
    plan_runs( P.ulev, P.uruns );
+   // what the solves by levels take: 0.65 us per level of a narrow run, a
+   // launch (6 us) per wide level, measured on 5- and 7-point grid factors
+   auto level_us = []( const std::vector< tnlmi_preconditioner::Run >& runs ) {
+      double us = 0;
+      for( const auto& R : runs )
+         us += R.narrow ? 10 + 0.65 * (double) ( R.l1 - R.l0 ) : 6.0;
+      return us;
+   };
+   const char* fenv = std::getenv( "TNLMI_ILU_FLOW" );
+   const bool flow_on = ! ( fenv && std::string( fenv ) == "0" );  // (off: no solve without barriers)
+   TriStripsPlan lplan, uplan;
+   if( flow_on ) {
+      // (the two factors' schedules at the same time)
+      auto later = std::async( std::launch::async, [ & ] {
+         return tri_strips_plan( N, lp, lc, lv, false, level_us( P.lruns ) );
+      } );
+      uplan = tri_strips_plan( N, up, uc, uv, true, level_us( P.uruns ) );
+      lplan = later.get();
+      if( lplan.strips )
+         tri_strips_upload( P.lstrips, lplan, s );
+      if( uplan.strips )
+         tri_strips_upload( P.ustrips, uplan, s );
+   }
+   if( P.lstrips.used() && P.ustrips.used() ) {
+      P.mid.allocate( P.ustrips.steps * 64 );
+      compose_map( P.ustrips.steps * 64, P.ustrips.row.ptr, P.lstrips.pos.ptr, P.mid.ptr, s );
+   }
    // the factors in level-order positions, and which narrow runs may keep
    // their recent solution entries in the LDS ring
    auto positions = [ & ]( bool upper, const std::vector< int32_t >& order, const std::vector< int64_t >& bounds,
@@ -700,8 +746,6 @@ void ilu0_build( tnlmi_preconditioner& P, const tnlmi_matrix& A, hipStream_t s )
       }
       // the sync-free solve: rows of at most kRingPre entries, every
       // dependency at most kFlowDist positions before its row
-      const char* fenv = std::getenv( "TNLMI_ILU_FLOW" );
-      const bool flow_on = ! ( fenv && std::string( fenv ) == "0" );
       for( auto& R : runs ) {
          R.flow = flow_on;
          for( int64_t p = bounds[ R.l0 ]; p < bounds[ R.l1 ] && R.flow; p++ ) {
@@ -752,20 +796,27 @@ void ilu0_build( tnlmi_preconditioner& P, const tnlmi_matrix& A, hipStream_t s )
       upload_vec( dridx, ridx, s );
       upload_vec( drval, rval, s );
    };
-   positions( false, lo, P.llev, P.lruns, P.lpp, P.ldep, P.lval, nullptr, P.lridx, P.lrval );
-   positions( true, uo, P.ulev, P.uruns, P.upp, P.udep, P.uval, &P.udiag, P.uridx, P.urval );
-   P.bpos.allocate( std::max< int64_t >( N, 1 ) );
-   P.xpos.allocate( std::max< int64_t >( N, 1 ) + kLvThreads );
-   upload_vec( P.dllev, P.llev, s );
-   upload_vec( P.dulev, P.ulev, s );
-   upload_vec( P.lp, lp, s );
-   upload_vec( P.lc, lc, s );
-   upload_vec( P.lv, lv, s );
-   upload_vec( P.up, up, s );
-   upload_vec( P.uc, uc, s );
-   upload_vec( P.uv, uv, s );
-   upload_vec( P.lrows, lo, s );
-   upload_vec( P.urows, uo, s );
+   // what the solves by levels read, for the factors that take them
+   if( ! P.lstrips.used() || ! P.ustrips.used() ) {
+      P.bpos.allocate( std::max< int64_t >( N, 1 ) );
+      P.xpos.allocate( std::max< int64_t >( N, 1 ) + kLvThreads );
+   }
+   if( ! P.lstrips.used() ) {
+      positions( false, lo, P.llev, P.lruns, P.lpp, P.ldep, P.lval, nullptr, P.lridx, P.lrval );
+      upload_vec( P.dllev, P.llev, s );
+      upload_vec( P.lp, lp, s );
+      upload_vec( P.lc, lc, s );
+      upload_vec( P.lv, lv, s );
+      upload_vec( P.lrows, lo, s );
+   }
+   if( ! P.ustrips.used() ) {
+      positions( true, uo, P.ulev, P.uruns, P.upp, P.udep, P.uval, &P.udiag, P.uridx, P.urval );
+      upload_vec( P.dulev, P.ulev, s );
+      upload_vec( P.up, up, s );
+      upload_vec( P.uc, uc, s );
+      upload_vec( P.uv, uv, s );
+      upload_vec( P.urows, uo, s );
+   }
    TNLMI_HIP( hipStreamSynchronize( s ) );
 }
 
@@ -801,32 +852,51 @@ void precond_apply( const tnlmi_preconditioner* P, int64_t n, const double* b, d
          hipLaunchKernelGGL( scatter_pos, dim3( (unsigned) ceil_div( p1 - p0, 256 ) ), dim3( 256 ), 0, s, p0, p1,
                              rows, (const double*) P->xpos.ptr, x );
    };
-   if( any_ring( P->lruns ) )
-      hipLaunchKernelGGL( gather_pos, gpos, dim3( 256 ), 0, s, n, P->lrows.ptr, b, P->bpos.ptr );
-   for( const auto& R : P->lruns ) {
-      if( R.flow ) {
-         const int64_t p0 = P->llev[ R.l0 ], p1 = P->llev[ R.l1 ];
-         hipLaunchKernelGGL( tri_flow< false >, dim3( 1 ), dim3( kLvThreads ), 0, s, P->lrows.ptr, p0, p1,
-                             (const RingIdx*) P->lridx.ptr, (const RingVal*) P->lrval.ptr, P->bpos.ptr,
-                             (const double*) x, P->xpos.ptr, n, spin_cap );
-         scatter_run( P->lrows.ptr, p0, p1 );
-         continue;
+   // (the strips' arrays are work space of the preconditioner, as bpos and xpos are)
+   TriStrips &LS = const_cast< TriStrips& >( P->lstrips ), &US = const_cast< TriStrips& >( P->ustrips );
+   if( LS.used() ) {
+      tri_strips_load( LS, b, LS.row.ptr, s );
+      tri_strips_solve( LS, spin_cap, s );
+      if( US.used() )
+         tri_strips_load( US, LS.x.ptr, P->mid.ptr, s );
+      else
+         tri_strips_store( LS, x, s );
+   }
+   else {
+      if( any_ring( P->lruns ) )
+         hipLaunchKernelGGL( gather_pos, gpos, dim3( 256 ), 0, s, n, P->lrows.ptr, b, P->bpos.ptr );
+      for( const auto& R : P->lruns ) {
+         if( R.flow ) {
+            const int64_t p0 = P->llev[ R.l0 ], p1 = P->llev[ R.l1 ];
+            hipLaunchKernelGGL( tri_flow< false >, dim3( 1 ), dim3( kLvThreads ), 0, s, P->lrows.ptr, p0, p1,
+                                (const RingIdx*) P->lridx.ptr, (const RingVal*) P->lrval.ptr, P->bpos.ptr,
+                                (const double*) x, P->xpos.ptr, n, spin_cap );
+            scatter_run( P->lrows.ptr, p0, p1 );
+            continue;
+         }
+         if( R.ring ) {
+            hipLaunchKernelGGL( tri_ring< false >, dim3( 1 ), dim3( kLvThreads ), 0, s, P->lrows.ptr, P->dllev.ptr, R.l0,
+                                R.l1, (const RingIdx*) P->lridx.ptr, (const RingVal*) P->lrval.ptr, P->bpos.ptr,
+                                (const double*) x, P->xpos.ptr, n );
+            scatter_run( P->lrows.ptr, P->llev[ R.l0 ], P->llev[ R.l1 ] );
+            continue;
+         }
+         if( R.narrow ) {
+            hipLaunchKernelGGL( tri_levels< false >, dim3( 1 ), dim3( kLvThreads ), 0, s, P->lrows.ptr, P->dllev.ptr,
+                                R.l0, R.l1, n, P->lp.ptr, P->lc.ptr, P->lv.ptr, b, x );
+            continue;
+         }
+         const int64_t cnt = P->llev[ R.l0 + 1 ] - P->llev[ R.l0 ];
+         hipLaunchKernelGGL( lower_level, dim3( (unsigned) ceil_div( cnt, 256 ) ), dim3( 256 ), 0, s,
+                             P->lrows.ptr + P->llev[ R.l0 ], cnt, P->lp.ptr, P->lc.ptr, P->lv.ptr, b, x );
       }
-      if( R.ring ) {
-         hipLaunchKernelGGL( tri_ring< false >, dim3( 1 ), dim3( kLvThreads ), 0, s, P->lrows.ptr, P->dllev.ptr, R.l0,
-                             R.l1, (const RingIdx*) P->lridx.ptr, (const RingVal*) P->lrval.ptr, P->bpos.ptr,
-                             (const double*) x, P->xpos.ptr, n );
-         scatter_run( P->lrows.ptr, P->llev[ R.l0 ], P->llev[ R.l1 ] );
-         continue;
-      }
-      if( R.narrow ) {
-         hipLaunchKernelGGL( tri_levels< false >, dim3( 1 ), dim3( kLvThreads ), 0, s, P->lrows.ptr, P->dllev.ptr,
-                             R.l0, R.l1, n, P->lp.ptr, P->lc.ptr, P->lv.ptr, b, x );
-         continue;
-      }
-      const int64_t cnt = P->llev[ R.l0 + 1 ] - P->llev[ R.l0 ];
-      hipLaunchKernelGGL( lower_level, dim3( (unsigned) ceil_div( cnt, 256 ) ), dim3( 256 ), 0, s,
-                          P->lrows.ptr + P->llev[ R.l0 ], cnt, P->lp.ptr, P->lc.ptr, P->lv.ptr, b, x );
+   }
+   if( US.used() ) {
+      if( ! LS.used() )
+         tri_strips_load( US, x, US.row.ptr, s );
+      tri_strips_solve( US, spin_cap, s );
+      tri_strips_store( US, x, s );
+      return;
    }
    // the upper solve's right-hand side is the lower solve's result
    if( any_ring( P->uruns ) )
