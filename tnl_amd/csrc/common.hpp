@@ -99,6 +99,12 @@ struct DeviceArray
          TNLMI_HIP( hipMalloc( (void**) &ptr, sizeof( T ) * (size_t) n ) );
       size = n;
    }
+   // room for n elements at least (the contents are not kept)
+   void reserve( int64_t n )
+   {
+      if( n > size )
+         allocate( n );
+   }
 };
 
 inline hipStream_t as_stream( tnlmi_stream s )

@@ -22,6 +22,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "segments.hpp"
@@ -233,7 +235,9 @@ __global__ void __launch_bounds__( 64 ) reduce_parts_chunks( const float* __rest
 struct Graph
 {
    int64_t n = 0, E = 0;
-   DeviceArray< int32_t > erow, cperm, cptr, deg;
+   DeviceArray< int32_t > erow, cperm, cptr, deg, ids;
+   DeviceArray< uint32_t > keys, skeys;
+   DeviceArray< char > sort_tmp;
    DeviceArray< double > diag;
    DeviceArray< float > xe, xn;
    DeviceArray< uint8_t > isd;
@@ -289,22 +293,26 @@ __global__ void g_features( int64_t n, const int32_t* __restrict__ off, const in
    xn[ i * 4 + 3 ] = 1.f;
 }
 
-__global__ void g_colptr( int64_t E, int64_t n, const int32_t* __restrict__ skeys, int32_t* __restrict__ cptr )
+__global__ void g_colptr( int64_t E, int64_t n, const uint32_t* __restrict__ skeys, int32_t* __restrict__ cptr )
 {
    const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
    if( p > E )
       return;
-   const int32_t prev = p == 0 ? -1 : skeys[ p - 1 ];
-   const int32_t cur = p == E ? (int32_t) n : skeys[ p ];
+   const int32_t prev = p == 0 ? -1 : (int32_t) skeys[ p - 1 ] - 1;
+   const int32_t cur = p == E ? (int32_t) n : (int32_t) skeys[ p ] - 1;
    for( int32_t c = prev + 1; c <= cur; c++ )
       cptr[ c ] = (int32_t) p;
 }
 
-__global__ void iota_k( int64_t E, int32_t* __restrict__ v )
+// sort keys column + 1 (0: a padding slot), so that only the bits of n are sorted
+__global__ void iota_k( int64_t E, const int32_t* __restrict__ cols, uint32_t* __restrict__ keys,
+                        int32_t* __restrict__ v )
 {
    const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-   if( p < E )
+   if( p < E ) {
+      keys[ p ] = (uint32_t) ( cols[ p ] + 1 );
       v[ p ] = (int32_t) p;
+   }
 }
 
 // ------------------------------------------------------------ forward parts
@@ -561,15 +569,60 @@ inline dim3 g1( int64_t cnt, int b = 256 )
 
 using namespace tnlmi;
 
+namespace tnlmi {
+namespace {
+
+struct Acts
+{
+   DeviceArray< uint16_t > E[ kL + 1 ], H[ kL + 1 ], G[ kL + 1 ];
+   DeviceArray< float > P, Q;
+};
+
+// What a call works in: the graph, the activations and the backward pass's
+// arrays.  A network keeps one, as large as the largest matrix it has seen,
+// and gives it back when it is destroyed: 45 allocations and frees of up to
+// 84 MB took 7 of the 10 ms of a training step on a 256^2 grid.
+struct Workspace
+{
+   Graph g;
+   Acts a;
+   DeviceArray< double > M, dM, Y, Rk, lpart, Z;
+   DeviceArray< float > dE, dEn, dH, dG, part, bpart, dpart, rwork;
+   DeviceArray< uint16_t > dS, dT, dP, dQ;
+   DeviceArray< double > lout;
+};
+
+}  // namespace
+}  // namespace tnlmi
+
 struct tnlmi_spai
 {
    DeviceArray< float > params, grads, m, v;
    DeviceArray< uint16_t > W, WT;  // BF16 copies of the 15 64 x 64 matrices
    int64_t step = 0;
+   mutable std::mutex busy;  // held by the call that works in `work`
+   mutable Workspace work;
 };
 
 namespace tnlmi {
 namespace {
+
+// A call's workspace: the network's, or one of its own while another thread's
+// call works in that.  The stream is waited for before the workspace passes on.
+struct Working
+{
+   std::unique_lock< std::mutex > lock;
+   std::unique_ptr< Workspace > own;
+   Workspace* w;
+   hipStream_t s;
+   Working( const tnlmi_spai& S, hipStream_t stream ) : lock( S.busy, std::try_to_lock ), s( stream )
+   {
+      if( ! lock.owns_lock() )
+         own = std::make_unique< Workspace >();
+      w = own ? own.get() : &S.work;
+   }
+   ~Working() { (void) hipStreamSynchronize( s ); }
+};
 
 const uint16_t* Wn( const tnlmi_spai& S, int l, int m )  // Bn for X W^T
 {
@@ -605,40 +658,35 @@ void build_graph( Graph& g, const tnlmi_matrix& A, hipStream_t s )
    const int32_t* off = A.segments->offsets.ptr;
    const int32_t* cols = A.column_indexes;
    const double* vals = (const double*) A.values;
-   g.erow.allocate( g.E );
-   g.deg.allocate( g.n );
-   g.diag.allocate( g.n );
-   g.isd.allocate( g.E );
-   g.xe.allocate( g.E * 4 );
-   g.xn.allocate( g.n * 4 );
+   g.erow.reserve( g.E );
+   g.deg.reserve( g.n );
+   g.diag.reserve( g.n );
+   g.isd.reserve( g.E );
+   g.xe.reserve( g.E * 4 );
+   g.xn.reserve( g.n * 4 );
    hipLaunchKernelGGL( g_rows, g1( g.n ), dim3( 256 ), 0, s, g.n, off, cols, vals, g.erow.ptr, g.deg.ptr,
                        g.diag.ptr, g.isd.ptr );
    hipLaunchKernelGGL( g_features, g1( g.n ), dim3( 256 ), 0, s, g.n, off, cols, vals, g.diag.ptr, g.xe.ptr,
                        g.xn.ptr );
    // edges grouped by column (stable radix sort by column): the transposed scatter
-   DeviceArray< int32_t > ids, skeys;
-   ids.allocate( g.E );
-   skeys.allocate( g.E );
-   g.cperm.allocate( g.E );
-   g.cptr.allocate( g.n + 1 );
-   hipLaunchKernelGGL( iota_k, g1( g.E ), dim3( 256 ), 0, s, g.E, ids.ptr );
+   g.ids.reserve( g.E );
+   g.keys.reserve( g.E );
+   g.skeys.reserve( g.E );
+   g.cperm.reserve( g.E );
+   g.cptr.reserve( g.n + 1 );
+   int bits = 1;
+   while( ( g.n >> bits ) != 0 )
+      bits++;
+   hipLaunchKernelGGL( iota_k, g1( g.E ), dim3( 256 ), 0, s, g.E, cols, g.keys.ptr, g.ids.ptr );
    size_t bytes = 0;
-   TNLMI_HIP( hipcub::DeviceRadixSort::SortPairs( nullptr, bytes, cols, skeys.ptr, ids.ptr, g.cperm.ptr, (int) g.E,
-                                                  0, 32, s ) );
-   DeviceArray< char > tmp;
-   tmp.allocate( (int64_t) bytes + 1 );
-   TNLMI_HIP( hipcub::DeviceRadixSort::SortPairs( tmp.ptr, bytes, cols, skeys.ptr, ids.ptr, g.cperm.ptr, (int) g.E,
-                                                  0, 32, s ) );
-   hipLaunchKernelGGL( g_colptr, g1( g.E + 1 ), dim3( 256 ), 0, s, g.E, g.n, skeys.ptr, g.cptr.ptr );
+   TNLMI_HIP( hipcub::DeviceRadixSort::SortPairs( nullptr, bytes, g.keys.ptr, g.skeys.ptr, g.ids.ptr, g.cperm.ptr,
+                                                  (int) g.E, 0, bits, s ) );
+   g.sort_tmp.reserve( (int64_t) bytes + 1 );
+   TNLMI_HIP( hipcub::DeviceRadixSort::SortPairs( g.sort_tmp.ptr, bytes, g.keys.ptr, g.skeys.ptr, g.ids.ptr,
+                                                  g.cperm.ptr, (int) g.E, 0, bits, s ) );
+   hipLaunchKernelGGL( g_colptr, g1( g.E + 1 ), dim3( 256 ), 0, s, g.E, g.n, g.skeys.ptr, g.cptr.ptr );
    TNLMI_HIP( hipGetLastError() );
-   TNLMI_HIP( hipStreamSynchronize( s ) );  // the temporaries go out of scope
 }
-
-struct Acts
-{
-   DeviceArray< uint16_t > E[ kL + 1 ], H[ kL + 1 ], G[ kL + 1 ];
-   DeviceArray< float > P, Q;
-};
 
 template< int NT, int EPI >
 void gemm( int64_t R, Term t0, Term t1, Term t2, const EpiArgs& e, hipStream_t s )
@@ -654,13 +702,13 @@ void forward( const tnlmi_spai& S, const Graph& g, const int32_t* off, const int
    const float* p = S.params.ptr;
    const int nE = keep ? kL + 1 : 2, nH = keep ? kL + 1 : 2;
    for( int i = 0; i < nE; i++ )
-      a.E[ i ].allocate( E * kH );
+      a.E[ i ].reserve( E * kH );
    for( int i = 0; i < nH; i++ ) {
-      a.H[ i ].allocate( n * kH );
-      a.G[ i ].allocate( n * kH );
+      a.H[ i ].reserve( n * kH );
+      a.G[ i ].reserve( n * kH );
    }
-   a.P.allocate( n * kH );
-   a.Q.allocate( n * kH );
+   a.P.reserve( n * kH );
+   a.Q.reserve( n * kH );
    hipLaunchKernelGGL( encode_k, g1( E * kH ), dim3( 256 ), 0, s, E, g.xe.ptr, p + oAe, p + oae, a.E[ 0 ].ptr );
    hipLaunchKernelGGL( encode_k, g1( n * kH ), dim3( 256 ), 0, s, n, g.xn.ptr, p + oAn, p + oan, a.H[ 0 ].ptr );
    const Term none{ nullptr, nullptr };
@@ -716,18 +764,19 @@ void wgrad( int64_t R, const uint16_t* X, const uint16_t* dY, float* gW, float* 
 }
 
 // probe loss on the device: returns L (host) and dL/dM per edge in dM
-double probe_loss( const tnlmi_matrix& A, const Graph& g, const double* M, const double* Z, int K, double* dM,
+double probe_loss( const tnlmi_matrix& A, Workspace& w, const double* M, const double* Z, int K, double* dM,
                    hipStream_t s )
 {
+   const Graph& g = w.g;
    const int64_t n = g.n, E = g.E;
    const int32_t* off = A.segments->offsets.ptr;
    const int32_t* cols = A.column_indexes;
-   DeviceArray< double > Y, Rk, part, out;
-   Y.allocate( n * K );
-   Rk.allocate( n * K );
+   DeviceArray< double >&Y = w.Y, &Rk = w.Rk, &part = w.lpart, &out = w.lout;
+   Y.reserve( n * K );
+   Rk.reserve( n * K );
    const int64_t nb = ceil_div( n, 256 );
-   part.allocate( nb * K );
-   out.allocate( 1 );
+   part.reserve( nb * K );
+   out.reserve( 1 );
    for( int k = 0; k < K; k++ ) {
       hipLaunchKernelGGL( csr_mv, g1( n ), dim3( 256 ), 0, s, n, off, cols, (const double*) A.values, Z + k * n,
                           Y.ptr + k * n );
@@ -746,38 +795,41 @@ double probe_loss( const tnlmi_matrix& A, const Graph& g, const double* M, const
 }
 
 // gradients of the loss into S.grads
-double loss_grad( tnlmi_spai& S, const tnlmi_matrix& A, const double* Z, int K, double* Mout, hipStream_t s )
+double loss_grad( tnlmi_spai& S, Workspace& w, const tnlmi_matrix& A, const double* Z, int K, double* Mout,
+                  hipStream_t s )
 {
-   Graph g;
+   Graph& g = w.g;
    build_graph( g, A, s );
    const int64_t n = g.n, E = g.E;
    const int32_t* off = A.segments->offsets.ptr;
    const int32_t* cols = A.column_indexes;
-   Acts a;
-   DeviceArray< double > M, dM;
-   M.allocate( E );
-   dM.allocate( E );
-   forward( S, g, off, cols, a, true, M.ptr, s );
-   const double L = probe_loss( A, g, M.ptr, Z, K, dM.ptr, s );
-   if( Mout )
-      TNLMI_HIP( hipMemcpyAsync( Mout, M.ptr, sizeof( double ) * E, hipMemcpyDeviceToDevice, s ) );
+   Acts& a = w.a;
+   w.dM.reserve( E );
+   if( ! Mout ) {
+      w.M.reserve( E );
+      Mout = w.M.ptr;
+   }
+   forward( S, g, off, cols, a, true, Mout, s );
+   const double L = probe_loss( A, w, Mout, Z, K, w.dM.ptr, s );
    float* gr = S.grads.ptr;
    const float* p = S.params.ptr;
-   DeviceArray< float > dE, dEn, dH, dG, part, bpart, dpart, rwork;
-   DeviceArray< uint16_t > dS, dT, dP, dQ;
-   dE.allocate( E * kH );
-   dEn.allocate( E * kH );
-   dH.allocate( n * kH );
-   dG.allocate( n * kH );
-   dS.allocate( E * kH );
-   dT.allocate( n * kH );
-   dP.allocate( n * kH );
-   dQ.allocate( n * kH );
-   const int64_t nbE = ceil_div( E, kWRows );
-   part.allocate( nbE * kH * kH );
-   bpart.allocate( nbE * kH );
-   dpart.allocate( ceil_div( E, 256 ) * ( 5 * kH ) + 1 );
-   rwork.allocate( (int64_t) kRedChunks * kH * kH );  // chunk sums of reduce_partials (widest: kH * kH)
+   DeviceArray< double >& dM = w.dM;
+   DeviceArray< float >&dE = w.dE, &dEn = w.dEn, &dH = w.dH, &dG = w.dG, &part = w.part, &bpart = w.bpart,
+                       &dpart = w.dpart, &rwork = w.rwork;
+   DeviceArray< uint16_t >&dS = w.dS, &dT = w.dT, &dP = w.dP, &dQ = w.dQ;
+   dE.reserve( E * kH );
+   dEn.reserve( E * kH );
+   dH.reserve( n * kH );
+   dG.reserve( n * kH );
+   dS.reserve( E * kH );
+   dT.reserve( n * kH );
+   dP.reserve( n * kH );
+   dQ.reserve( n * kH );
+   const int64_t nbE = ceil_div( std::max( E, n ), kWRows );
+   part.reserve( nbE * kH * kH );
+   bpart.reserve( nbE * kH );
+   dpart.reserve( ceil_div( std::max( E, n ), 256 ) * ( 5 * kH ) + 1 );
+   rwork.reserve( (int64_t) kRedChunks * kH * kH );  // chunk sums of reduce_partials (widest: kH * kH)
    // decoder
    const int64_t nb256 = ceil_div( E, 256 );
    hipLaunchKernelGGL( dec_bwd_k, dim3( (unsigned) nb256 ), dim3( 256 ), 0, s, E, dM.ptr, g.erow.ptr, g.diag.ptr,
@@ -884,10 +936,9 @@ tnlmi_status tnlmi_spai_apply( const tnlmi_spai* S, const tnlmi_matrix* A, doubl
          fail( TNLMI_INVALID_ARGUMENT, "spai_apply: NULL argument" );
       check_csr( A );
       hipStream_t s = as_stream( stream );
-      Graph g;
-      build_graph( g, *A, s );
-      Acts a;
-      forward( *S, g, A->segments->offsets.ptr, A->column_indexes, a, false, d_M, s );
+      const Working work( *S, s );
+      build_graph( work.w->g, *A, s );
+      forward( *S, work.w->g, A->segments->offsets.ptr, A->column_indexes, work.w->a, false, d_M, s );
       TNLMI_HIP( hipStreamSynchronize( s ) );
    } );
 }
@@ -899,7 +950,8 @@ tnlmi_status tnlmi_spai_loss_grad( tnlmi_spai* S, const tnlmi_matrix* A, const d
       if( ! S || ! d_Z || K <= 0 || ! loss )
          fail( TNLMI_INVALID_ARGUMENT, "spai_loss_grad: invalid argument" );
       check_csr( A );
-      *loss = loss_grad( *S, *A, d_Z, K, d_M, as_stream( stream ) );
+      const Working work( *S, as_stream( stream ) );
+      *loss = loss_grad( *S, *work.w, *A, d_Z, K, d_M, as_stream( stream ) );
    } );
 }
 
@@ -911,11 +963,12 @@ tnlmi_status tnlmi_spai_train_step( tnlmi_spai* S, const tnlmi_matrix* A, int32_
          fail( TNLMI_INVALID_ARGUMENT, "spai_train_step: invalid argument" );
       check_csr( A );
       hipStream_t s = as_stream( stream );
-      DeviceArray< double > Z;
-      Z.allocate( (int64_t) K * A->rows );
+      const Working work( *S, s );
+      DeviceArray< double >& Z = work.w->Z;
+      Z.reserve( (int64_t) K * A->rows );
       hipLaunchKernelGGL( rademacher_k, g1( (int64_t) K * A->rows ), dim3( 256 ), 0, s, (int64_t) K * A->rows,
                           probe_seed, Z.ptr );
-      *loss = loss_grad( *S, *A, Z.ptr, K, nullptr, s );
+      *loss = loss_grad( *S, *work.w, *A, Z.ptr, K, nullptr, s );
       S->step++;
       const float b1 = 0.9f, b2 = 0.999f;
       const float c1 = 1.f - std::pow( b1, (float) S->step ), c2 = 1.f - std::pow( b2, (float) S->step );
