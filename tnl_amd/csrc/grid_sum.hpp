@@ -1,0 +1,119 @@
+// grid_sum.hpp -- sums over all workgroups of a running kernel, and data
+// passed between its workgroups, for kernels whose whole grid is resident
+// (cooperative launches): an iteration of a Krylov solver then needs no kernel
+// boundary.  A launch costs about 5 us on MI355X and each reduction of an
+// iteration used to end one; a grid sum takes about 2 us.
+#pragma once
+
+#include "common.hpp"
+
+namespace tnlmi {
+
+constexpr int kGridMax = 256;        // workgroups at most: one per CU
+constexpr int kGridValues = 4;       // values per sum at most
+constexpr uint64_t kGridWait = 200'000'000;  // 100 MHz ticks (2 s) until a wait gives up
+
+// One value of one workgroup: two words, each with half of the value and the
+// sum's number, so that a reader sees from each word whether it belongs to
+// the sum it waits for.  Two buffers in turn: a workgroup that publishes sum k
+// has seen every workgroup's part of sum k - 1, so all are done with k - 2.
+struct GridSlots
+{
+   uint64_t word[ 2 ][ kGridValues ][ kGridMax ][ 2 ];
+};
+
+// Accesses seen by all workgroups of the running kernel (the XCDs' L2 caches
+// are not coherent with each other: these go past them).
+template< typename T >
+__device__ __forceinline__ T shared_load( const T* p )
+{
+   return __hip_atomic_load( p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+}
+template< typename T >
+__device__ __forceinline__ void shared_store( T* p, T v )
+{
+   __hip_atomic_store( p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+}
+
+// this wave's shared_stores have reached where every workgroup sees them
+__device__ __forceinline__ void shared_stores_done()
+{
+   asm volatile( "s_waitcnt vmcnt(0)" ::: "memory" );
+}
+
+// v[j] = the sum over all threads of all workgroups, in a fixed order (the same
+// bits in every workgroup).  What a workgroup shared_stores before the sum is
+// seen by all after it.  sm: N * T / 64 doubles of LDS.  Returns false when a
+// workgroup did not arrive in time (then every workgroup gives up).
+template< int T, int N >
+__device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restrict__ slots, uint32_t number, double* sm )
+{
+   static_assert( N <= kGridValues && T >= kGridMax, "one thread per workgroup's slot" );
+   constexpr int W = T / 64;
+   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, G = gridDim.x;
+   auto block_total = [ & ]( int j ) {
+      double r = 0;
+#pragma unroll
+      for( int i = 0; i < W; i++ )
+         r += sm[ j * W + i ];
+      return r;
+   };
+   auto wave_totals = [ & ] {
+#pragma unroll
+      for( int j = 0; j < N; j++ )
+         v[ j ] = group_sum< 64 >( v[ j ] );
+      if( lane == 0 )
+#pragma unroll
+         for( int j = 0; j < N; j++ )
+            sm[ j * W + w ] = v[ j ];
+   };
+   wave_totals();
+   shared_stores_done();
+   __syncthreads();
+   uint64_t( &buf )[ kGridValues ][ kGridMax ][ 2 ] = slots->word[ number & 1 ];
+   if( threadIdx.x < N ) {
+      const uint64_t bits = (uint64_t) __double_as_longlong( block_total( threadIdx.x ) );
+      const uint64_t tag = (uint64_t) number << 32;
+      shared_store( &buf[ threadIdx.x ][ blockIdx.x ][ 0 ], tag | ( bits & 0xffffffffu ) );
+      shared_store( &buf[ threadIdx.x ][ blockIdx.x ][ 1 ], tag | ( bits >> 32 ) );
+   }
+   __syncthreads();  // (sm is read above and written below)
+   int late = 0;
+   if( (int) threadIdx.x < G ) {
+      const uint64_t begin = wall_clock64();
+      uint64_t lo[ N ], hi[ N ];
+      while( true ) {
+         bool there = true;
+#pragma unroll
+         for( int j = 0; j < N; j++ ) {
+            lo[ j ] = shared_load( &buf[ j ][ threadIdx.x ][ 0 ] );
+            hi[ j ] = shared_load( &buf[ j ][ threadIdx.x ][ 1 ] );
+         }
+#pragma unroll
+         for( int j = 0; j < N; j++ )
+            there = there && (uint32_t) ( lo[ j ] >> 32 ) == number && (uint32_t) ( hi[ j ] >> 32 ) == number;
+         if( there )
+            break;
+         if( wall_clock64() - begin > kGridWait ) {
+            late = 1;
+            break;
+         }
+      }
+#pragma unroll
+      for( int j = 0; j < N; j++ )
+         v[ j ] = __longlong_as_double( (long long) ( ( hi[ j ] << 32 ) | ( lo[ j ] & 0xffffffffu ) ) );
+   }
+   else
+#pragma unroll
+      for( int j = 0; j < N; j++ )
+         v[ j ] = 0;
+   wave_totals();
+   late = __syncthreads_or( late );
+#pragma unroll
+   for( int j = 0; j < N; j++ )
+      v[ j ] = wave_uniform( block_total( j ) );
+   __syncthreads();  // (sm may be written again)
+   return ! late;
+}
+
+}  // namespace tnlmi
