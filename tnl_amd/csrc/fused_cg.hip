@@ -913,6 +913,369 @@ bool grid_cg_launch( const GridCg< T, X >& a, hipStream_t s )
    return false;
 }
 
+// ---- row masks: the iteration of large matrices whose entries take few
+// distinct (column - row, value) pairs -- a constant-coefficient stencil: 7 for
+// the 3D 7-point Laplacian.  The pairs travel as kernel arguments and a row is
+// a bit mask over them (1 or 2 bytes instead of 12 per entry), so the product
+// costs little more than reading p, and an iteration forms it twice instead of
+// writing and reading A p:
+//   mk_dot   partial sums of (A p, p)                                   reads p
+//   mk_upd   r -= alpha A p, partial sums of (r, z)                     reads p, r; writes r
+//   mk_dir   x += alpha p, then cg_dir's end of the iteration           reads r, p, x; writes p, x
+// 9 vectors of n (10 and 11 with a diagonal that varies) instead of 13 and
+// the matrix.  A row's entries are added in their order with the stored values,
+// so products are those of spmv_dot_ell bit for bit.
+// Poisson 256^3, per iteration: FP64 68 + 122 + 105 us against 356 + 5 + 162 + 109
+// us on the stored matrix (a solve 321 against 687 ms); reliable BF16 27 + 46 + 52
+// against 127 + 5 + 72 + 44 us (148 against 283 ms).  The products' 7 reads of p
+// per row (L1 hits mostly) bound mk_dot: 65 us where its 151 MB take 30 at copy
+// speed.  16 bytes of rows per thread (2 FP64, 4 FP32) are best: FP64 91 us with 1
+// row and 76 with 4.
+constexpr int kPairs = 16;
+constexpr int kPairHash = 256;
+
+template< typename T >
+struct PairDict
+{
+   int32_t off[ kPairs ];
+   T val[ kPairs ];
+};
+
+struct PairTable  // the pairs found so far
+{
+   unsigned long long key[ kPairHash ];  // mix of the pair (kEmpty: free)
+   unsigned long long val[ kPairHash ];  // value bits
+   int32_t off[ kPairHash ];
+   int32_t count, reject;
+};
+
+template< typename V >
+__device__ __forceinline__ uint64_t value_bits( const V* vals, int64_t g )
+{
+   uint64_t b = 0;
+   __builtin_memcpy( &b, vals + g, sizeof( V ) );
+   return b;
+}
+__device__ __forceinline__ uint64_t pair_mix( int32_t off, uint64_t bits )
+{
+   uint64_t z = bits * 0x9e3779b97f4a7c15ull + (uint32_t) off;
+   z = ( z ^ ( z >> 29 ) ) * 0xbf58476d1ce4e5b9ull;
+   z ^= z >> 32;
+   return z == kEmpty ? 0 : z;
+}
+
+template< typename V >
+__global__ void __launch_bounds__( kFT ) pairs_collect( SegView v, const int32_t* __restrict__ cols,
+                                                        const V* __restrict__ vals, PairTable* table )
+{
+   __shared__ unsigned long long seen[ kFT ];  // by the key's low bits: pairs that are in the table
+   seen[ threadIdx.x ] = kEmpty;
+   __syncthreads();
+   constexpr int kEntries = 8;  // loaded together
+   for( int64_t r = (int64_t) blockIdx.x * kFT + threadIdx.x; r < v.n; r += (int64_t) gridDim.x * kFT ) {
+      const int32_t reject = *(volatile int32_t*) &table->reject;
+      int32_t w = 0;
+      ell_slot( v, r, 0, &w );
+      for( int32_t k0 = 0; k0 < w; k0 += kEntries ) {
+         int32_t c[ kEntries ];
+         uint64_t bits[ kEntries ];
+#pragma unroll
+         for( int u = 0; u < kEntries; u++ ) {
+            const int64_t g = ell_slot( v, r, min( k0 + u, w - 1 ), &w );
+            c[ u ] = cols[ g ];
+            bits[ u ] = value_bits( vals, g );
+         }
+         if( reject )
+            return;
+         uint32_t fresh = 0;  // entries that this workgroup has not seen
+#pragma unroll
+         for( int u = 0; u < kEntries; u++ ) {
+            const unsigned long long key = pair_mix( c[ u ] - (int32_t) r, bits[ u ] );
+            if( c[ u ] >= 0
+                && __hip_atomic_load( seen + ( key & ( kFT - 1 ) ), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP )
+                      != key )
+               fresh |= 1u << u;
+         }
+         if( ! fresh )
+            continue;
+         for( int u = 0; u < kEntries; u++ ) {  // (rarely)
+            if( ! ( fresh >> u & 1 ) )
+               continue;
+            const int64_t g = ell_slot( v, r, min( k0 + u, w - 1 ), &w );
+            const int32_t off = cols[ g ] - (int32_t) r;
+            const uint64_t bit = value_bits( vals, g );
+            const unsigned long long key = pair_mix( off, bit );
+            bool placed = false;
+            for( int probe = 0, h = (int) ( key >> 40 ) & ( kPairHash - 1 ); probe < kPairHash && ! placed;
+                 probe++, h = ( h + 1 ) & ( kPairHash - 1 ) ) {
+               // (a read first: one atomic by every thread at the same pair would queue up)
+               unsigned long long prev = shared_load( &table->key[ h ] );
+               if( prev == kEmpty )
+                  prev = atomicCAS( &table->key[ h ], kEmpty, key );
+               if( prev == kEmpty ) {
+                  table->val[ h ] = bit;
+                  table->off[ h ] = off;
+                  if( atomicAdd( &table->count, 1 ) >= kPairs )
+                     atomicExch( &table->reject, 1 );
+               }
+               placed = prev == kEmpty || prev == key;
+            }
+            if( ! placed )
+               atomicExch( &table->reject, 1 );
+            __hip_atomic_store( seen + ( key & ( kFT - 1 ) ), key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
+         }
+      }
+   }
+}
+
+struct RawDict  // the pairs by offset, then value bits
+{
+   int32_t count;
+   int32_t off[ kPairs ];
+   uint64_t bits[ kPairs ];
+};
+
+// mask[r] = bit q for each entry that is pair q; a row whose entries are not
+// pairs in increasing order (another order of the sum, a repeated column, a
+// pair that shares another's key) rejects the matrix
+template< typename V, typename M >
+__global__ void __launch_bounds__( kFT ) pairs_encode( SegView v, const int32_t* __restrict__ cols,
+                                                       const V* __restrict__ vals, RawDict D, M* __restrict__ mask,
+                                                       int64_t rows, int32_t* reject )
+{
+   for( int64_t r = (int64_t) blockIdx.x * kFT + threadIdx.x; r < rows; r += (int64_t) gridDim.x * kFT ) {
+      uint32_t m = 0;
+      if( r < v.n ) {
+         int32_t w = 0, last = -1;
+         ell_slot( v, r, 0, &w );
+         for( int32_t k = 0; k < w; k++ ) {
+            const int64_t g = ell_slot( v, r, k, &w );
+            const int32_t c = cols[ g ];
+            if( c < 0 )
+               continue;
+            const uint64_t bits = value_bits( vals, g );
+            int32_t q = -1;
+#pragma unroll
+            for( int i = 0; i < kPairs; i++ )
+               if( i < D.count && D.off[ i ] == c - (int32_t) r && D.bits[ i ] == bits )
+                  q = i;
+            if( q <= last || ( last >= 0 && D.off[ q ] == D.off[ last ] ) ) {
+               *reject = 1;
+               break;
+            }
+            m |= 1u << q;
+            last = q;
+         }
+      }
+      mask[ r ] = (M) m;
+   }
+}
+
+// is d one value throughout (bit for bit)?
+__global__ void __launch_bounds__( kFT ) varies( int64_t n, const double* __restrict__ d, int32_t* __restrict__ out )
+{
+   const uint64_t first = (uint64_t) __double_as_longlong( d[ 0 ] );
+   bool other = false;
+   for( int64_t i = (int64_t) blockIdx.x * kFT + threadIdx.x; i < n; i += (int64_t) gridDim.x * kFT )
+      other = other || (uint64_t) __double_as_longlong( d[ i ] ) != first;
+   if( other )
+      *out = 1;
+}
+
+// R rows of A p from row r0 (p has room for every pair's offset at both ends)
+template< int R, int NP, typename M, typename T >
+__device__ __forceinline__ void mask_rows( const PairDict< T >& D, const M* __restrict__ mask, const T* __restrict__ p,
+                                           int64_t r0, T ( &y )[ R ] )
+{
+   typename Vec< M, R >::type m = *(const typename Vec< M, R >::type*) ( mask + r0 );
+   T g[ NP ][ R ];
+#pragma unroll
+   for( int k = 0; k < NP; k++ )
+      __builtin_memcpy( g[ k ], p + ( r0 + D.off[ k ] ), sizeof( g[ k ] ) );
+#pragma unroll
+   for( int j = 0; j < R; j++ )
+      y[ j ] = 0;
+#pragma unroll
+   for( int k = 0; k < NP; k++ )
+#pragma unroll
+      for( int j = 0; j < R; j++ ) {
+         const T t = y[ j ] + D.val[ k ] * g[ k ][ j ];
+         y[ j ] = m[ j ] >> k & 1 ? t : y[ j ];
+      }
+}
+
+// The tiles of kFT * R rows in the order of the sweep: each XCD has one
+// contiguous range, which its workgroups go through side by side (the planes a
+// row reads are then in the XCD's L2).
+template< int R, typename F >
+__device__ __forceinline__ void sweep( int64_t n, F&& f )
+{
+   const int64_t tiles = ( n + kFT * R - 1 ) / ( kFT * R );
+   const int64_t x = blockIdx.x % kXcds, j = blockIdx.x / kXcds, per = gridDim.x / kXcds;
+   const int64_t t0 = tiles * x / kXcds, t1 = tiles * ( x + 1 ) / kXcds;
+   for( int64_t t = t0 + j; t < t1; t += per )
+      f( ( t * kFT + threadIdx.x ) * R );
+}
+
+template< int R, int NP, typename M, typename T >
+__global__ void __launch_bounds__( kFT ) mk_dot( int64_t n, PairDict< T > D, const M* __restrict__ mask,
+                                                 const T* __restrict__ p, double* __restrict__ part1,
+                                                 const CgDev* __restrict__ st )
+{
+   __shared__ double sm[ kFT / 64 ];
+   if( ! st->active )
+      return;
+   double acc = 0;
+   sweep< R >( n, [ & ]( int64_t r0 ) {
+      if( r0 < n ) {  // (a last group's rows past n: no entries)
+         T y[ R ], pr[ R ];
+         __builtin_memcpy( pr, p + r0, sizeof( pr ) );
+         mask_rows< R, NP >( D, mask, p, r0, y );
+#pragma unroll
+         for( int j = 0; j < R; j++ )
+            acc += r0 + j < n ? (double) y[ j ] * (double) pr[ j ] : 0.0;
+      }
+   } );
+   put_part( acc, sm, part1 );
+}
+
+// d: the diagonal where it varies (else NULL and d0)
+template< int R, int NP, typename M, typename T, typename DT >
+__global__ void __launch_bounds__( kFT ) mk_upd( int64_t n, PairDict< T > D, const M* __restrict__ mask,
+                                                 const double* __restrict__ part1, T* __restrict__ r,
+                                                 const T* __restrict__ p, const DT* __restrict__ d, T d0,
+                                                 double* __restrict__ part2, double* __restrict__ part3,
+                                                 const CgDev* __restrict__ st )
+{
+   __shared__ double sm[ kFT / 64 ];
+   if( ! st->active )
+      return;
+   const double s2 = sum_parts( part1, sm, (int) gridDim.x );
+   if( s2 == 0.0 )
+      return;  // the direction step ends the solve
+   const T alpha = (T) ( st->s1 / s2 );
+   double a2 = 0, a3 = 0;
+   sweep< R >( n, [ & ]( int64_t r0 ) {
+      if( r0 < n ) {
+         T y[ R ], rr[ R ], dd[ R ];
+         // r has room for a last group's rows past n
+         __builtin_memcpy( rr, r + r0, sizeof( rr ) );
+#pragma unroll
+         for( int j = 0; j < R; j++ )
+            dd[ j ] = d && r0 + j < n ? (T) d[ r0 + j ] : d0;
+         mask_rows< R, NP >( D, mask, p, r0, y );
+#pragma unroll
+         for( int j = 0; j < R; j++ ) {
+            const T ri = rr[ j ] - alpha * y[ j ];
+            rr[ j ] = ri;
+            const T zi = ri / dd[ j ];
+            if( r0 + j < n ) {
+               a2 += (double) ri * (double) zi;
+               a3 += (double) ri * (double) ri;
+            }
+         }
+         __builtin_memcpy( r + r0, rr, sizeof( rr ) );
+      }
+   } );
+   put_part( a2, sm, part2 );
+   if( part3 )
+      put_part( a3, sm, part3 );
+}
+
+// x += alpha p; the end of the iteration as cg_dir (or, MIXED, mx_dir)
+template< int R, bool MIXED, typename T, typename X, typename DT >
+__global__ void __launch_bounds__( kFT ) mk_dir( int64_t n, const double* __restrict__ part1,
+                                                 const double* __restrict__ part2, const double* __restrict__ part3,
+                                                 const T* __restrict__ r, const DT* __restrict__ d, T d0,
+                                                 T* __restrict__ p, X* __restrict__ x, const CgDev* __restrict__ cur,
+                                                 CgDev* __restrict__ nxt, StopRule S, double delta2 )
+{
+   __shared__ double sm[ 3 * ( kFT / 64 ) ];
+   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+   if( ! cur->active ) {
+      if( lead )
+         *nxt = *cur;
+      return;
+   }
+   double t[ 3 ] = { 0, 0, 0 };
+   if( MIXED || S.kind == 1 )
+      sum_parts_n< 3 >( { part1, part2, part3 }, sm, t, (int) gridDim.x );
+   else {
+      double t2[ 2 ];
+      sum_parts_n< 2 >( { part1, part2 }, sm, t2, (int) gridDim.x );
+      t[ 0 ] = t2[ 0 ], t[ 1 ] = t2[ 1 ];
+   }
+   const double s2 = t[ 0 ], s1n = t[ 1 ], rr = t[ 2 ], s1 = cur->s1;
+   const double beta = s1 == 0.0 ? 0.0 : s1n / s1;
+   bool go;
+   if( MIXED ) {
+      const int64_t it = cur->it + 1;
+      const double rr_max = fmax( cur->rr_max, rr );
+      go = ! ( s2 == 0.0 || rr < delta2 * rr_max || sqrt( rr ) < S.tol * cur->normb || it >= S.maxit || isnan( rr ) );
+      if( lead ) {
+         *nxt = *cur;
+         nxt->it = it;
+         nxt->s1_prev = s1;
+         if( s2 != 0.0 ) {
+            nxt->s1 = s1n;
+            nxt->beta = beta;
+            nxt->rr = rr;
+            nxt->rr_max = rr_max;
+         }
+         if( ! go ) {
+            nxt->want_update = 1;
+            nxt->active = 0;
+         }
+      }
+   }
+   else {
+      const double res = s2 == 0.0 ? 0.0 : sqrt( S.kind == 1 ? rr : s1n ) / cur->normb;
+      go = s2 != 0.0 && check_next( S, res, cur->it );
+      if( lead ) {
+         *nxt = *cur;
+         nxt->res = res;
+         nxt->active = go ? 1 : 0;
+         if( s2 == 0.0 )
+            nxt->s2zero = 1;
+         else {
+            nxt->s1 = s1n;
+            nxt->beta = beta;
+            nxt->it = cur->it + 1;
+         }
+      }
+   }
+   if( s2 == 0.0 )
+      return;
+   const T alpha = (T) ( s1 / s2 ), tb = (T) beta;
+   sweep< R >( n, [ & ]( int64_t r0 ) {
+      if( r0 + R <= n ) {
+         T rv[ R ], pv[ R ], dd[ R ];
+         X xv[ R ];
+         __builtin_memcpy( rv, r + r0, sizeof( rv ) );
+         __builtin_memcpy( pv, p + r0, sizeof( pv ) );
+         __builtin_memcpy( xv, x + r0, sizeof( xv ) );
+#pragma unroll
+         for( int j = 0; j < R; j++ )
+            dd[ j ] = d ? (T) d[ r0 + j ] : d0;
+#pragma unroll
+         for( int j = 0; j < R; j++ ) {
+            xv[ j ] += (X) ( alpha * pv[ j ] );
+            pv[ j ] = rv[ j ] / dd[ j ] + tb * pv[ j ];
+         }
+         __builtin_memcpy( x + r0, xv, sizeof( xv ) );
+         if( go )
+            __builtin_memcpy( p + r0, pv, sizeof( pv ) );
+      }
+      else
+         for( int64_t i = r0; i < n; i++ ) {
+            const T pi = p[ i ];
+            x[ i ] += (X) ( alpha * pi );
+            if( go )
+               p[ i ] = r[ i ] / ( d ? (T) d[ i ] : d0 ) + tb * pi;
+         }
+   } );
+}
+
 // ---- set-up kernels
 __global__ void cg_start( CgDev* st, const double* s1, const double* normb, const double* rr, StopRule R )
 {
@@ -1050,7 +1413,138 @@ struct Stage
    std::shared_ptr< DeviceArray< uint8_t > > codes;
    std::shared_ptr< DeviceArray< int32_t > > dict;
    int32_t ndict = 0;
+   // kind 1 as row masks (pairs > 0)
+   std::shared_ptr< DeviceArray< uint8_t > > masks;  // a row: 1 byte (pairs <= 8) or 2
+   int32_t pairs = 0, reach = 0;  // distinct pairs; the largest |column - row|
+   PairDict< double > dict64{};
+   PairDict< float > dict32{};
 };
+
+// The row masks of a column-major Ellpack / SlicedEllpack stage, or nothing
+// (more than kPairs distinct pairs, or rows with another order of entries).
+// Two passes over the matrix: 0.5 + 0.6 ms for 117 M FP64 entries.
+// TNLMI_COLUMN_CODES=0 in the environment keeps the matrix as it is.
+template< typename V >
+void make_masks_v( Stage& S, hipStream_t s )
+{
+   DeviceArray< PairTable > table;
+   table.allocate( 1 );
+   PairTable ht;
+   TNLMI_HIP( hipMemsetAsync( table.ptr, 0xff, offsetof( PairTable, val ), s ) );
+   TNLMI_HIP( hipMemsetAsync( &table.ptr->count, 0, 2 * sizeof( int32_t ), s ) );
+   hipLaunchKernelGGL( pairs_collect< V >, dim3( 2048 ), dim3( kFT ), 0, s, S.v, S.cols, (const V*) S.vals, table.ptr );
+   TNLMI_HIP( hipGetLastError() );
+   TNLMI_HIP( hipMemcpyAsync( &ht, table.ptr, sizeof( ht ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipStreamSynchronize( s ) );
+   if( ht.reject || ht.count > kPairs || ht.count == 0 )
+      return;
+   std::vector< std::pair< int32_t, uint64_t > > pairs;
+   for( int h = 0; h < kPairHash; h++ )
+      if( ht.key[ h ] != kEmpty )
+         pairs.push_back( { ht.off[ h ], ht.val[ h ] } );
+   std::sort( pairs.begin(), pairs.end() );
+   RawDict D{};
+   D.count = (int32_t) pairs.size();
+   for( int q = 0; q < D.count; q++ ) {
+      D.off[ q ] = pairs[ q ].first;
+      D.bits[ q ] = pairs[ q ].second;
+      V v;
+      memcpy( &v, &pairs[ q ].second, sizeof( V ) );
+      double d;
+      if constexpr( std::is_same_v< V, bf16 > )
+         d = (double) bf16_to_float( v.bits );
+      else
+         d = (double) v;
+      S.dict64.off[ q ] = S.dict32.off[ q ] = D.off[ q ];
+      S.dict64.val[ q ] = d;
+      S.dict32.val[ q ] = (float) d;
+      S.reach = std::max( S.reach, std::abs( D.off[ q ] ) );
+   }
+   // (whole tiles of mk_dot: the rows past n hold no entry)
+   const int64_t rows = ceil_div( S.v.n, kFT * 4 ) * ( kFT * 4 );
+   auto masks = std::make_shared< DeviceArray< uint8_t > >();
+   masks->allocate( rows * ( D.count <= 8 ? 1 : 2 ) );
+   if( D.count <= 8 )
+      hipLaunchKernelGGL( ( pairs_encode< V, uint8_t > ), dim3( 4096 ), dim3( kFT ), 0, s, S.v, S.cols,
+                          (const V*) S.vals, D, masks->ptr, rows, &table.ptr->reject );
+   else
+      hipLaunchKernelGGL( ( pairs_encode< V, uint16_t > ), dim3( 4096 ), dim3( kFT ), 0, s, S.v, S.cols,
+                          (const V*) S.vals, D, (uint16_t*) masks->ptr, rows, &table.ptr->reject );
+   TNLMI_HIP( hipGetLastError() );
+   int32_t reject = 0;
+   TNLMI_HIP( hipMemcpyAsync( &reject, &table.ptr->reject, sizeof( reject ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipStreamSynchronize( s ) );
+   if( reject )
+      return;
+   S.masks = masks;
+   S.pairs = D.count;
+   S.ecols.reset();  // (a copy of a CSR matrix's slots is not read any more)
+   S.evals.reset();
+}
+
+void make_masks( Stage& S, hipStream_t s )
+{
+   const char* env = std::getenv( "TNLMI_COLUMN_CODES" );
+   if( S.kind != 1 || S.v.n == 0 || ( env && std::string( env ) == "0" ) )
+      return;
+   switch( S.A->value_type ) {
+      case TNLMI_F64:
+         return make_masks_v< double >( S, s );
+      case TNLMI_F32:
+         return make_masks_v< float >( S, s );
+      case TNLMI_BF16:
+         return make_masks_v< bf16 >( S, s );
+   }
+}
+
+// One iteration by row masks, T: the vectors' type.  p has S.reach + kMaskRoom
+// values of room at both ends, r kMaskRoom at its end.
+constexpr int64_t kMaskRoom = kFT * 4;
+template< typename T, typename X, typename DT, bool MIXED >
+void mask_iteration( const Stage& S, T* r, T* p, X* x, const DT* d, T d0, double* part1, double* part2, double* part3,
+                     const CgDev* cur, CgDev* nxt, const StopRule& R, double delta2, hipStream_t s )
+{
+   constexpr int kR = sizeof( T ) == 8 ? 2 : 4;  // rows per thread: 16 bytes
+   const dim3 grid( kFB ), block( kFT );
+   auto go = [ & ]( auto tag, auto np ) {
+      using M = decltype( tag );
+      constexpr int NP = decltype( np )::value;
+      const M* mask = (const M*) S.masks->ptr;
+      const PairDict< T >* D;
+      if constexpr( sizeof( T ) == 8 )
+         D = &S.dict64;
+      else
+         D = &S.dict32;
+      hipLaunchKernelGGL( ( mk_dot< kR, NP, M, T > ), grid, block, 0, s, S.v.n, *D, mask, (const T*) p, part1, cur );
+      hipLaunchKernelGGL( ( mk_upd< kR, NP, M, T, DT > ), grid, block, 0, s, S.v.n, *D, mask, (const double*) part1, r,
+                          (const T*) p, d, d0, part2, part3, cur );
+   };
+   if( S.pairs <= 5 )
+      go( uint8_t(), std::integral_constant< int, 5 >() );
+   else if( S.pairs <= 7 )
+      go( uint8_t(), std::integral_constant< int, 7 >() );
+   else if( S.pairs <= 8 )
+      go( uint8_t(), std::integral_constant< int, 8 >() );
+   else
+      go( uint16_t(), std::integral_constant< int, 16 >() );
+   hipLaunchKernelGGL( ( mk_dir< kR, MIXED, T, X, DT > ), grid, block, 0, s, S.v.n, (const double*) part1,
+                       (const double*) part2, (const double*) part3, (const T*) r, d, d0, p, x, cur, nxt, R, delta2 );
+}
+
+// the diagonal's one value if it has one, else NAN (n > 0)
+double uniform_diagonal( int64_t n, const double* d, hipStream_t s )
+{
+   DeviceArray< int32_t > other;
+   other.allocate( 1 );
+   TNLMI_HIP( hipMemsetAsync( other.ptr, 0, sizeof( int32_t ), s ) );
+   hipLaunchKernelGGL( varies, dim3( 2048 ), dim3( kFT ), 0, s, n, d, other.ptr );
+   int32_t more = 0;
+   double first = 0;
+   TNLMI_HIP( hipMemcpyAsync( &more, other.ptr, sizeof( more ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipMemcpyAsync( &first, d, sizeof( first ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipStreamSynchronize( s ) );
+   return more ? std::nan( "" ) : first;
+}
 
 // The column codes of a column-major Ellpack / SlicedEllpack matrix, or
 // nothing (more than kCodes distinct offsets).  Set TNLMI_COLUMN_CODES=0 in
@@ -1401,7 +1895,7 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
    const double* d = precond_diagonal( M );
    DeviceArray< double > r, p, Ap, sc;
    DeviceArray< CgDev > dev;
-   r.allocate( n );
+   r.allocate( n + kMaskRoom );
    p.allocate( n );
    Ap.allocate( n );
    sc.allocate( 4 );
@@ -1437,12 +1931,35 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
       dot( n, r.ptr, r.ptr, sc.ptr + 2, w, s );
    hipLaunchKernelGGL( cg_start, dim3( 1 ), dim3( 1 ), 0, s, dev.ptr, sc.ptr + 0, sc.ptr + 1, sc.ptr + 2, R );
    TNLMI_HIP( hipGetLastError() );
-   const Stage S = make_stage( A.A, A.plan, s, column_codes );
+   Stage S = make_stage( A.A, A.plan, s );
+   const bool resident = grid && S.A->value_type == TNLMI_F64 && grid_cg_takes( S );
+   if( ! resident ) {
+      make_masks( S, s );
+      if( column_codes && S.kind == 1 && ! S.pairs )
+         make_codes( S, s );
+   }
+   DeviceArray< double > room;
+   double* pp = p.ptr;
+   double d0 = 1.0;  // (r / 1 is r: no preconditioner)
+   const double* dv = d;
+   if( S.pairs ) {
+      const int64_t at = S.reach + kMaskRoom;
+      room.allocate( n + 2 * at );
+      pp = room.ptr + at;
+      TNLMI_HIP( hipMemcpyAsync( pp, p.ptr, sizeof( double ) * n, hipMemcpyDeviceToDevice, s ) );
+      TNLMI_HIP( hipStreamSynchronize( s ) );
+      p.reset();
+      if( d ) {
+         d0 = uniform_diagonal( n, d, s );
+         if( ! std::isnan( d0 ) )
+            dv = nullptr;
+      }
+   }
    // the state is double-buffered by iteration parity: iteration k reads
    // dev[k & 1] and its last kernel writes dev[(k + 1) & 1]
    int par = 0;
    const CgDev* h = &hs.read( dev.ptr, s );
-   if( grid && h->active && S.A->value_type == TNLMI_F64 && grid_cg_takes( S ) ) {
+   if( resident && h->active ) {
       GridWork< double > work( n, s );
       GridCg< double, double > a{};
       a.r = r.ptr;
@@ -1464,8 +1981,13 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
    while( h->active ) {
       for( int k = 0; k < kBatch; k++, par ^= 1 ) {
          CgDev* cur = dev.ptr + par;
-         stage_launch< double >( S, p.ptr, Ap.ptr, parts.a.ptr, cur, s );
          double* part3 = residue_kind == 1 ? parts.c.ptr : nullptr;
+         if( S.pairs ) {
+            mask_iteration< double, double, double, false >( S, r.ptr, pp, x, dv, d0, parts.a.ptr, parts.b.ptr, part3,
+                                                             cur, dev.ptr + ( par ^ 1 ), R, 0.0, s );
+            continue;
+         }
+         stage_launch< double >( S, p.ptr, Ap.ptr, parts.a.ptr, cur, s );
          hipLaunchKernelGGL( ( cg_upd< double, double, double > ), dim3( blocks_of< double >() ), dim3( kFT ), 0, s, n,
                              parts.a.ptr,
                              r.ptr, p.ptr, Ap.ptr, x, d, parts.b.ptr, part3, cur );
@@ -1524,7 +2046,7 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
       for( auto* v : { &r64, &d64 } )
          v->allocate( n );
       for( auto* v : { &r, &p, &Ap, &xc, &d32 } )
-         v->allocate( n );
+         v->allocate( n + kMaskRoom );
       sc.allocate( 4 );
       dev.allocate( 2 );
       TNLMI_HIP( hipMemsetAsync( p.ptr, 0, sizeof( float ) * n, s ) );
@@ -1532,12 +2054,14 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
       RedWork w;
       HostState hs;
       // Jacobi: d = diag(A) (Diagonal.hpp:27-30); d32 = (float) d
+      double dia;
       {
          tnlmi_preconditioner* M = nullptr;
          const tnlmi_status rc = tnlmi_preconditioner_create( TNLMI_PRECOND_DIAGONAL, A, stream, &M );
          if( rc != TNLMI_OK )
             fail( rc, tnlmi_last_error() );
          hipLaunchKernelGGL( to_f32< double >, dim3( kFB32 ), dim3( kFT ), 0, s, n, precond_diagonal( M ), d32.ptr );
+         dia = n > kGridRows ? uniform_diagonal( n, precond_diagonal( M ), s ) : std::nan( "" );
          TNLMI_HIP( hipStreamSynchronize( s ) );
          tnlmi_preconditioner_destroy( M );
       }
@@ -1556,8 +2080,20 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
          return;
       }
       Stage S = make_stage( A_lo, nullptr, s );
-      if( S.kind == 1 && ! grid_cg_takes( S ) )
-         make_codes( S, s );
+      if( S.kind == 1 && ! grid_cg_takes( S ) ) {
+         make_masks( S, s );
+         if( ! S.pairs )
+            make_codes( S, s );
+      }
+      DeviceArray< float > room;
+      float* pp = p.ptr;
+      if( S.pairs ) {
+         const int64_t at = S.reach + kMaskRoom;
+         room.allocate( n + 2 * at );
+         TNLMI_HIP( hipMemsetAsync( room.ptr, 0, sizeof( float ) * ( n + 2 * at ), s ) );
+         pp = room.ptr + at;
+         p.reset();
+      }
       const StopRule R{ st->max_iterations, st->min_iterations, st->convergence_residue, st->divergence_residue };
       int64_t it = 0;
       double res = 0;
@@ -1580,11 +2116,11 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
             break;
          // replace the FP32 residual by the FP64 one and form the next direction
          CgDev* cur = dev.ptr + par;
-         hipLaunchKernelGGL( mx_restart, dim3( kFB32 ), dim3( kFT ), 0, s, n, r64.ptr, r.ptr, d32.ptr, p.ptr, xc.ptr,
+         hipLaunchKernelGGL( mx_restart, dim3( kFB32 ), dim3( kFT ), 0, s, n, r64.ptr, r.ptr, d32.ptr, pp, xc.ptr,
                              parts.a.ptr, parts.b.ptr, parts.c.ptr );
          hipLaunchKernelGGL( mx_state, dim3( 1 ), dim3( kFT ), 0, s, cur, parts.a.ptr, parts.b.ptr, parts.c.ptr,
                              sc.ptr + 0, it, first ? 1 : 0, kFB32 );
-         hipLaunchKernelGGL( mx_redir, dim3( kFB32 ), dim3( kFT ), 0, s, n, r.ptr, d32.ptr, p.ptr, cur,
+         hipLaunchKernelGGL( mx_redir, dim3( kFB32 ), dim3( kFT ), 0, s, n, r.ptr, d32.ptr, pp, cur,
                              first ? 1 : 0 );
          first = false;
          const CgDev* h = nullptr;
@@ -1620,6 +2156,12 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
          while( ! late && ( ! h || ( ! grid && h->active ) ) ) {
             for( int k = 0; k < kBatch; k++, par ^= 1 ) {
                cur = dev.ptr + par;
+               if( S.pairs ) {
+                  mask_iteration< float, float, float, true >(
+                     S, r.ptr, pp, xc.ptr, std::isnan( dia ) ? d32.ptr : nullptr, (float) dia, parts.a.ptr, parts.b.ptr,
+                     parts.c.ptr, cur, dev.ptr + ( par ^ 1 ), R, delta * delta, s );
+                  continue;
+               }
                stage_launch< float >( S, p.ptr, Ap.ptr, parts.a.ptr, cur, s );
                hipLaunchKernelGGL( ( cg_upd< float, float, float > ), dim3( kFB32 ), dim3( kFT ), 0, s, n, parts.a.ptr,
                                    r.ptr, p.ptr, Ap.ptr, xc.ptr, d32.ptr, parts.b.ptr, parts.c.ptr, cur );
