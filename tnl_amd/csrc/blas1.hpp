@@ -48,4 +48,32 @@ void rsub( int64_t n, const double* x, double* y, hipStream_t s );
 void copy( int64_t n, const double* x, double* y, hipStream_t s );
 void fill( int64_t n, double v, double* y, hipStream_t s );
 
+constexpr int kDotGroup = 8;  // columns of V summed together (the multi-dot's first pass)
+
+// A wave's 64 lanes hold the partial sums of kDotGroup columns each; three
+// halving steps (4 + 2 + 1 exchanges) leave lane l with column l >> 3 summed
+// over the 8 lanes that share bits 5..3 of l, and three more exchanges sum
+// those 8 lanes.
+__device__ __forceinline__ double wave_sum_group( double ( &acc )[ kDotGroup ] )
+{
+   static_assert( kDotGroup == 8, "three halving steps" );
+   const int lane = threadIdx.x & 63;
+#pragma unroll
+   for( int o = 32, m = kDotGroup / 2; m >= 1; o /= 2, m /= 2 ) {
+      const bool upper = lane & o;
+#pragma unroll
+      for( int j = 0; j < m; j++ ) {
+         // keep one half of the columns, send the other to the partner lane
+         const double keep = upper ? acc[ j + m ] : acc[ j ];
+         const double send = upper ? acc[ j ] : acc[ j + m ];
+         acc[ j ] = keep + __shfl_xor( send, o, 64 );
+      }
+   }
+   double t = acc[ 0 ];
+   t += __shfl_xor( t, 4, 64 );
+   t += __shfl_xor( t, 2, 64 );
+   t += __shfl_xor( t, 1, 64 );
+   return t;
+}
+
 }  // namespace tnlmi

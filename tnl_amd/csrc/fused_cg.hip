@@ -2009,6 +2009,23 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
 
 }  // namespace
 
+bool ell_slots( const Operator& A, EllSlots& out, hipStream_t s )
+{
+   if( A.plan || A.A->value_type != TNLMI_F64 || A.rows > kGridRows )
+      return false;
+   const Stage S = make_stage( A.A, nullptr, s );
+   if( ! grid_cg_takes( S ) )
+      return false;
+   out.n = S.v.n;
+   out.stride = S.v.ell_aligned;
+   out.w = S.v.ell_width;
+   out.cols = S.cols;
+   out.vals = (const double*) S.vals;
+   out.own_cols = S.ecols;
+   out.own_vals = S.evals;
+   return true;
+}
+
 void fused_cg_solve( const Operator& A, const tnlmi_preconditioner* M, const double* b, double* x,
                      tnlmi_solver_state* st, hipStream_t s, int residue_kind, bool column_codes )
 {

@@ -10,7 +10,7 @@
 namespace tnlmi {
 
 constexpr int kGridMax = 256;        // workgroups at most: one per CU
-constexpr int kGridValues = 4;       // values per sum at most
+constexpr int kGridValues = 32;      // values per sum at most
 constexpr uint64_t kGridWait = 200'000'000;  // 100 MHz ticks (2 s) until a wait gives up
 
 // One value of one workgroup: two words, each with half of the value and the
@@ -113,6 +113,83 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
    for( int j = 0; j < N; j++ )
       v[ j ] = wave_uniform( block_total( j ) );
    __syncthreads();  // (sm may be written again)
+   return ! late;
+}
+
+// A barrier: what a workgroup shared_stores before it is seen by all after it.
+template< int T >
+__device__ __forceinline__ bool grid_barrier( GridSlots* __restrict__ slots, uint32_t number, double* sm )
+{
+   double none[ 1 ] = { 0 };
+   return grid_sum< T >( none, slots, number, sm );
+}
+
+// grid_sum of `count` values whose wave totals are in sm[ j * T / 64 + wave ]
+// already; the results in out[ j ] (LDS).  sm: kGridValues * T / 64 doubles.
+// Each wave polls 64 workgroups' slots of one value at a time.
+template< int T >
+__device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict__ slots, uint32_t number, double* sm,
+                                               double* out )
+{
+   constexpr int W = T / 64, kAtOnce = 4;
+   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, G = gridDim.x;
+   shared_stores_done();
+   __syncthreads();
+   uint64_t( &buf )[ kGridValues ][ kGridMax ][ 2 ] = slots->word[ number & 1 ];
+   if( (int) threadIdx.x < count ) {
+      double r = 0;
+#pragma unroll
+      for( int i = 0; i < W; i++ )
+         r += sm[ threadIdx.x * W + i ];
+      const uint64_t bits = (uint64_t) __double_as_longlong( r );
+      const uint64_t tag = (uint64_t) number << 32;
+      shared_store( &buf[ threadIdx.x ][ blockIdx.x ][ 0 ], tag | ( bits & 0xffffffffu ) );
+      shared_store( &buf[ threadIdx.x ][ blockIdx.x ][ 1 ], tag | ( bits >> 32 ) );
+   }
+   __syncthreads();  // (sm is read above and written below)
+   const int quarters = ( G + 63 ) / 64, jobs = count * quarters;  // job: value job / quarters, slots of quarter job % quarters
+   int late = 0;
+   for( int job0 = w * kAtOnce; job0 < jobs; job0 += W * kAtOnce ) {
+      uint64_t lo[ kAtOnce ], hi[ kAtOnce ];
+      const uint64_t begin = wall_clock64();
+      while( true ) {
+         bool there = true;
+#pragma unroll
+         for( int u = 0; u < kAtOnce; u++ ) {
+            const int job = min( job0 + u, jobs - 1 ), slot = min( job % quarters * 64 + lane, G - 1 );
+            lo[ u ] = shared_load( &buf[ job / quarters ][ slot ][ 0 ] );
+            hi[ u ] = shared_load( &buf[ job / quarters ][ slot ][ 1 ] );
+         }
+#pragma unroll
+         for( int u = 0; u < kAtOnce; u++ )
+            there = there && (uint32_t) ( lo[ u ] >> 32 ) == number && (uint32_t) ( hi[ u ] >> 32 ) == number;
+         if( __ballot( ! there ) == 0 )
+            break;
+         if( wall_clock64() - begin > kGridWait ) {
+            late = 1;
+            break;
+         }
+      }
+#pragma unroll
+      for( int u = 0; u < kAtOnce; u++ ) {
+         const int job = job0 + u;
+         if( job < jobs ) {  // (uniform over the wave)
+            const bool mine = job % quarters * 64 + lane < G;
+            double v = mine ? __longlong_as_double( (long long) ( ( hi[ u ] << 32 ) | ( lo[ u ] & 0xffffffffu ) ) ) : 0.0;
+            v = group_sum< 64 >( v );
+            if( lane == 0 )
+               sm[ job ] = v;
+         }
+      }
+   }
+   late = __syncthreads_or( late );
+   if( (int) threadIdx.x < count ) {
+      double r = 0;
+      for( int q = 0; q < quarters; q++ )
+         r += sm[ threadIdx.x * quarters + q ];
+      out[ threadIdx.x ] = r;
+   }
+   __syncthreads();
    return ! late;
 }
 

@@ -1520,6 +1520,42 @@ void gmres_solve( const Operator& A, const tnlmi_preconditioner* M, const double
          hipLaunchKernelGGL( cwy_add_y, dim3( 1 ), dim3( 64 ), 0, s, x, G, L, k );
       }
    };
+   // whole cycles in one resident launch, where the matrix and preconditioner allow
+   ResidentGmres q{};
+   if( ! cwy && ! inner && ( ! pre || M->kind == TNLMI_PRECOND_DIAGONAL ) && S.check() && ell_slots( A, q.A, s ) ) {
+      auto work = resident_work( n, s );
+      q.d = precond_diagonal( M );
+      q.b = b;
+      q.r = r.ptr;
+      q.V = V.ptr;
+      q.x = x;
+      q.ld = ld;
+      q.classical = classical;
+      q.passes = passes;
+      q.rmin = rmin;
+      q.rmax = rmax;
+      q.dmin = dmin;
+      q.dmax = dmax;
+      q.normb = hs.read( G + L.sc, 1, s )[ 0 ];
+      ResidentEnd end = kResidentMore;
+      while( end == kResidentMore && S.check() )
+         end = resident_gmres( *work, q, S, beta, beta_ratio, cycles, m, s );
+      if( end == kResidentZeroPivot )
+         fail( TNLMI_RUNTIME_ERROR, "GMRES: zero on the diagonal of the Hessenberg matrix" );
+      if( end == kResidentStopped || end == kResidentMore ) {
+         st->iterations = S.it;
+         st->residue = S.res;
+         st->converged = S.converged();
+         return;
+      }
+      // nothing was launched, or a sum was given up: launch by launch from x
+      compute_residue();
+      nrm2( n, r.ptr, G + L.sc + 1, rw, s );
+      hipLaunchKernelGGL( gm_residue_beta, dim3( 1 ), dim3( 1 ), 0, s, G, L );
+      const double* h = hs.read( G + L.sc, 4, s );
+      beta = h[ 1 ];
+      S.res = h[ 3 ];
+   }
    while( S.check() ) {
       if( rmax > rmin && cycles > 0 ) {  // Baker-Jessup-Kolev adaptive restart, :121-146
          if( beta_ratio > 0.99 )

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cmath>
+#include <memory>
 
 #include "common.hpp"
 
@@ -87,5 +88,56 @@ struct HostScalars
 // matrix of few distinct column offsets (as the mixed solver's inner matrix).
 void fused_cg_solve( const Operator& A, const tnlmi_preconditioner* M, const double* b, double* x,
                      tnlmi_solver_state* st, hipStream_t s, int residue_kind = 0, bool column_codes = false );
+
+// ---- solvers whose iterations run in one resident launch (krylov_resident.hip)
+
+// An FP64 matrix's rows as column-major Ellpack slots: its own, or a copy of a
+// CSR matrix's with short rows of about one length.
+struct EllSlots
+{
+   int64_t n = 0, stride = 0;
+   int32_t w = 0;
+   const int32_t* cols = nullptr;
+   const double* vals = nullptr;
+   std::shared_ptr< void > own_cols, own_vals;
+};
+// false: the matrix has no such slots, or more rows than a resident launch takes
+bool ell_slots( const Operator& A, EllSlots& out, hipStream_t s );
+
+// BiCGStab's iterations from an admitted one on (sc: the solver's scalars).
+// Returns what ended them, or kResidentNot when nothing was launched.
+enum ResidentEnd { kResidentNot, kResidentStopped, kResidentMore, kResidentRestart, kResidentLate, kResidentZeroPivot };
+
+struct ResidentState  // on the device, and its host copy
+{
+   double res, beta, normb, beta_ratio;
+   int64_t it;
+   int32_t end, cycles, m, pad;
+};
+
+struct ResidentBicgstab
+{
+   EllSlots A;
+   const double *d, *rast;  // Jacobi diagonal (or NULL); the shadow residual
+   double *r, *p, *Ap, *x, *sc;
+   double b_norm, eps2;
+};
+class Resident;  // work space of a solve
+std::shared_ptr< Resident > resident_work( int64_t n, hipStream_t s );
+ResidentEnd resident_bicgstab( Resident& w, const ResidentBicgstab& a, Stop& S, hipStream_t s );
+
+struct ResidentGmres
+{
+   EllSlots A;
+   const double *d, *b;
+   double *r, *V, *x;
+   int64_t ld;
+   bool classical;
+   int passes, rmin, rmax, dmin, dmax;
+   double normb;
+};
+// whole cycles from S, beta and r on; x, r, beta, S, cycles and beta_ratio as they end
+ResidentEnd resident_gmres( Resident& w, const ResidentGmres& a, Stop& S, double& beta, double& beta_ratio, int& cycles,
+                            int& m, hipStream_t s );
 
 }  // namespace tnlmi

@@ -167,6 +167,54 @@ void bicgstab_solve( const Operator& A, const tnlmi_preconditioner* M, bool exac
    hipLaunchKernelGGL( bs_init, dim3( 1 ), dim3( 1 ), 0, s, sc.ptr );
    const double eps2 = std::numeric_limits< double >::epsilon() * std::numeric_limits< double >::epsilon();
    S.res = std::sqrt( hs.read( sc.ptr + kRho, 1, s )[ 0 ] ) / b_norm;
+   // (r, r*) = too small: restart with r* = r = M^-1 (b - A x); the next direction into pn
+   auto restart = [ & ]() {
+      presidue( A, M, x, b, r.ptr, tmp.ptr, s );
+      copy( n, r.ptr, rast.ptr, s );
+      dot( n, r.ptr, r.ptr, sc.ptr + kRhoNew, w, s );
+      hipLaunchKernelGGL( bs_restart, dim3( 1 ), dim3( 1 ), 0, s, sc.ptr );
+      hipLaunchKernelGGL( bs_dir, vg( n ), dim3( 256 ), 0, s, n, r.ptr, p.ptr, Ap.ptr, pn.ptr, sc.ptr );
+   };
+   const bool jacobi = pre && precond_kind( M ) == TNLMI_PRECOND_DIAGONAL;
+   ResidentBicgstab q{};
+   if( ! exact && ( ! pre || jacobi ) && ell_slots( A, q.A, s ) ) {
+      auto work = resident_work( n, s );
+      q.d = precond_diagonal( M );
+      q.rast = rast.ptr;
+      q.r = r.ptr;
+      q.p = p.ptr;
+      q.Ap = Ap.ptr;
+      q.x = x;
+      q.sc = sc.ptr;
+      q.b_norm = b_norm;
+      q.eps2 = eps2;
+      ResidentEnd end = kResidentMore;
+      bool admitted = S.next();
+      while( admitted ) {
+         end = resident_bicgstab( *work, q, S, s );
+         if( end == kResidentRestart ) {
+            restart();
+            nrm2( n, r.ptr, sc.ptr + kRnorm, w, s );
+            std::swap( p.ptr, pn.ptr );
+            q.p = p.ptr;
+            S.res = hs.read( sc.ptr + kRnorm, 1, s )[ 0 ] / b_norm;
+            admitted = S.next();
+         }
+         else if( end != kResidentMore )
+            break;
+      }
+      if( end == kResidentStopped || ! admitted ) {
+         finish( st, S );
+         return;
+      }
+      // nothing was launched, or a sum was given up: launch by launch from x
+      S.it--;
+      presidue( A, M, x, b, r.ptr, tmp.ptr, s );
+      copy( n, r.ptr, p.ptr, s );
+      copy( n, r.ptr, rast.ptr, s );
+      dot( n, r.ptr, rast.ptr, sc.ptr + kRhoNew, w, s );
+      hipLaunchKernelGGL( bs_init, dim3( 1 ), dim3( 1 ), 0, s, sc.ptr );
+   }
    while( S.next() ) {
       pmatvec( A, M, p.ptr, Ap.ptr, tmp.ptr, s );
       dot( n, Ap.ptr, rast.ptr, sc.ptr + kApR, w, s );
@@ -185,12 +233,8 @@ void bicgstab_solve( const Operator& A, const tnlmi_preconditioner* M, bool exac
       const double* h = hs.read( sc.ptr + kRnorm, 2, s );  // ||r||, restart flag
       double rnorm = h[ 0 ];
       if( h[ 1 ] != 0.0 ) {
-         // r has become too orthogonal to r*: restart with r* = r = M^{-1}(b - A x)
-         presidue( A, M, x, b, r.ptr, tmp.ptr, s );
-         copy( n, r.ptr, rast.ptr, s );
-         dot( n, r.ptr, r.ptr, sc.ptr + kRhoNew, w, s );
-         hipLaunchKernelGGL( bs_restart, dim3( 1 ), dim3( 1 ), 0, s, sc.ptr );
-         hipLaunchKernelGGL( bs_dir, vg( n ), dim3( 256 ), 0, s, n, r.ptr, p.ptr, Ap.ptr, pn.ptr, sc.ptr );
+         // r has become too orthogonal to r*
+         restart();
          if( ! exact ) {
             nrm2( n, r.ptr, sc.ptr + kRnorm, w, s );
             rnorm = hs.read( sc.ptr + kRnorm, 1, s )[ 0 ];
