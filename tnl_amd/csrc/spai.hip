@@ -56,7 +56,6 @@ __host__ __device__ constexpr int64_t obh( int l )
 }
 enum { mWe = 0, mWu = 1, mWv = 2, mWh = 3, mWg = 4 };
 
-typedef short s4 __attribute__( ( ext_vector_type( 4 ) ) );
 typedef float f4 __attribute__( ( ext_vector_type( 4 ) ) );
 
 __device__ __forceinline__ uint16_t bf( float f )
@@ -70,165 +69,237 @@ __device__ __forceinline__ float fb( uint16_t b )
 
 // ------------------------------------------------------------- dense layers
 // Y[R x 64] = sum_t X_t[R x 64] B_t[64 x 64], X_t BF16 row-major, B_t given
-// as Bn[n][k] = B[k][n] (BF16).  Block: 4 wavefronts x 16 rows; each
-// wavefront the full 64 columns (4 column blocks x 4 k-steps of 16).
-// MFMA 16x16x16 operand layout: A lane l holds A[l % 16][4 (l / 16) + 0..3],
-// B lane l holds B[4 (l / 16) + 0..3][l % 16], C lane l holds
-// C[4 (l / 16) + i][l % 16], i = 0..3.
+// as Bn[n][k] = B[k][n] (BF16).  A wavefront has all of B_t in registers (as the
+// first operand of v_mfma_f32_16x16x32_bf16, so that a lane ends up with 4
+// consecutive columns of one row: 8- and 16-byte epilogue accesses) and takes
+// kTiles tiles of 16 rows.  Bound by memory (32 flop per byte): the layer over
+// 326 K edges (EPI_EDGE) takes 40 us for 84 MB of edges and 84 + 84 MB of gathered
+// P and Q, most of them in L2, against 89 us with 16x16x16 products, weights read
+// per 16 rows and 2-byte stores; the backward one (EPI_DEDGE) 41 us against 70 + 66
+// us for the product and a separate pass.
+// MFMA 16x16x32 operand layout: lane l holds row l % 16, k = 8 (l / 16) + 0..7
+// of either operand (any order of k would do: both have the same), and of the
+// result rows 4 (l / 16) + 0..3 (columns of Y), column l % 16 (a row of Y).
+typedef __bf16 bf8 __attribute__( ( ext_vector_type( 8 ) ) );
+typedef uint16_t u4 __attribute__( ( ext_vector_type( 4 ) ) );
 struct Term
 {
    const uint16_t* X;
    const uint16_t* Bn;
 };
-enum Epi { EPI_STORE = 0, EPI_ADD = 1, EPI_EDGE = 2, EPI_NODE = 3 };
+enum Epi { EPI_STORE = 0, EPI_EDGE, EPI_NODE, EPI_DNODE, EPI_DMEAN, EPI_DEDGE };
 struct EpiArgs
 {
-   float* yf;            // EPI_STORE / EPI_ADD (FP32 out)
-   uint16_t* yb;         // EPI_EDGE / EPI_NODE (BF16 out)
+   float* yf;            // EPI_STORE, EPI_DMEAN (FP32 out)
+   uint16_t* yb;         // the others (BF16 out)
    const float* bias;    // EPI_EDGE / EPI_NODE
-   const float* P;       // EPI_EDGE: + P[col[r]] + Q[row[r]]
+   const float* P;       // EPI_EDGE: + P[col[r]] + Q[row[r]];  EPI_DEDGE: + P[row[r]]
    const float* Q;
    const int32_t* col;
    const int32_t* row;
+   const uint16_t* mask;  // EPI_DNODE / EPI_DEDGE: 0 where the activation is not positive
+   const int32_t* deg;    // EPI_DMEAN: / deg[r]
 };
 
-template< int NT, int EPI >
+__device__ __forceinline__ f4 relu4( f4 v )
+{
+   return f4{ fmaxf( v[ 0 ], 0.f ), fmaxf( v[ 1 ], 0.f ), fmaxf( v[ 2 ], 0.f ), fmaxf( v[ 3 ], 0.f ) };
+}
+__device__ __forceinline__ u4 bf4( f4 v )
+{
+   return u4{ bf( v[ 0 ] ), bf( v[ 1 ] ), bf( v[ 2 ] ), bf( v[ 3 ] ) };
+}
+// v where the activation m is positive
+__device__ __forceinline__ f4 masked4( u4 m, f4 v )
+{
+#pragma unroll
+   for( int i = 0; i < 4; i++ )
+      v[ i ] = fb( m[ i ] ) > 0.f ? v[ i ] : 0.f;
+   return v;
+}
+
+template< int NT, int EPI, int kTiles >
 __global__ void __launch_bounds__( 256 ) gemm64( int64_t R, Term t0, Term t1, Term t2, EpiArgs e )
 {
    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-   const int64_t r0 = (int64_t) blockIdx.x * 64 + w * 16;
-   const int lr = lane & 15, lk = 4 * ( lane >> 4 );
-   f4 acc[ 4 ];
-#pragma unroll
-   for( int cb = 0; cb < 4; cb++ )
-      acc[ cb ] = f4{ 0.f, 0.f, 0.f, 0.f };
+   const int lr = lane & 15, lq = lane >> 4;
    const Term ts[ 3 ] = { t0, t1, t2 };
+   bf8 B[ NT ][ 4 ][ 2 ];
 #pragma unroll
-   for( int t = 0; t < NT; t++ ) {
-      const int64_t ra = r0 + lr;
+   for( int t = 0; t < NT; t++ )
 #pragma unroll
-      for( int kb = 0; kb < 4; kb++ ) {
-         s4 a = s4{ 0, 0, 0, 0 };
-         if( ra < R )
-            a = *(const s4*) ( ts[ t ].X + ra * kH + kb * 16 + lk );
+      for( int nb = 0; nb < 4; nb++ )
 #pragma unroll
-         for( int cb = 0; cb < 4; cb++ ) {
-            const s4 b = *(const s4*) ( ts[ t ].Bn + ( cb * 16 + lr ) * kH + kb * 16 + lk );
-            acc[ cb ] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k( a, b, acc[ cb ], 0, 0, 0 );
+         for( int kb = 0; kb < 2; kb++ )
+            B[ t ][ nb ][ kb ] = *(const bf8*) ( ts[ t ].Bn + ( nb * 16 + lr ) * kH + kb * 32 + lq * 8 );
+   const int64_t base = ( (int64_t) blockIdx.x * 4 + w ) * ( 16 * kTiles );
+#pragma unroll
+   for( int tile = 0; tile < kTiles; tile++ ) {
+      const int64_t r = base + tile * 16 + lr;
+      if( base + tile * 16 >= R )  // (uniform)
+         return;
+      const int64_t rc = r < R ? r : R - 1;  // a last tile's rows past R: read again, not stored
+      f4 acc[ 4 ];
+#pragma unroll
+      for( int nb = 0; nb < 4; nb++ )
+         acc[ nb ] = f4{ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+      for( int t = 0; t < NT; t++ )
+#pragma unroll
+         for( int kb = 0; kb < 2; kb++ ) {
+            const bf8 x = *(const bf8*) ( ts[ t ].X + rc * kH + kb * 32 + lq * 8 );
+#pragma unroll
+            for( int nb = 0; nb < 4; nb++ )
+               acc[ nb ] = __builtin_amdgcn_mfma_f32_16x16x32_bf16( B[ t ][ nb ][ kb ], x, acc[ nb ], 0, 0, 0 );
          }
-      }
-   }
+      int32_t j = 0, i = 0;
+      float d = 1.f;
+      if( EPI == EPI_EDGE )
+         j = e.col[ rc ];  // -1: a padding slot, no edge
+      if( EPI == EPI_EDGE || EPI == EPI_DEDGE )
+         i = e.row[ rc ];
+      if( EPI == EPI_DMEAN )
+         d = (float) e.deg[ rc ];
 #pragma unroll
-   for( int cb = 0; cb < 4; cb++ ) {
-      const int c = cb * 16 + lr;
-#pragma unroll
-      for( int i = 0; i < 4; i++ ) {
-         const int64_t r = r0 + lk + i;
-         if( r >= R )
-            continue;
-         const float v = acc[ cb ][ i ];
-         if( EPI == EPI_STORE )
-            e.yf[ r * kH + c ] = v;
-         else if( EPI == EPI_ADD )
-            e.yf[ r * kH + c ] += v;
-         else if( EPI == EPI_EDGE ) {
-            const int32_t j = e.col[ r ];  // -1: a padding slot, no edge
-            const float pj = j >= 0 ? e.P[ (int64_t) j * kH + c ] : 0.f;
-            e.yb[ r * kH + c ] = bf( fmaxf( v + pj + e.Q[ (int64_t) e.row[ r ] * kH + c ] + e.bias[ c ], 0.f ) );
+      for( int nb = 0; nb < 4; nb++ ) {
+         const int c = nb * 16 + lq * 4;
+         f4 v = acc[ nb ];
+         if( EPI == EPI_EDGE ) {
+            const f4 p = j >= 0 ? *(const f4*) ( e.P + (int64_t) j * kH + c ) : f4{ 0.f, 0.f, 0.f, 0.f };
+            v = v + p + *(const f4*) ( e.Q + (int64_t) i * kH + c ) + *(const f4*) ( e.bias + c );
          }
-         else
-            e.yb[ r * kH + c ] = bf( fmaxf( v + e.bias[ c ], 0.f ) );
+         else if( EPI == EPI_NODE )
+            v = v + *(const f4*) ( e.bias + c );
+         else if( EPI == EPI_DMEAN )
+            v = f4{ v[ 0 ] / d, v[ 1 ] / d, v[ 2 ] / d, v[ 3 ] / d };
+         else if( EPI == EPI_DEDGE )
+            v = v + *(const f4*) ( e.P + (int64_t) i * kH + c );
+         if( EPI == EPI_EDGE || EPI == EPI_NODE )
+            v = relu4( v );
+         if( EPI == EPI_DNODE || EPI == EPI_DEDGE )
+            v = masked4( *(const u4*) ( e.mask + rc * kH + c ), v );
+         if( r < R ) {
+            if( EPI == EPI_STORE || EPI == EPI_DMEAN )
+               *(f4*) ( e.yf + r * kH + c ) = v;
+            else
+               *(u4*) ( e.yb + r * kH + c ) = bf4( v );
+         }
       }
    }
 }
 
-// dW[64 x 64] = X^T dY over R rows (and the column sums of dY): per block of
-// kWRows rows a partial product from LDS-staged tiles, summed over the blocks
-// in a fixed order by reduce_partials (chunks of consecutive blocks, then the
-// chunk sums).
+// dW[64 x 64] = X^T dY over R rows and the column sums of dY.  A workgroup takes
+// tiles of kWRows rows in turn, sums in registers and leaves one partial: the
+// rows are the k of the products, so a tile goes to LDS transposed (two rows'
+// values packed per 32-bit write) and the fragments are 16-byte LDS reads.  The
+// column sums are a product with ones.  The next tile's loads are in flight
+// while a tile is multiplied.  326 K rows 26 us (84 MB) against 35 us, with 512
+// partials instead of 1,276.
+constexpr int kWStride = kWRows + 8;  // (16-byte reads of 16 features on different banks)
+constexpr int kPart = kH * kH + kH;   // a partial: dW, then the column sums
+constexpr int kWBlocks = 512;         // partials at most (two workgroups per CU)
+
 __global__ void __launch_bounds__( 256 ) wgrad64( int64_t R, const uint16_t* __restrict__ X,
-                                                  const uint16_t* __restrict__ dY, float* __restrict__ part,
-                                                  float* __restrict__ bpart )
+                                                  const uint16_t* __restrict__ dY, float* __restrict__ part )
 {
-   __shared__ uint16_t sx[ kWRows * kH ], sy[ kWRows * kH ];
-   const int64_t base = (int64_t) blockIdx.x * kWRows;
-   // stage the tiles (16 bytes per thread per step), zero past R
-   for( int q = threadIdx.x; q < kWRows * kH / 8; q += 256 ) {
-      const int64_t r = base + q / 8;
-      typedef int i4 __attribute__( ( ext_vector_type( 4 ) ) );
-      i4 vx = i4{ 0, 0, 0, 0 }, vy = i4{ 0, 0, 0, 0 };
-      if( r < R ) {
-         vx = *(const i4*) ( X + base * kH + (int64_t) q * 8 );
-         vy = *(const i4*) ( dY + base * kH + (int64_t) q * 8 );
+   typedef uint16_t u8v __attribute__( ( ext_vector_type( 8 ) ) );
+   __shared__ __align__( 16 ) uint16_t sx[ kH * kWStride ], sy[ kH * kWStride ];
+   // (w known to be uniform: a matrix instruction does not look at the exec mask)
+   const int lane = threadIdx.x & 63, w = wave_uniform( (int32_t) ( threadIdx.x >> 6 ) );
+   const int lr = lane & 15, lq = lane >> 4;
+   const int64_t tiles = ( R + kWRows - 1 ) / kWRows;
+   const int fg = threadIdx.x & 7, rp = threadIdx.x >> 3;  // 8 features of row pairs rp + 32 u
+   u8v x0[ 4 ], x1[ 4 ], y0[ 4 ], y1[ 4 ];
+   auto fetch = [ & ]( int64_t tile ) {
+#pragma unroll
+      for( int u = 0; u < 4; u++ ) {
+         const int64_t r = tile * kWRows + 2 * ( rp + 32 * u );
+         const int64_t a = r < R ? r : R - 1, b = r + 1 < R ? r + 1 : R - 1;
+         x0[ u ] = *(const u8v*) ( X + a * kH + fg * 8 );
+         x1[ u ] = *(const u8v*) ( X + b * kH + fg * 8 );
+         y0[ u ] = *(const u8v*) ( dY + a * kH + fg * 8 );
+         y1[ u ] = *(const u8v*) ( dY + b * kH + fg * 8 );
+         if( r >= R )
+            x0[ u ] = y0[ u ] = u8v{};
+         if( r + 1 >= R )
+            x1[ u ] = y1[ u ] = u8v{};
       }
-      *(i4*) ( sx + q * 8 ) = vx;
-      *(i4*) ( sy + q * 8 ) = vy;
-   }
-   __syncthreads();
-   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-   const int lr = lane & 15, lk = 4 * ( lane >> 4 );
-   f4 acc[ 4 ];
+   };
+   f4 acc[ 4 ], sums = f4{ 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-   for( int cb = 0; cb < 4; cb++ )
-      acc[ cb ] = f4{ 0.f, 0.f, 0.f, 0.f };
-   const int m = w * 16 + lr;  // feature of X = row of dW
-   for( int ks = 0; ks < kWRows / 16; ks++ ) {
-      const int k = ks * 16 + lk;  // row of the tile
-      const s4 a = s4{ (short) sx[ ( k + 0 ) * kH + m ], (short) sx[ ( k + 1 ) * kH + m ],
-                       (short) sx[ ( k + 2 ) * kH + m ], (short) sx[ ( k + 3 ) * kH + m ] };
+   for( int nb = 0; nb < 4; nb++ )
+      acc[ nb ] = f4{ 0.f, 0.f, 0.f, 0.f };
+   const bf8 ones = { (__bf16) 1.f, (__bf16) 1.f, (__bf16) 1.f, (__bf16) 1.f,
+                      (__bf16) 1.f, (__bf16) 1.f, (__bf16) 1.f, (__bf16) 1.f };
+   fetch( blockIdx.x );
+   for( int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x ) {
+      __syncthreads();  // (the tile before is read)
 #pragma unroll
-      for( int cb = 0; cb < 4; cb++ ) {
-         const int n = cb * 16 + lr;
-         const s4 b = s4{ (short) sy[ ( k + 0 ) * kH + n ], (short) sy[ ( k + 1 ) * kH + n ],
-                          (short) sy[ ( k + 2 ) * kH + n ], (short) sy[ ( k + 3 ) * kH + n ] };
-         acc[ cb ] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k( a, b, acc[ cb ], 0, 0, 0 );
+      for( int u = 0; u < 4; u++ )
+#pragma unroll
+         for( int f = 0; f < 8; f++ ) {
+            const int at = ( fg * 8 + f ) * kWStride + 2 * ( rp + 32 * u );
+            *(uint32_t*) ( sx + at ) = (uint32_t) x0[ u ][ f ] | (uint32_t) x1[ u ][ f ] << 16;
+            *(uint32_t*) ( sy + at ) = (uint32_t) y0[ u ][ f ] | (uint32_t) y1[ u ][ f ] << 16;
+         }
+      __syncthreads();
+      if( tile + gridDim.x < tiles )
+         fetch( tile + gridDim.x );
+#pragma unroll
+      for( int ks = 0; ks < kWRows / 32; ks++ ) {
+         const bf8 a = *(const bf8*) ( sx + ( w * 16 + lr ) * kWStride + ks * 32 + lq * 8 );
+#pragma unroll
+         for( int nb = 0; nb < 4; nb++ ) {
+            const bf8 b = *(const bf8*) ( sy + ( nb * 16 + lr ) * kWStride + ks * 32 + lq * 8 );
+            acc[ nb ] = __builtin_amdgcn_mfma_f32_16x16x32_bf16( a, b, acc[ nb ], 0, 0, 0 );
+            if( nb == w )
+               sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16( ones, b, sums, 0, 0, 0 );
+         }
       }
    }
-   float* out = part + (int64_t) blockIdx.x * kH * kH;
+   float* out = part + (int64_t) blockIdx.x * kPart;
 #pragma unroll
-   for( int cb = 0; cb < 4; cb++ )
+   for( int nb = 0; nb < 4; nb++ )
 #pragma unroll
       for( int i = 0; i < 4; i++ )
-         out[ ( w * 16 + lk + i ) * kH + cb * 16 + lr ] = acc[ cb ][ i ];
-   if( bpart && threadIdx.x < kH ) {
-      float sum = 0.f;
-      for( int r = 0; r < kWRows; r++ )
-         sum += fb( sy[ r * kH + threadIdx.x ] );
-      bpart[ (int64_t) blockIdx.x * kH + threadIdx.x ] = sum;
-   }
+         out[ ( w * 16 + lq * 4 + i ) * kH + nb * 16 + lr ] = acc[ nb ][ i ];
+   if( lq == 0 )
+      out[ kH * kH + w * 16 + lr ] = sums[ 0 ];
 }
 
-// out[e] = sum over blocks b (in order) of part[b * width + e]
-__global__ void reduce_parts( const float* __restrict__ part, int64_t nblk, int width, float* __restrict__ out )
+// out[e] (e < split) and out2[e - split] = the sum over nblk partials of
+// part[b * width + e]: 16 waves take consecutive shares of the partials, then
+// their sums in order -- a fixed order.  out2 NULL: those columns are not wanted.
+__global__ void __launch_bounds__( 1024 ) reduce_parts( const float* __restrict__ part, int64_t nblk, int width, int split,
+                                                        float* __restrict__ out, float* __restrict__ out2 )
 {
-   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-   if( e >= width )
-      return;
+   __shared__ float sm[ 16 ][ 64 ];
+   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+   const int e = blockIdx.x * 64 + lane;
+   const int64_t share = ( nblk + 15 ) / 16, b0 = min( nblk, w * share ), b1 = min( nblk, b0 + share );
    float s = 0.f;
-   for( int64_t b = 0; b < nblk; b++ )
-      s += part[ b * width + e ];
-   out[ e ] = s;
-}
-
-// Two-level form of reduce_parts for long partial lists: chunk c of at most
-// L consecutive blocks per column (in block order) by one lane each, then the
-// chunk sums in chunk order -- a fixed order, so deterministic, with
-// (columns / 64) x chunks waves in the first level instead of one thread
-// walking every block.
-constexpr int kRedChunks = 64;
-
-__global__ void __launch_bounds__( 64 ) reduce_parts_chunks( const float* __restrict__ part, int64_t nblk, int width,
-                                                             int64_t L, float* __restrict__ out )
-{
-   const int e = blockIdx.x * 64 + threadIdx.x;
-   if( e >= width )
+   if( e < width )
+      for( int64_t b = b0; b < b1; b += 8 ) {
+         float v[ 8 ];
+#pragma unroll
+         for( int u = 0; u < 8; u++ )
+            v[ u ] = b + u < b1 ? part[ ( b + u ) * width + e ] : 0.f;
+#pragma unroll
+         for( int u = 0; u < 8; u++ )
+            s += v[ u ];
+      }
+   sm[ w ][ lane ] = s;
+   __syncthreads();
+   if( w != 0 || e >= width )
       return;
-   const int64_t c = blockIdx.y;
-   const int64_t b0 = c * L, b1 = std::min< int64_t >( nblk, b0 + L );
-   float s = 0.f;
-   for( int64_t b = b0; b < b1; b++ )
-      s += part[ b * width + e ];
-   out[ c * width + e ] = s;
+   float t = 0.f;
+#pragma unroll
+   for( int i = 0; i < 16; i++ )
+      t += sm[ i ][ lane ];
+   if( e < split )
+      out[ e ] = t;
+   else if( out2 )
+      out2[ e - split ] = t;
 }
 
 // ------------------------------------------------------------ graph and IO
@@ -316,55 +387,58 @@ __global__ void iota_k( int64_t E, const int32_t* __restrict__ cols, uint32_t* _
 }
 
 // ------------------------------------------------------------ forward parts
-// relu(x W + b) for K = 4 inputs (FP32), BF16 out
-__global__ void encode_k( int64_t R, const float* __restrict__ x, const float* __restrict__ W,
-                          const float* __restrict__ b, uint16_t* __restrict__ y )
+// relu(x W + b) for K = 4 inputs (FP32), BF16 out; 4 columns per thread
+__global__ void __launch_bounds__( 256 ) encode_k( int64_t R, const float* __restrict__ x, const float* __restrict__ W,
+                                                   const float* __restrict__ b, uint16_t* __restrict__ y )
 {
-   const int64_t q = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-   if( q >= R * kH )
+   const int64_t q = (int64_t) blockIdx.x * 256 + threadIdx.x, r = q / 16;
+   const int c = (int) ( q % 16 ) * 4;
+   if( r >= R )
       return;
-   const int64_t r = q / kH;
-   const int c = (int) ( q % kH );
-   float v = b[ c ];
+   const f4 xr = *(const f4*) ( x + r * 4 );
+   f4 v = *(const f4*) ( b + c );
 #pragma unroll
    for( int k = 0; k < 4; k++ )
-      v += x[ r * 4 + k ] * W[ k * kH + c ];
-   y[ q ] = bf( fmaxf( v, 0.f ) );
+      v += xr[ k ] * *(const f4*) ( W + k * kH + c );
+   *(u4*) ( y + r * kH + c ) = bf4( relu4( v ) );
 }
 
-// G = BF16 of the mean of the row's edge features
-__global__ void mean_k( int64_t n, const int32_t* __restrict__ off, const uint16_t* __restrict__ E,
-                        uint16_t* __restrict__ G )
+__device__ __forceinline__ f4 fb4( u4 v )
 {
-   const int64_t q = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-   if( q >= n * kH )
+   return f4{ fb( v[ 0 ] ), fb( v[ 1 ] ), fb( v[ 2 ] ), fb( v[ 3 ] ) };
+}
+
+// G = BF16 of the mean of the row's edge features; 4 columns per thread
+__global__ void __launch_bounds__( 256 ) mean_k( int64_t n, const int32_t* __restrict__ off, const uint16_t* __restrict__ E,
+                                                 uint16_t* __restrict__ G )
+{
+   const int64_t q = (int64_t) blockIdx.x * 256 + threadIdx.x, i = q / 16;
+   const int c = (int) ( q % 16 ) * 4;
+   if( i >= n )
       return;
-   const int64_t i = q / kH;
-   const int c = (int) ( q % kH );
-   float s = 0.f;
-   for( int32_t e = off[ i ]; e < off[ i + 1 ]; e++ )
-      s += fb( E[ (int64_t) e * kH + c ] );
-   const int32_t d = off[ i + 1 ] - off[ i ];
-   G[ q ] = bf( d > 0 ? s / (float) d : 0.f );
+   f4 s = f4{ 0.f, 0.f, 0.f, 0.f };
+   const int32_t e0 = off[ i ], d = off[ i + 1 ] - e0;
+   for( int32_t e = 0; e < d; e++ )
+      s += fb4( *(const u4*) ( E + (int64_t) ( e0 + e ) * kH + c ) );
+   if( d > 0 )
+      s = f4{ s[ 0 ] / (float) d, s[ 1 ] / (float) d, s[ 2 ] / (float) d, s[ 3 ] / (float) d };
+   *(u4*) ( G + i * kH + c ) = bf4( s );
 }
 
-// o_e = E_e . wo + bo (FP32), M_e = (delta + o) / a_ii (FP64)
-__global__ void decode_k( int64_t E, const uint16_t* __restrict__ X, const float* __restrict__ wo,
-                          const float* __restrict__ bo, const int32_t* __restrict__ erow,
-                          const int32_t* __restrict__ cols, const uint8_t* __restrict__ isd,
-                          const double* __restrict__ diag, double* __restrict__ M )
+// o_e = E_e . wo + bo (FP32), M_e = (delta + o) / a_ii (FP64); 16 lanes per edge
+__global__ void __launch_bounds__( 256 ) decode_k( int64_t E, const uint16_t* __restrict__ X, const float* __restrict__ wo,
+                                                   const float* __restrict__ bo, const int32_t* __restrict__ erow,
+                                                   const int32_t* __restrict__ cols, const uint8_t* __restrict__ isd,
+                                                   const double* __restrict__ diag, double* __restrict__ M )
 {
-   const int64_t e = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+   const int64_t q = (int64_t) blockIdx.x * 256 + threadIdx.x, e = q / 16;
+   const int c = (int) ( q % 16 ) * 4;
    if( e >= E )
-      return;
-   if( cols[ e ] < 0 ) {
-      M[ e ] = 0.0;
-      return;
-   }
-   float o = bo[ 0 ];
-   for( int c = 0; c < kH; c++ )
-      o += fb( X[ e * kH + c ] ) * wo[ c ];
-   M[ e ] = ( (double) isd[ e ] + (double) o ) / diag[ erow[ e ] ];
+      return;  // (uniform over the 16 lanes)
+   const f4 v = fb4( *(const u4*) ( X + e * kH + c ) ), w = *(const f4*) ( wo + c );
+   const float o = group_sum< 16 >( v[ 0 ] * w[ 0 ] + v[ 1 ] * w[ 1 ] + v[ 2 ] * w[ 2 ] + v[ 3 ] * w[ 3 ] ) + bo[ 0 ];
+   if( c == 0 )
+      M[ e ] = cols[ e ] < 0 ? 0.0 : ( (double) isd[ e ] + (double) o ) / diag[ erow[ e ] ];
 }
 
 // ------------------------------------------------------------ probe loss
@@ -382,11 +456,13 @@ __global__ void rademacher_k( int64_t cnt, uint64_t seed, double* __restrict__ Z
       Z[ q ] = ( mix64( seed * 0x2545f4914f6cdd1dull + (uint64_t) q ) >> 63 ) ? 1.0 : -1.0;
 }
 
-// y = V x over the CSR pattern (one thread per row)
+// y = V x over the CSR pattern (one thread per row; blockIdx.y: the probe)
 __global__ void csr_mv( int64_t n, const int32_t* __restrict__ off, const int32_t* __restrict__ cols,
                         const double* __restrict__ V, const double* __restrict__ x, double* __restrict__ y )
 {
    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+   x += blockIdx.y * n;
+   y += blockIdx.y * n;
    if( i >= n )
       return;
    double s = 0.0;
@@ -402,6 +478,9 @@ __global__ void __launch_bounds__( 256 ) resid_k( int64_t n, const double* __res
 {
    __shared__ double sm[ 4 ];
    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+   z += blockIdx.y * n;
+   w += blockIdx.y * n;
+   part += blockIdx.y * gridDim.x;
    double v = 0.0;
    if( i < n ) {
       const double r = z[ i ] - w[ i ];
@@ -439,96 +518,115 @@ __global__ void dM_k( int64_t E, int64_t n, int K, const int32_t* __restrict__ e
 }
 
 // ------------------------------------------------------------ backward parts
-// do_e = dM_e / a_ii;  dE = do x wo;  per block partial sums of do_e E_e and do_e
+// do_e = dM_e / a_ii;  dS = BF16( do x wo * [E > 0] ) of the last layer (its node
+// features reach nothing);  per wave partial sums of do_e E_e and do_e
 __global__ void __launch_bounds__( 256 ) dec_bwd_k( int64_t E, const double* __restrict__ dM,
                                                     const int32_t* __restrict__ erow, const double* __restrict__ diag,
                                                     const uint16_t* __restrict__ X, const float* __restrict__ wo,
-                                                    float* __restrict__ dE, float* __restrict__ part )
+                                                    uint16_t* __restrict__ dS, float* __restrict__ part )
 {
-   __shared__ float sdo[ 256 ];
-   const int64_t e0 = (int64_t) blockIdx.x * 256;
-   const int64_t e = e0 + threadIdx.x;
-   float d = 0.f;
-   if( e < E )
-      d = (float) ( dM[ e ] / diag[ erow[ e ] ] );
-   sdo[ threadIdx.x ] = d;
-   __syncthreads();
-   const int64_t cnt = min( (int64_t) 256, E - e0 );
-   for( int64_t q = threadIdx.x; q < cnt * kH; q += 256 ) {
-      const int64_t r = e0 + q / kH;
-      const int c = (int) ( q % kH );
-      dE[ r * kH + c ] = sdo[ q / kH ] * wo[ c ];
+   const int lane = threadIdx.x & 63, c = ( lane & 15 ) * 4, sub = lane >> 4;  // 4 columns of every 4th row
+   const f4 wc = *(const f4*) ( wo + c );
+   f4 s = f4{ 0.f, 0.f, 0.f, 0.f };
+   float so = 0.f;
+   constexpr int kAt = 4;  // rows loaded together
+   const int64_t wave = (int64_t) blockIdx.x * 4 + ( threadIdx.x >> 6 ), waves = (int64_t) gridDim.x * 4;
+   for( int64_t r0 = wave * ( 4 * kAt ); r0 < E; r0 += waves * ( 4 * kAt ) ) {
+      float d[ kAt ];
+      u4 v[ kAt ];
+#pragma unroll
+      for( int u = 0; u < kAt; u++ ) {
+         const int64_t r = r0 + u * 4 + sub, q = r < E ? r : E - 1;
+         d[ u ] = r < E ? (float) ( dM[ q ] / diag[ erow[ q ] ] ) : 0.f;
+         v[ u ] = *(const u4*) ( X + q * kH + c );
+      }
+#pragma unroll
+      for( int u = 0; u < kAt; u++ ) {
+         const int64_t r = r0 + u * 4 + sub;
+         s += d[ u ] * fb4( v[ u ] );
+         so += d[ u ];
+         if( r < E )
+            *(u4*) ( dS + r * kH + c ) = bf4( masked4( v[ u ], d[ u ] * wc ) );
+      }
    }
-   if( threadIdx.x < kH + 1 ) {
-      float s = 0.f;
-      for( int64_t r = 0; r < cnt; r++ )
-         s += threadIdx.x < kH ? sdo[ r ] * fb( X[ ( e0 + r ) * kH + threadIdx.x ] ) : sdo[ r ];
-      part[ (int64_t) blockIdx.x * ( kH + 1 ) + threadIdx.x ] = s;
+   float* out = part + wave * ( kH + 1 );
+#pragma unroll
+   for( int i = 0; i < 4; i++ ) {
+      float t = s[ i ];
+      t += __shfl_xor( t, 16, 64 );
+      t += __shfl_xor( t, 32, 64 );
+      if( sub == 0 )
+         out[ c + i ] = t;
    }
+   so += __shfl_xor( so, 16, 64 );
+   so += __shfl_xor( so, 32, 64 );
+   if( lane == 0 )
+      out[ kH ] = so;
 }
 
-// dT = BF16( dH * [H > 0] )
-__global__ void mask_k( int64_t cnt, const float* __restrict__ dX, const uint16_t* __restrict__ Y,
-                        uint16_t* __restrict__ out )
+// dQ_i = BF16( sum over row i of dS ),  dP_j = BF16( sum over column j of dS ); 4 columns per thread
+__global__ void __launch_bounds__( 256 ) scatter_k( int64_t n, const int32_t* __restrict__ off,
+                                                    const int32_t* __restrict__ cptr, const int32_t* __restrict__ cperm,
+                                                    const uint16_t* __restrict__ dS, uint16_t* __restrict__ dP,
+                                                    uint16_t* __restrict__ dQ )
 {
-   const int64_t q = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-   if( q < cnt )
-      out[ q ] = bf( fb( Y[ q ] ) > 0.f ? dX[ q ] : 0.f );
-}
-
-// dS = BF16( (dE + dG[row] / deg[row]) * [E > 0] )
-__global__ void edge_bwd_k( int64_t E, const float* __restrict__ dE, const float* __restrict__ dG,
-                            const int32_t* __restrict__ erow, const int32_t* __restrict__ deg,
-                            const uint16_t* __restrict__ Y, uint16_t* __restrict__ dS )
-{
-   const int64_t q = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-   if( q >= E * kH )
+   const int64_t q = (int64_t) blockIdx.x * 256 + threadIdx.x, i = q / 16;
+   const int c = (int) ( q % 16 ) * 4;
+   if( i >= n )
       return;
-   const int64_t e = q / kH;
-   const int c = (int) ( q % kH );
-   const int32_t i = erow[ e ];
-   const float g = dE[ q ] + dG[ (int64_t) i * kH + c ] / (float) deg[ i ];
-   dS[ q ] = bf( fb( Y[ q ] ) > 0.f ? g : 0.f );
-}
-
-// dQ_i = BF16( sum over row i of dS ),  dP_j = BF16( sum over column j of dS )
-__global__ void scatter_k( int64_t n, const int32_t* __restrict__ off, const int32_t* __restrict__ cptr,
-                           const int32_t* __restrict__ cperm, const uint16_t* __restrict__ dS,
-                           uint16_t* __restrict__ dP, uint16_t* __restrict__ dQ )
-{
-   const int64_t q = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-   if( q >= n * kH )
-      return;
-   const int64_t i = q / kH;
-   const int c = (int) ( q % kH );
-   float sq = 0.f, sp = 0.f;
+   f4 sq = f4{ 0.f, 0.f, 0.f, 0.f }, sp = sq;
    for( int32_t e = off[ i ]; e < off[ i + 1 ]; e++ )
-      sq += fb( dS[ (int64_t) e * kH + c ] );
+      sq += fb4( *(const u4*) ( dS + (int64_t) e * kH + c ) );
    for( int32_t p = cptr[ i ]; p < cptr[ i + 1 ]; p++ )
-      sp += fb( dS[ (int64_t) cperm[ p ] * kH + c ] );
-   dQ[ q ] = bf( sq );
-   dP[ q ] = bf( sp );
+      sp += fb4( *(const u4*) ( dS + (int64_t) cperm[ p ] * kH + c ) );
+   *(u4*) ( dQ + i * kH + c ) = bf4( sq );
+   *(u4*) ( dP + i * kH + c ) = bf4( sp );
 }
 
-// encoder gradients: per block partials of x^T (dX * [Y > 0]) (4 x 64) and
-// of the column sums (64)
+// encoder gradients: per wave partials of x^T (dX * [Y > 0]) (4 x 64) and of the
+// column sums (64)
 __global__ void __launch_bounds__( 256 ) enc_bwd_k( int64_t R, const float* __restrict__ x,
                                                     const float* __restrict__ dX, const uint16_t* __restrict__ Y,
                                                     float* __restrict__ part )
 {
-   const int64_t r0 = (int64_t) blockIdx.x * 256;
-   const int64_t cnt = min( (int64_t) 256, R - r0 );
-   const int c = threadIdx.x & 63, k = threadIdx.x >> 6;  // k = 0..3: input feature
-   float s = 0.f, sb = 0.f;
-   for( int64_t r = r0; r < r0 + cnt; r++ ) {
-      const float g = fb( Y[ r * kH + c ] ) > 0.f ? dX[ r * kH + c ] : 0.f;
-      s += x[ r * 4 + k ] * g;
-      sb += g;
+   const int lane = threadIdx.x & 63, c = ( lane & 15 ) * 4, sub = lane >> 4;  // 4 columns of every 4th row
+   f4 s[ 5 ];  // by input, then the column sums
+#pragma unroll
+   for( int k = 0; k < 5; k++ )
+      s[ k ] = f4{ 0.f, 0.f, 0.f, 0.f };
+   constexpr int kAt = 4;  // rows loaded together
+   const int64_t wave = (int64_t) blockIdx.x * 4 + ( threadIdx.x >> 6 ), waves = (int64_t) gridDim.x * 4;
+   for( int64_t r0 = wave * ( 4 * kAt ); r0 < R; r0 += waves * ( 4 * kAt ) ) {
+      f4 xr[ kAt ], g[ kAt ];
+      u4 y[ kAt ];
+#pragma unroll
+      for( int u = 0; u < kAt; u++ ) {
+         const int64_t r = r0 + u * 4 + sub, q = r < R ? r : R - 1;
+         xr[ u ] = *(const f4*) ( x + q * 4 );
+         g[ u ] = *(const f4*) ( dX + q * kH + c );
+         y[ u ] = *(const u4*) ( Y + q * kH + c );
+      }
+#pragma unroll
+      for( int u = 0; u < kAt; u++ )
+         if( r0 + u * 4 + sub < R ) {
+            const f4 m = masked4( y[ u ], g[ u ] );
+#pragma unroll
+            for( int k = 0; k < 4; k++ )
+               s[ k ] += xr[ u ][ k ] * m;
+            s[ 4 ] += m;
+         }
    }
-   float* out = part + (int64_t) blockIdx.x * ( 5 * kH );
-   out[ k * kH + c ] = s;
-   if( k == 0 )
-      out[ 4 * kH + c ] = sb;
+   float* out = part + wave * ( 5 * kH );
+#pragma unroll
+   for( int k = 0; k < 5; k++ )
+#pragma unroll
+      for( int i = 0; i < 4; i++ ) {
+         float t = s[ k ][ i ];
+         t += __shfl_xor( t, 16, 64 );
+         t += __shfl_xor( t, 32, 64 );
+         if( sub == 0 )
+            out[ k * kH + c + i ] = t;
+      }
 }
 
 // ------------------------------------------------------------ parameters
@@ -587,8 +685,8 @@ struct Workspace
    Graph g;
    Acts a;
    DeviceArray< double > M, dM, Y, Rk, lpart, Z;
-   DeviceArray< float > dE, dEn, dH, dG, part, bpart, dpart, rwork;
-   DeviceArray< uint16_t > dS, dT, dP, dQ;
+   DeviceArray< float > dE, dH, dG, part;
+   DeviceArray< uint16_t > dS, dSn, dT, dTn, dP, dQ;
    DeviceArray< double > lout;
 };
 
@@ -691,7 +789,11 @@ void build_graph( Graph& g, const tnlmi_matrix& A, hipStream_t s )
 template< int NT, int EPI >
 void gemm( int64_t R, Term t0, Term t1, Term t2, const EpiArgs& e, hipStream_t s )
 {
-   hipLaunchKernelGGL( ( gemm64< NT, EPI > ), g1( R, 64 ), dim3( 256 ), 0, s, R, t0, t1, t2, e );
+   // (4 tiles per wave read the weights once per 64 rows; with fewer rows more waves matter more)
+   if( R >= 131072 )
+      hipLaunchKernelGGL( ( gemm64< NT, EPI, 4 > ), g1( R, 256 ), dim3( 256 ), 0, s, R, t0, t1, t2, e );
+   else
+      hipLaunchKernelGGL( ( gemm64< NT, EPI, 1 > ), g1( R, 64 ), dim3( 256 ), 0, s, R, t0, t1, t2, e );
 }
 
 // forward pass; keep = every layer's activations (training), else only the last
@@ -709,8 +811,8 @@ void forward( const tnlmi_spai& S, const Graph& g, const int32_t* off, const int
    }
    a.P.reserve( n * kH );
    a.Q.reserve( n * kH );
-   hipLaunchKernelGGL( encode_k, g1( E * kH ), dim3( 256 ), 0, s, E, g.xe.ptr, p + oAe, p + oae, a.E[ 0 ].ptr );
-   hipLaunchKernelGGL( encode_k, g1( n * kH ), dim3( 256 ), 0, s, n, g.xn.ptr, p + oAn, p + oan, a.H[ 0 ].ptr );
+   hipLaunchKernelGGL( encode_k, g1( E * 16 ), dim3( 256 ), 0, s, E, g.xe.ptr, p + oAe, p + oae, a.E[ 0 ].ptr );
+   hipLaunchKernelGGL( encode_k, g1( n * 16 ), dim3( 256 ), 0, s, n, g.xn.ptr, p + oAn, p + oan, a.H[ 0 ].ptr );
    const Term none{ nullptr, nullptr };
    for( int l = 0; l < kL; l++ ) {
       const int ci = keep ? l : ( l & 1 ), ni = keep ? l + 1 : ( ( l + 1 ) & 1 );
@@ -727,7 +829,9 @@ void forward( const tnlmi_spai& S, const Graph& g, const int32_t* off, const int
       ee.col = cols;
       ee.row = g.erow.ptr;
       gemm< 1, EPI_EDGE >( E, Term{ a.E[ ci ].ptr, WTn( S, l, mWe ) }, none, none, ee, s );
-      hipLaunchKernelGGL( mean_k, g1( n * kH ), dim3( 256 ), 0, s, n, off, a.E[ ni ].ptr, a.G[ ni ].ptr );
+      if( l == kL - 1 )
+         break;  // (the decoder reads the edges alone)
+      hipLaunchKernelGGL( mean_k, g1( n * 16 ), dim3( 256 ), 0, s, n, off, a.E[ ni ].ptr, a.G[ ni ].ptr );
       EpiArgs en{};
       en.yb = a.H[ ni ].ptr;
       en.bias = p + obh( l );
@@ -735,32 +839,23 @@ void forward( const tnlmi_spai& S, const Graph& g, const int32_t* off, const int
                            en, s );
    }
    const int last = keep ? kL : ( kL & 1 );
-   hipLaunchKernelGGL( decode_k, g1( E ), dim3( 256 ), 0, s, E, a.E[ last ].ptr, p + owo, p + obo, g.erow.ptr,
+   hipLaunchKernelGGL( decode_k, g1( E * 16 ), dim3( 256 ), 0, s, E, a.E[ last ].ptr, p + owo, p + obo, g.erow.ptr,
                        cols, g.isd.ptr, g.diag.ptr, M );
    TNLMI_HIP( hipGetLastError() );
 }
 
-// out[e] = sum of part[b * width + e] over the nblk blocks: chunks of
-// consecutive blocks (reduce_parts_chunks), then the chunk sums in order;
-// work holds kRedChunks * width floats
-void reduce_partials( const float* part, int64_t nblk, int width, float* out, float* work, hipStream_t s )
+// sums of nblk partials of `width` columns: the first `split` to out, the others to out2
+void reduce( const float* part, int64_t nblk, int width, int split, float* out, float* out2, hipStream_t s )
 {
-   const int64_t L = ceil_div( std::max< int64_t >( nblk, 1 ), kRedChunks );
-   const int64_t chunks = std::max< int64_t >( 1, ceil_div( nblk, L ) );
-   hipLaunchKernelGGL( reduce_parts_chunks, dim3( (unsigned) ceil_div( width, 64 ), (unsigned) chunks ), dim3( 64 ),
-                       0, s, part, nblk, width, L, work );
-   hipLaunchKernelGGL( reduce_parts, g1( width ), dim3( 256 ), 0, s, work, chunks, width, out );
+   hipLaunchKernelGGL( reduce_parts, dim3( (unsigned) ceil_div( width, 64 ) ), dim3( 1024 ), 0, s, part, nblk, width,
+                       split, out, out2 );
 }
 
-void wgrad( int64_t R, const uint16_t* X, const uint16_t* dY, float* gW, float* gb, DeviceArray< float >& part,
-            DeviceArray< float >& bpart, float* work, hipStream_t s )
+void wgrad( int64_t R, const uint16_t* X, const uint16_t* dY, float* gW, float* gb, float* part, hipStream_t s )
 {
-   const int64_t nb = ceil_div( R, kWRows );
-   hipLaunchKernelGGL( wgrad64, dim3( (unsigned) nb ), dim3( 256 ), 0, s, R, X, dY, part.ptr,
-                       gb ? bpart.ptr : (float*) nullptr );
-   reduce_partials( part.ptr, nb, kH * kH, gW, work, s );
-   if( gb )
-      reduce_partials( bpart.ptr, nb, kH, gb, work, s );
+   const int64_t nb = std::min< int64_t >( kWBlocks, ceil_div( R, kWRows ) );
+   hipLaunchKernelGGL( wgrad64, dim3( (unsigned) nb ), dim3( 256 ), 0, s, R, X, dY, part );
+   reduce( part, nb, kPart, kH * kH, gW, gb, s );
 }
 
 // probe loss on the device: returns L (host) and dL/dM per edge in dM
@@ -777,13 +872,10 @@ double probe_loss( const tnlmi_matrix& A, Workspace& w, const double* M, const d
    const int64_t nb = ceil_div( n, 256 );
    part.reserve( nb * K );
    out.reserve( 1 );
-   for( int k = 0; k < K; k++ ) {
-      hipLaunchKernelGGL( csr_mv, g1( n ), dim3( 256 ), 0, s, n, off, cols, (const double*) A.values, Z + k * n,
-                          Y.ptr + k * n );
-      hipLaunchKernelGGL( csr_mv, g1( n ), dim3( 256 ), 0, s, n, off, cols, M, Y.ptr + k * n, Rk.ptr + k * n );
-      hipLaunchKernelGGL( resid_k, dim3( (unsigned) nb ), dim3( 256 ), 0, s, n, Z + k * n, Rk.ptr + k * n,
-                          part.ptr + k * nb );
-   }
+   const dim3 probes( (unsigned) nb, (unsigned) K );
+   hipLaunchKernelGGL( csr_mv, probes, dim3( 256 ), 0, s, n, off, cols, (const double*) A.values, Z, Y.ptr );
+   hipLaunchKernelGGL( csr_mv, probes, dim3( 256 ), 0, s, n, off, cols, M, (const double*) Y.ptr, Rk.ptr );
+   hipLaunchKernelGGL( resid_k, probes, dim3( 256 ), 0, s, n, Z, Rk.ptr, part.ptr );
    hipLaunchKernelGGL( sum_k, dim3( 1 ), dim3( 256 ), 0, s, part.ptr, nb * K, 1.0 / ( (double) K * (double) n ),
                        out.ptr );
    if( dM )
@@ -813,63 +905,81 @@ double loss_grad( tnlmi_spai& S, Workspace& w, const tnlmi_matrix& A, const doub
    const double L = probe_loss( A, w, Mout, Z, K, w.dM.ptr, s );
    float* gr = S.grads.ptr;
    const float* p = S.params.ptr;
-   DeviceArray< double >& dM = w.dM;
-   DeviceArray< float >&dE = w.dE, &dEn = w.dEn, &dH = w.dH, &dG = w.dG, &part = w.part, &bpart = w.bpart,
-                       &dpart = w.dpart, &rwork = w.rwork;
-   DeviceArray< uint16_t >&dS = w.dS, &dT = w.dT, &dP = w.dP, &dQ = w.dQ;
+   DeviceArray< float >&dE = w.dE, &dH = w.dH, &dG = w.dG, &part = w.part;
+   DeviceArray< uint16_t >&dS = w.dS, &dSn = w.dSn, &dT = w.dT, &dTn = w.dTn, &dP = w.dP, &dQ = w.dQ;
    dE.reserve( E * kH );
-   dEn.reserve( E * kH );
    dH.reserve( n * kH );
    dG.reserve( n * kH );
-   dS.reserve( E * kH );
-   dT.reserve( n * kH );
-   dP.reserve( n * kH );
-   dQ.reserve( n * kH );
-   const int64_t nbE = ceil_div( std::max( E, n ), kWRows );
-   part.reserve( nbE * kH * kH );
-   bpart.reserve( nbE * kH );
-   dpart.reserve( ceil_div( std::max( E, n ), 256 ) * ( 5 * kH ) + 1 );
-   rwork.reserve( (int64_t) kRedChunks * kH * kH );  // chunk sums of reduce_partials (widest: kH * kH)
+   for( auto* v : { &dS, &dSn } )
+      v->reserve( E * kH );
+   for( auto* v : { &dT, &dTn, &dP, &dQ } )
+      v->reserve( n * kH );
+   constexpr int64_t kSumBlocks = 512;  // workgroups of dec_bwd_k and enc_bwd_k, four partials each
+   part.reserve( std::max< int64_t >( (int64_t) kWBlocks * kPart, kSumBlocks * 4 * 5 * kH ) );
    // decoder
-   const int64_t nb256 = ceil_div( E, 256 );
-   hipLaunchKernelGGL( dec_bwd_k, dim3( (unsigned) nb256 ), dim3( 256 ), 0, s, E, dM.ptr, g.erow.ptr, g.diag.ptr,
-                       a.E[ kL ].ptr, p + owo, dE.ptr, dpart.ptr );
-   reduce_partials( dpart.ptr, nb256, kH + 1, gr + owo, rwork.ptr, s );
-   TNLMI_HIP( hipMemsetAsync( dH.ptr, 0, sizeof( float ) * n * kH, s ) );
+   hipLaunchKernelGGL( dec_bwd_k, dim3( (unsigned) kSumBlocks ), dim3( 256 ), 0, s, E, w.dM.ptr, g.erow.ptr, g.diag.ptr,
+                       a.E[ kL ].ptr, p + owo, dS.ptr, part.ptr );
+   reduce( part.ptr, kSumBlocks * 4, kH + 1, kH + 1, gr + owo, nullptr, s );
+   // the last layer's node update reaches nothing: no gradient
+   static_assert( mWg == mWh + 1, "Wh and Wg side by side" );
+   TNLMI_HIP( hipMemsetAsync( gr + oW( kL - 1, mWh ), 0, sizeof( float ) * 2 * kH * kH, s ) );
+   TNLMI_HIP( hipMemsetAsync( gr + obh( kL - 1 ), 0, sizeof( float ) * kH, s ) );
    const Term none{ nullptr, nullptr };
    for( int l = kL - 1; l >= 0; l-- ) {
-      // node update: dT = dH * [H > 0]
-      hipLaunchKernelGGL( mask_k, g1( n * kH ), dim3( 256 ), 0, s, n * kH, dH.ptr, a.H[ l + 1 ].ptr, dT.ptr );
-      wgrad( n, a.H[ l ].ptr, dT.ptr, gr + oW( l, mWh ), gr + obh( l ), part, bpart, rwork.ptr, s );
-      wgrad( n, a.G[ l + 1 ].ptr, dT.ptr, gr + oW( l, mWg ), nullptr, part, bpart, rwork.ptr, s );
+      const bool top = l == kL - 1;  // dT = 0 there
+      // the edge update's weights; its node terms' gradients
+      wgrad( E, a.E[ l ].ptr, dS.ptr, gr + oW( l, mWe ), gr + obe( l ), part.ptr, s );
+      hipLaunchKernelGGL( scatter_k, g1( n * 16 ), dim3( 256 ), 0, s, n, off, g.cptr.ptr, g.cperm.ptr, dS.ptr, dP.ptr,
+                          dQ.ptr );
+      wgrad( n, a.H[ l ].ptr, dP.ptr, gr + oW( l, mWu ), nullptr, part.ptr, s );
+      wgrad( n, a.H[ l ].ptr, dQ.ptr, gr + oW( l, mWv ), nullptr, part.ptr, s );
+      const Term tP{ dP.ptr, Wn( S, l, mWu ) }, tQ{ dQ.ptr, Wn( S, l, mWv ) }, tT{ dT.ptr, Wn( S, l, mWh ) },
+         tS{ dS.ptr, Wn( S, l, mWe ) };
+      if( l == 0 ) {
+         // the encoders' gradients want dH and dE in FP32
+         EpiArgs eh{};
+         eh.yf = dH.ptr;
+         if( top )
+            gemm< 2, EPI_STORE >( n, tP, tQ, none, eh, s );
+         else
+            gemm< 3, EPI_STORE >( n, tT, tP, tQ, eh, s );
+         EpiArgs ee{};
+         ee.yf = dE.ptr;
+         gemm< 1, EPI_STORE >( E, tS, none, none, ee, s );
+         break;
+      }
+      // the node update below: dT = BF16( dH * [H > 0] ), its weights, and what it
+      // passes to its row's edges, dG / deg
+      EpiArgs eh{};
+      eh.yb = dTn.ptr;
+      eh.mask = a.H[ l ].ptr;
+      if( top )
+         gemm< 2, EPI_DNODE >( n, tP, tQ, none, eh, s );
+      else
+         gemm< 3, EPI_DNODE >( n, tT, tP, tQ, eh, s );
+      std::swap( dT, dTn );
+      wgrad( n, a.H[ l - 1 ].ptr, dT.ptr, gr + oW( l - 1, mWh ), gr + obh( l - 1 ), part.ptr, s );
+      wgrad( n, a.G[ l ].ptr, dT.ptr, gr + oW( l - 1, mWg ), nullptr, part.ptr, s );
       EpiArgs eg{};
       eg.yf = dG.ptr;
-      gemm< 1, EPI_STORE >( n, Term{ dT.ptr, Wn( S, l, mWg ) }, none, none, eg, s );
-      // edge update: dS = (dE + dG[row] / deg) * [E > 0]
-      hipLaunchKernelGGL( edge_bwd_k, g1( E * kH ), dim3( 256 ), 0, s, E, dE.ptr, dG.ptr, g.erow.ptr, g.deg.ptr,
-                          a.E[ l + 1 ].ptr, dS.ptr );
-      wgrad( E, a.E[ l ].ptr, dS.ptr, gr + oW( l, mWe ), gr + obe( l ), part, bpart, rwork.ptr, s );
+      eg.deg = g.deg.ptr;
+      gemm< 1, EPI_DMEAN >( n, Term{ dT.ptr, Wn( S, l - 1, mWg ) }, none, none, eg, s );
+      // the edge update below: dS = BF16( (dE + dG[row] / deg) * [E > 0] )
       EpiArgs ed{};
-      ed.yf = dEn.ptr;
-      gemm< 1, EPI_STORE >( E, Term{ dS.ptr, Wn( S, l, mWe ) }, none, none, ed, s );
-      hipLaunchKernelGGL( scatter_k, g1( n * kH ), dim3( 256 ), 0, s, n, off, g.cptr.ptr, g.cperm.ptr, dS.ptr, dP.ptr,
-                          dQ.ptr );
-      wgrad( n, a.H[ l ].ptr, dP.ptr, gr + oW( l, mWu ), nullptr, part, bpart, rwork.ptr, s );
-      wgrad( n, a.H[ l ].ptr, dQ.ptr, gr + oW( l, mWv ), nullptr, part, bpart, rwork.ptr, s );
-      EpiArgs eh{};
-      eh.yf = dH.ptr;
-      gemm< 3, EPI_STORE >( n, Term{ dT.ptr, Wn( S, l, mWh ) }, Term{ dP.ptr, Wn( S, l, mWu ) },
-                            Term{ dQ.ptr, Wn( S, l, mWv ) }, eh, s );
-      std::swap( dE.ptr, dEn.ptr );
+      ed.yb = dSn.ptr;
+      ed.P = dG.ptr;
+      ed.row = g.erow.ptr;
+      ed.mask = a.E[ l ].ptr;
+      gemm< 1, EPI_DEDGE >( E, tS, none, none, ed, s );
+      std::swap( dS, dSn );
    }
    // encoder
-   hipLaunchKernelGGL( enc_bwd_k, dim3( (unsigned) nb256 ), dim3( 256 ), 0, s, E, g.xe.ptr, dE.ptr, a.E[ 0 ].ptr,
-                       dpart.ptr );
-   reduce_partials( dpart.ptr, nb256, 5 * kH, gr + oAe, rwork.ptr, s );
-   const int64_t nbn = ceil_div( n, 256 );
-   hipLaunchKernelGGL( enc_bwd_k, dim3( (unsigned) nbn ), dim3( 256 ), 0, s, n, g.xn.ptr, dH.ptr, a.H[ 0 ].ptr,
-                       dpart.ptr );
-   reduce_partials( dpart.ptr, nbn, 5 * kH, gr + oAn, rwork.ptr, s );
+   hipLaunchKernelGGL( enc_bwd_k, dim3( (unsigned) kSumBlocks ), dim3( 256 ), 0, s, E, g.xe.ptr, dE.ptr, a.E[ 0 ].ptr,
+                       part.ptr );
+   reduce( part.ptr, kSumBlocks * 4, 5 * kH, 5 * kH, gr + oAe, nullptr, s );
+   hipLaunchKernelGGL( enc_bwd_k, dim3( (unsigned) kSumBlocks ), dim3( 256 ), 0, s, n, g.xn.ptr, dH.ptr, a.H[ 0 ].ptr,
+                       part.ptr );
+   reduce( part.ptr, kSumBlocks * 4, 5 * kH, 5 * kH, gr + oAn, nullptr, s );
    TNLMI_HIP( hipGetLastError() );
    TNLMI_HIP( hipStreamSynchronize( s ) );
    return L;
