@@ -588,6 +588,10 @@ tnlmi_status tnlmi_bf16_gemm64( int64_t rows, const uint16_t* d_X, const uint16_
  * iterations (mixed: inner iterations) and final residues.  use_graph: the
  * launch (counter reset + solve) is captured in a hipGraph once per argument
  * set and replayed.  Asynchronous.  Calls with one object must not overlap.
+ * block_size and lanes_per_row are those of the general kernels; an FP64 solve
+ * of systems of at most 16,384 rows with at most 8 slots per row runs in a
+ * kernel of its own from LDS and registers, on a copy of the slots (10 bytes
+ * each) that every solve lays out anew.
  * No reference counterpart (TNL solves one system per solver call). */
 typedef struct tnlmi_batched_cg tnlmi_batched_cg;
 tnlmi_status tnlmi_batched_cg_create( const tnlmi_matrix* A, const tnlmi_matrix* A_lo, const int64_t* sys_rows,

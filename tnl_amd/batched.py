@@ -34,7 +34,9 @@ def diffusion_batch(nsys, smin=16, smax=128, seed=0):
 class BatchedCG:
     """One persistent launch solving every diagonal block of A (FP64 values).
     lanes_per_row (1, 2, 4, 8): the lanes that sum one row, so a wavefront
-    covers 64 / lanes_per_row rows."""
+    covers 64 / lanes_per_row rows.  Both shapes are those of the general
+    kernel; systems of at most 16,384 rows with at most 8 slots per row are
+    solved from LDS and registers by workgroups of the library's choice."""
 
     def __init__(self, A, sys_rows, A_lo=None, block_size=512, lanes_per_row=1, stream=None):
         self.sys_rows = np.ascontiguousarray(sys_rows, np.int64)

@@ -21,6 +21,7 @@
 #include <cstring>
 #include <map>
 #include <tuple>
+#include <vector>
 
 #include "segments.hpp"
 
@@ -198,6 +199,165 @@ __device__ __forceinline__ void put_result( int64_t* iters, double* res, int64_t
    }
 }
 
+// ---- a system in its workgroup's registers and LDS: p in LDS, r and A p in
+// registers (ROWS rows per thread), the matrix read through slots that every
+// solve lays out first -- column-major, so that a wave's reads are contiguous,
+// with the column as a 16-bit distance from the row.  CSR rows read in place cost a
+// wave about 20 cache lines per load, and vectors in memory an L2 round trip per
+// step.  Bound by the slots' L2 reads (10 bytes per entry) for the large systems
+// and by the workgroup's two sums (about 2 us) for the small ones.
+// 1,024 diffusion systems of 256 to 16,384 rows, 1e-10: 22.4 against 77 ms (one of
+// 16,384 rows alone 23 us an iteration for its 1.2 MB); 500 of 144 to 9,216 rows
+// 8.8 against 67 ms; 1,024 of 64 to 2,304 rows 2.2 against 6.2 ms.  1,024 threads
+// and 16 rows each for the largest: 512 threads and 32 rows took 25.9 ms.  Systems
+// go out largest first, so that no long one is left for the end.
+constexpr int64_t kLocalMost = 16384;  // rows of a system at most (128 KiB of LDS)
+constexpr int kLocalWidth = 8;         // slots per row at most
+constexpr int16_t kNoEntry = INT16_MIN;
+
+__global__ void widest_row( SegView v, int32_t* __restrict__ out )
+{
+   const int64_t r = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+   if( r < v.n )
+      atomicMax( out, segment_size( v, r ) );
+}
+
+// slot k of row r at [ k * n + r ]
+__global__ void __launch_bounds__( 256 ) lay_out( SegView v, int32_t w, const int32_t* __restrict__ cols,
+                                                  const double* __restrict__ vals, int16_t* __restrict__ dist,
+                                                  double* __restrict__ val )
+{
+   const int64_t r = (int64_t) blockIdx.x * 256 + threadIdx.x;
+   if( r >= v.n )
+      return;
+   const int32_t size = segment_size( v, r );
+   for( int32_t k = 0; k < w; k++ ) {
+      int64_t g = k < size ? ( v.format == TNLMI_CSR ? (int64_t) v.offsets[ r ] + k : global_index( v, r, k ) ) : -1;
+      const int32_t c = g >= 0 ? cols[ g ] : -1;
+      dist[ k * v.n + r ] = c >= 0 ? (int16_t) ( c - (int32_t) r ) : kNoEntry;
+      val[ k * v.n + r ] = c >= 0 ? vals[ g ] : 0.0;
+   }
+}
+
+struct LocalArgs
+{
+   const int32_t* order;  // systems, largest first
+   const int16_t* dist;
+   const double* val;
+   int64_t n;             // rows of all systems
+};
+
+// FP64 Jacobi-CG per system of at most B * ROWS rows and W slots per row,
+// as batched_cg64
+template< int B, int ROWS, int W >
+__global__ void __launch_bounds__( B, ROWS == 4 ? 8 : 4 ) batched_cg_local( BatchArgs a, LocalArgs L )
+{
+   __shared__ double p[ B * ROWS ];
+   __shared__ double red[ B / 64 ];
+   __shared__ int slot;
+   for( int64_t q = next_system( a.counter, &slot ); q < a.nsys; q = next_system( a.counter, &slot ) ) {
+      const int64_t sys = L.order[ q ];
+      const int64_t r0 = a.sys_rows[ sys ];
+      const int32_t n = (int32_t) ( a.sys_rows[ sys + 1 ] - r0 );
+      double r[ ROWS ], y[ ROWS ];
+      // y = A p, kRows rows' slots requested together
+      constexpr int kRows = ROWS == 8 ? 2 : 1;
+      auto product = [ & ]() {
+         int t = threadIdx.x;
+         asm volatile( "" : "+v"( t ) );  // (the rows' offsets are not worth registers across iterations)
+#pragma unroll
+         for( int j = 0; j < ROWS; j += kRows )
+            if( j * B < n ) {
+               int32_t c[ kRows ][ W ];
+               double v[ kRows ][ W ];
+#pragma unroll
+               for( int u = 0; u < kRows; u++ ) {
+                  const int32_t i = min( t + ( j + u ) * B, n - 1 );  // (rows past the system: its last one again)
+#pragma unroll
+                  for( int k = 0; k < W; k++ ) {  // (a uniform base and a 32-bit offset)
+                     c[ u ][ k ] = ( L.dist + k * L.n + r0 )[ (uint32_t) i ];
+                     v[ u ][ k ] = ( L.val + k * L.n + r0 )[ (uint32_t) i ];
+                  }
+               }
+#pragma unroll
+               for( int u = 0; u < kRows; u++ ) {
+                  const int32_t i = min( t + ( j + u ) * B, n - 1 );
+                  double s = 0;
+#pragma unroll
+                  for( int k = 0; k < W; k++ ) {
+                     const double f = s + v[ u ][ k ] * p[ c[ u ][ k ] != kNoEntry ? i + c[ u ][ k ] : i ];
+                     s = c[ u ][ k ] != kNoEntry ? f : s;
+                  }
+                  y[ j + u ] = s;
+               }
+               asm volatile( "" ::: "memory" );  // (no more rows at a time: they would not fit the registers)
+            }
+      };
+      auto rows = [ & ]( auto&& f ) {
+         int t = threadIdx.x;
+         asm volatile( "" : "+v"( t ) );
+#pragma unroll
+         for( int j = 0; j < ROWS; j++ )
+            if( j * B < n ) {
+               if( t + j * B < n )
+                  f( j, t + j * B );
+               if( j % 4 == 3 )
+                  asm volatile( "" ::: "memory" );
+            }
+      };
+      // r = b - A x, p = z = D^{-1} r, s1 = (r, z), normb = ||D^{-1} b||
+      rows( [ & ]( int, int32_t i ) { p[ i ] = a.x[ r0 + i ]; } );
+      __syncthreads();
+      product();
+      double acc1 = 0, acc2 = 0;
+      rows( [ & ]( int j, int32_t i ) {
+         const double bi = ( a.b + r0 )[ (uint32_t) i ], di = ( a.dinv + r0 )[ (uint32_t) i ];
+         r[ j ] = bi - y[ j ];
+         y[ j ] = r[ j ] * di;
+         acc1 += r[ j ] * y[ j ];
+         const double mb = bi * di;
+         acc2 += mb * mb;
+      } );
+      double s1 = block_sum< B >( acc1, red );
+      const double normb = sqrt( block_sum< B >( acc2, red ) );
+      rows( [ & ]( int j, int32_t i ) { p[ i ] = y[ j ]; } );
+      __syncthreads();
+      int64_t it = 0;
+      double res = 0;
+      if( normb == 0.0 )
+         rows( [ & ]( int, int32_t i ) { a.x[ r0 + i ] = 0.0; } );
+      else {
+         res = sqrt( s1 ) / normb;
+         while( ! ( isnan( res ) || it > a.maxit || res < a.tol ) ) {
+            it++;
+            product();
+            double acc = 0;
+            rows( [ & ]( int j, int32_t i ) { acc += y[ j ] * p[ i ]; } );
+            const double s2 = block_sum< B >( acc, red );
+            if( s2 == 0.0 ) {
+               res = 0.0;
+               break;
+            }
+            const double alpha = s1 / s2;
+            acc = 0;
+            rows( [ & ]( int j, int32_t i ) {
+               ( a.x + r0 )[ (uint32_t) i ] += alpha * p[ i ];
+               r[ j ] = r[ j ] - alpha * y[ j ];
+               y[ j ] = r[ j ] * ( a.dinv + r0 )[ (uint32_t) i ];
+               acc += r[ j ] * y[ j ];
+            } );
+            const double s1n = block_sum< B >( acc, red );
+            const double beta = s1 == 0.0 ? 0.0 : s1n / s1;
+            s1 = s1n;
+            rows( [ & ]( int j, int32_t i ) { p[ i ] = y[ j ] + beta * p[ i ]; } );
+            __syncthreads();
+            res = sqrt( s1 ) / normb;
+         }
+      }
+      put_result( a.iters, a.res, sys, it, res );
+   }
+}
+
 // FP64 Jacobi-CG per system, TNL's stopping rule with default min/divergence
 template< int B, int T >
 __global__ void __launch_bounds__( B ) batched_cg64( BatchArgs a )
@@ -361,6 +521,12 @@ struct tnlmi_batched_cg
    int32_t block = 512;
    int32_t lanes = 1;  // lanes per row in the row sums (64 / lanes rows per wavefront)
    int64_t grid = 1;  // persistent workgroups: a few per CU, at most one per system
+   // the local solve (0 threads: some system or row is too large for it)
+   int32_t local_threads = 0, local_rows = 0, width = 0;
+   int64_t local_grid = 1;
+   DeviceArray< int32_t > order;
+   DeviceArray< int16_t > dist;
+   DeviceArray< double > val;
    DeviceArray< int64_t > sys_rows;
    DeviceArray< double > dinv, r, p, Ap;
    DeviceArray< float > r32, p32, Ap32, d32;
@@ -385,6 +551,24 @@ namespace {
 void launch( tnlmi_batched_cg& P, const BatchArgs& a, bool mixed, hipStream_t s )
 {
    hipLaunchKernelGGL( reset_counter, dim3( 1 ), dim3( 1 ), 0, s, a.counter );
+   if( P.local_threads && ! mixed ) {
+      hipLaunchKernelGGL( lay_out, dim3( (unsigned) ceil_div( P.rows, 256 ) ), dim3( 256 ), 0, s, a.v, P.width, a.cols,
+                          a.vals, P.dist.ptr, P.val.ptr );
+      const LocalArgs L{ P.order.ptr, P.dist.ptr, P.val.ptr, P.rows };
+      const dim3 grid( (unsigned) P.local_grid );
+#define TNLMI_LOCAL( BS, ROWS, W )                                                                                    \
+   if( P.local_threads == BS && P.local_rows == ROWS && P.width <= W ) {                                              \
+      hipLaunchKernelGGL( ( batched_cg_local< BS, ROWS, W > ), grid, dim3( BS ), 0, s, a, L );                        \
+      return;                                                                                                         \
+   }
+#define TNLMI_LOCAL_W( BS, ROWS ) TNLMI_LOCAL( BS, ROWS, 5 ) TNLMI_LOCAL( BS, ROWS, kLocalWidth )
+      TNLMI_LOCAL_W( 512, 4 )
+      TNLMI_LOCAL_W( 1024, 4 )
+      TNLMI_LOCAL_W( 1024, 8 )
+      TNLMI_LOCAL_W( 1024, 16 )
+#undef TNLMI_LOCAL_W
+#undef TNLMI_LOCAL
+   }
    const dim3 grid( (unsigned) P.grid );
 #define TNLMI_BATCH( BS, T )                                                                                          \
    if( P.block == BS && P.lanes == T ) {                                                                              \
@@ -472,6 +656,49 @@ tnlmi_status tnlmi_batched_cg_create( const tnlmi_matrix* A, const tnlmi_matrix*
          }
          hipLaunchKernelGGL( batch_inv_diag< double >, dim3( (unsigned) ceil_div( n, 256 ) ), dim3( 256 ), 0, s,
                              make_view( *A->segments ), A->column_indexes, (const double*) A->values, P->dinv.ptr );
+         // the local solve, its workgroups by the largest system (2,048 rows: 512
+         // threads, four per CU; 4,096: two of 1,024; else one): block size and lanes per
+         // row shape the general kernel only
+         int64_t largest = 0;
+         for( int64_t k = 0; k < nsys; k++ )
+            largest = std::max( largest, sys_rows[ k + 1 ] - sys_rows[ k ] );
+         if( n && largest <= kLocalMost ) {
+            DeviceArray< int32_t > w;
+            w.allocate( 1 );
+            int32_t h = 0;
+            TNLMI_HIP( hipMemsetAsync( w.ptr, 0, sizeof( int32_t ), s ) );
+            hipLaunchKernelGGL( widest_row, dim3( (unsigned) ceil_div( n, 256 ) ), dim3( 256 ), 0, s,
+                                make_view( *A->segments ), w.ptr );
+            TNLMI_HIP( hipMemcpyAsync( &h, w.ptr, sizeof( h ), hipMemcpyDeviceToHost, s ) );
+            TNLMI_HIP( hipStreamSynchronize( s ) );
+            if( h >= 1 && h <= kLocalWidth ) {
+               std::vector< int32_t > order( nsys );
+               for( int64_t k = 0; k < nsys; k++ )
+                  order[ k ] = (int32_t) k;
+               std::stable_sort( order.begin(), order.end(), [ & ]( int32_t x, int32_t y ) {
+                  return sys_rows[ x + 1 ] - sys_rows[ x ] > sys_rows[ y + 1 ] - sys_rows[ y ];
+               } );
+               P->order.allocate( nsys );
+               TNLMI_HIP( hipMemcpyAsync( P->order.ptr, order.data(), 4 * nsys, hipMemcpyHostToDevice, s ) );
+               // (all kernel widths read kLocalWidth or 5 slots per row)
+               P->width = h <= 5 ? 5 : kLocalWidth;
+               try {
+                  P->dist.allocate( P->width * n );
+                  P->val.allocate( P->width * n );
+                  P->local_threads = largest <= 2048 ? 512 : 1024;
+               }
+               catch( const Error& ) {  // no room for the slots: the general kernel
+                  (void) hipGetLastError();
+                  P->dist.reset();
+                  P->val.reset();
+               }
+               P->local_rows = largest <= 4096 ? 4 : largest <= 8192 ? 8 : 16;
+               // (2,048 threads per CU, with up to 64 registers each)
+               const int64_t per_cu = P->local_threads <= 512 ? 4 : P->local_rows == 4 ? 2 : 1;
+               P->local_grid = std::min< int64_t >( cus * per_cu, nsys );
+               TNLMI_HIP( hipStreamSynchronize( s ) );  // (order)
+            }
+         }
          TNLMI_HIP( hipGetLastError() );
          TNLMI_HIP( hipStreamSynchronize( s ) );
       }
