@@ -108,7 +108,7 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
       for( int j = 0; j < N; j++ )
          v[ j ] = 0;
    wave_totals();
-   late = __syncthreads_or( late );
+   late = wave_uniform( __syncthreads_or( late ) );
 #pragma unroll
    for( int j = 0; j < N; j++ )
       v[ j ] = wave_uniform( block_total( j ) );
@@ -182,7 +182,7 @@ __device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict_
          }
       }
    }
-   late = __syncthreads_or( late );
+   late = wave_uniform( __syncthreads_or( late ) );
    if( (int) threadIdx.x < count ) {
       double r = 0;
       for( int q = 0; q < quarters; q++ )

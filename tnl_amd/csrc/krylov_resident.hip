@@ -386,7 +386,10 @@ __global__ void __launch_bounds__( THREADS ) gmres_resident( GmresArgs a )
       w[ j ] = R.load( a.r, j );
    bool late = false;
    auto barrier = [ & ] { late = late || ! grid_barrier< THREADS >( a.slots, number++, sm ); };
-   auto sum = [ & ]( double ( &v )[ 1 ] ) { late = late || ! grid_sum< THREADS >( v, a.slots, number++, sm ); };
+   auto sum = [ & ]( double ( &v )[ 1 ] ) {
+      late = late || ! grid_sum< THREADS >( v, a.slots, number++, sm );
+      v[ 0 ] = wave_uniform( v[ 0 ] );  // (also where no sum was taken: what follows from it branches)
+   };
    // sums of `count` values, value k's per-thread part in acc[ k - k0 ] for the group at k0
    auto put = [ & ]( double ( &acc )[ kGroup ], int k0, int count ) {
       const double t = wave_sum_group( acc );  // lane l: value l >> 3
@@ -549,7 +552,7 @@ __global__ void __launch_bounds__( THREADS ) gmres_resident( GmresArgs a )
          if( threadIdx.x == 0 )
             givens( g, i, norm, a.normb );
          __syncthreads();
-         st.res = g.res;
+         st.res = wave_uniform( g.res );
          done++;
          if( ! goes_on( a, st.res, st.it ) ) {
             o = i;
@@ -563,7 +566,7 @@ __global__ void __launch_bounds__( THREADS ) gmres_resident( GmresArgs a )
       if( threadIdx.x < 64 )
          back_substitute( g, k );
       __syncthreads();
-      if( g.zero_pivot ) {
+      if( wave_uniform( g.zero_pivot ) ) {
          end = kResidentZeroPivot;
          break;
       }
