@@ -100,3 +100,16 @@ def test_nan_and_iteration_limit():
     x.zero_()
     its, res = bc.solve(b, x, 1e-10, max_iterations=3, use_graph=False)
     assert int(its[0]) == 4 and int(its[2]) == 4  # (the reference counts the refused iteration)
+
+
+def test_autotune_times_what_it_shapes(monkeypatch):
+    """Where the shapes leave the FP64 solve alone the mixed one is timed."""
+    rng = np.random.default_rng(4)
+    mixed = []
+    solve = B.BatchedCG.solve
+    monkeypatch.setattr(B.BatchedCG, "solve", lambda self, *a, **kw: (mixed.append(kw["mixed"]), solve(self, *a, **kw))[1])
+    for half, sizes, want in ((2, [900, 40], True), (4, [900, 40], False), (1, [16385], False)):
+        off, cols, vals, sys_rows = _batch(sizes, half, rng)
+        mixed.clear()
+        B.autotune(off, cols, vals, sys_rows, candidates=[(tnl.CSR, 0)], blocks=[256], lanes=[1, 4], cache=False)
+        assert set(mixed) == {want}

@@ -90,8 +90,9 @@ def _device_name():
 def autotune(off, cols, vals, sys_rows, sample=256, candidates=CANDIDATES, blocks=BLOCKS, lanes=LANES,
              tolerance=1e-10, cache=True, log=None):
     """Times every (format, slice size, workgroup size, rows per wavefront)
-    candidate on the first `sample` systems and returns the fastest as a dict;
-    results are cached in a JSON file keyed by the batch's shape, the device,
+    candidate on the first `sample` systems and returns the fastest as a dict.
+    The FP64 solve is timed, or the mixed one where the FP64 solve of these
+    systems runs in its own kernel, which no candidate shapes; results are cached in a JSON file keyed by the batch's shape, the device,
     the candidate lists and the tolerance."""
     import torch
     nsys = len(sys_rows) - 1
@@ -111,26 +112,29 @@ def autotune(off, cols, vals, sys_rows, sample=256, candidates=CANDIDATES, block
     c, v = cols[: int(o[-1])], vals[: int(o[-1])]
     b = torch.ones(rows, dtype=torch.float64, device="cuda")
     x = torch.zeros(rows, dtype=torch.float64, device="cuda")
+    # (the limits of the kernel from LDS and registers, see BatchedCG)
+    mixed = k > 0 and int(np.diff(sys_rows[: k + 1]).max()) <= 16384 and int((o[1:] - o[:-1]).max()) <= 8
     trials = []
     for fmt, param in candidates:
         A = SparseMatrix.from_csr(rows, rows, o, c, v, fmt=fmt, param=param)
+        A_lo = SparseMatrix(A.rows, A.columns, A.segments, A.values.float(), A.column_indexes) if mixed else None
         for bs in blocks:
             for lpr in lanes:
-                bc = BatchedCG(A, sys_rows[: k + 1], block_size=bs, lanes_per_row=lpr)
+                bc = BatchedCG(A, sys_rows[: k + 1], A_lo, block_size=bs, lanes_per_row=lpr)
                 x.zero_()
-                bc.solve(b, x, tolerance, use_graph=False)
+                bc.solve(b, x, tolerance, mixed=mixed, use_graph=False)
                 torch.cuda.synchronize()
                 t0 = time.perf_counter()
                 for _ in range(2):
                     x.zero_()
-                    bc.solve(b, x, tolerance, use_graph=False)
+                    bc.solve(b, x, tolerance, mixed=mixed, use_graph=False)
                 torch.cuda.synchronize()
                 t = (time.perf_counter() - t0) / 2
                 trials.append(dict(format=FORMAT_NAMES[fmt], format_id=fmt, param=param, block=bs, lanes_per_row=lpr,
                                    rows_per_wavefront=64 // lpr, seconds=t))
                 if log:
                     log(f"autotune {FORMAT_NAMES[fmt]}{param or ''} block {bs} lanes/row {lpr}: {t * 1e3:.2f} ms")
-        del A
+        del A, A_lo
     best = min(trials, key=lambda d: d["seconds"])
     result = dict(best, trials=trials)
     if cache:
