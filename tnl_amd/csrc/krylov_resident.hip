@@ -10,9 +10,9 @@
 // goes through memory once.
 //
 // Convection-diffusion, per iteration against launch by launch: GMRES(10) with
-// modified Gram-Schmidt twice on 200^2 43 against 199 us, GMRES(20) on 1024^2 154
+// modified Gram-Schmidt twice on 200^2 40 against 199 us, GMRES(20) on 1024^2 154
 // against 339 us; GMRES(30) with classical Gram-Schmidt twice on 120^2 27 against
-// 84 us, on 1024^2 113 against 173 us (the basis read three times, 390 MB on
+// 84 us, on 1024^2 111 against 173 us (the basis read three times, 390 MB on
 // average, is most of it); BiCGStab on 100^2 15 against 98 us, 500^2 30 against
 // 98 us, 1024^2 74 against 125 us.  Small systems: 2 grid sums per basis vector of
 // modified Gram-Schmidt, 5 per BiCGStab iteration, 2.2 us each.
