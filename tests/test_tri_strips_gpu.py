@@ -40,13 +40,44 @@ def _scattered(n, rng):
     return off, cols, np.where(cols == row, 9.0, rng.standard_normal(len(cols)))
 
 
+def _far(width, lines, rng):
+    """Three entries on each side of the diagonal, all about `width` rows away:
+    with lines of more rows than a strip keeps in LDS, every one is an import."""
+    n = width * lines
+    i = np.arange(n)
+    shifts = [-width - 1, -width, -width + 1, 0, width - 1, width, width + 1]
+    cols = np.stack([i + s for s in shifts], 1)
+    keep = (cols >= 0) & (cols < n)
+    vals = np.where(cols == i[:, None], 9.0, rng.standard_normal((n, 7)))
+    off = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    return off, cols[keep].astype(np.int32), vals[keep]
+
+
+def _scattered_band(n, low, high, rng):
+    """Up to three entries on each side of the diagonal, low to high rows away."""
+    i = np.arange(n)
+    d = np.sort(rng.integers(low, high, (n, 6)), 1)
+    cols = np.sort(np.concatenate([i[:, None] - d[:, :3], i[:, None], i[:, None] + d[:, 3:]], 1), 1)
+    keep = (cols >= 0) & (cols < n)
+    keep[:, 1:] &= cols[:, 1:] != cols[:, :-1]
+    vals = np.where(cols == i[:, None], 9.0, rng.standard_normal((n, 7)))
+    off = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    return off, cols[keep].astype(np.int32), vals[keep]
+
+
 CASES = {
     "rows127": lambda g: _grid(127, 1, 1, g), "rows128": lambda g: _grid(128, 1, 1, g),
     "line64": lambda g: _grid(64, 64, 1, g), "line65": lambda g: _grid(65, 130, 1, g),
     "thin": lambda g: _grid(700, 9, 1, g), "tall": lambda g: _grid(9, 700, 1, g),
     "plane": lambda g: _grid(17, 19, 23, g), "cube": lambda g: _grid(40, 40, 40, g),
     "scattered": lambda g: _scattered(2500, g), "scattered_strips": lambda g: _scattered(12000, g),
+    "far_one_strip": lambda g: _far(5000, 3, g), "far_strips": lambda g: _far(6000, 20, g),
+    "band_strips": lambda g: _scattered_band(60000, 200, 300, g),
 }
+# the strips of either factor (test_tri_strips_plan.py checks the plans): none, one or more than one
+STRIPS = {name: (1, 1) if name in ("line64", "thin", "scattered", "scattered_strips", "far_one_strip")
+          else (0, 0) if name == "rows127" else (2, 256) for name in CASES}
+FULL_RING = ("far_one_strip", "far_strips")  # more imports in two groups of steps than two per row
 
 
 @pytest.mark.parametrize("name", CASES)

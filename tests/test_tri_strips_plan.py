@@ -1,0 +1,80 @@
+"""The host's plans of the strip solves (ILU(0) factors): every factor that
+tests/test_tri_strips_gpu.py solves is planned as it is meant to be, and the
+imports that the solving wave can wait for fit the LDS ring that holds them."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import test_tri_strips_gpu as gpu_cases
+from test_barrier_loops import CSRC, HIPCC, ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIB = os.path.join(ROOT, "tnl_amd", "libtnlmi.so")
+
+
+@pytest.fixture(scope="module")
+def planner(tmp_path_factory):
+    if not os.path.exists(HIPCC) or not os.path.exists(LIB):
+        pytest.skip("hipcc or the library is missing")
+    so = str(tmp_path_factory.mktemp("plan") / "strips_plan.so")
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-x", "hip", "-O1", "-std=c++17", "-fPIC", "-shared",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, os.path.join(HERE, "strips_plan.cpp"), "-o", so,
+                    "-L" + os.path.dirname(LIB), "-ltnlmi", "-Wl,-rpath," + os.path.dirname(LIB)],
+                   check=True, capture_output=True)
+    lib = ctypes.CDLL(so)
+    lib.strips_plan.argtypes = [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_double,
+                                ctypes.c_void_p]
+    return lib
+
+
+def _factor(off, cols, upper):
+    """(ptr, col) of a factor's pattern in solve order, the upper rows reversed with the pivot first."""
+    n = len(off) - 1
+    row = np.repeat(np.arange(n), np.diff(off))
+    keep = cols >= row if upper else cols < row
+    r, c = row[keep], cols[keep]
+    order = np.lexsort((c, n - 1 - r if upper else r))
+    count = np.bincount(n - 1 - r if upper else r, minlength=n)
+    return np.concatenate([[0], np.cumsum(count)]).astype(np.int32), c[order].astype(np.int32)
+
+
+def _levels_us(ptr, col, upper):
+    """What the solves by levels are expected to take, as ilu0_build counts it."""
+    n = len(ptr) - 1
+    level = np.zeros(n, np.int64)
+    for t in range(n):
+        for g in range(ptr[t] + (1 if upper else 0), ptr[t + 1]):
+            level[t] = max(level[t], level[n - 1 - col[g] if upper else col[g]] + 1)
+    us, narrow = 0.0, False
+    for width in np.bincount(level):
+        if width > 2048:
+            us += 6.0
+        else:
+            us += 0.65 if narrow else 10.65
+        narrow = width <= 2048
+    return us
+
+
+def _plan(planner, off, cols, upper):
+    ptr, col = _factor(off, cols, upper)
+    strips = ctypes.c_int32()
+    most = planner.strips_plan(len(ptr) - 1, ptr.ctypes.data, col.ctypes.data, int(upper),
+                               _levels_us(ptr.tolist(), col.tolist(), upper), ctypes.byref(strips))
+    return strips.value, most
+
+
+@pytest.mark.parametrize("name", gpu_cases.CASES)
+def test_cases_are_planned_as_meant(planner, name):
+    off, cols, _ = gpu_cases.CASES[name](np.random.default_rng(61))
+    for upper in (False, True):
+        strips, most = _plan(planner, off, cols, upper)
+        low, high = gpu_cases.STRIPS[name]
+        assert low <= strips <= high
+        # the solving wave waits for a group's imports before it has published the
+        # group before as used: both must be in the ring at a time
+        assert most <= planner.strips_imports()
+        if name in gpu_cases.FULL_RING:
+            assert most > 1024  # (two groups of three imports per row: 1,152)

@@ -38,11 +38,12 @@ namespace tnlmi {
 namespace {
 
 constexpr int kWin = 48;                       // steps whose values stay in LDS (a multiple of kAhead)
-constexpr int kImports = 1024;                 // imported values in LDS
+constexpr int kImports = kTriImports;          // imported values in LDS
 constexpr int kExt = kWin * 64;                // LDS address of the first import
 constexpr int kZero = kExt + kImports;         // LDS address of a 0 (an absent entry)
+static_assert( 8 * kZero <= 0xffff, "LDS byte addresses of 16 bits" );
 constexpr int kAhead = 12;                     // steps whose records are requested ahead
-constexpr int kGroup = 3;                      // steps between two looks at the other waves' flags (divides kAhead)
+constexpr int kGroup = kTriGroup;              // steps between two looks at the other waves' flags (divides kAhead)
 constexpr int kBatches = 8;                    // batches of 64 imports requested together at most
 constexpr int kMaxStrips = 256;                // one per CU
 // pivots and quotients for which the quotient from the reciprocal is exact to
@@ -528,7 +529,7 @@ TriStripsPlan tri_strips_plan( int64_t N, const std::vector< int32_t >& ptr, con
                if( upper )
                   memcpy( block + R::kD + lane * 16, d, 16 );
             }
-            need[ q / kGroup ] = (int32_t) ( (int64_t) src.size() - src0 );  // (a group's own imports fit: 576 of kImports)
+            need[ q / kGroup ] = (int32_t) ( (int64_t) src.size() - src0 );
          }
          table[ 4 * k + 2 ] = (int32_t) src0;
          table[ 4 * k + 3 ] = (int32_t) ( (int64_t) src.size() - src0 );

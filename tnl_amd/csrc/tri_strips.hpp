@@ -8,6 +8,13 @@
 
 namespace tnlmi {
 
+constexpr int kTriGroup = 3;       // steps between two looks at the other waves' flags
+// Imported values in LDS.  Before a group of steps the solving wave waits for the
+// group's imports while the group before, in progress, still holds its own: two
+// groups' imports, three per row, have to fit.
+constexpr int kTriImports = 2048;
+static_assert( kTriImports >= 2 * kTriGroup * 64 * 3 && ( kTriImports & ( kTriImports - 1 ) ) == 0 );
+
 // One triangular factor prepared for the strip solve.  Rows are taken in solve
 // order t (lower: row t, upper: row N - 1 - t); a position is 64 * step + lane
 // over all strips.
