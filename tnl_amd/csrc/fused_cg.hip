@@ -681,6 +681,7 @@ struct GridCg
    const void* d;             // Jacobi diagonal (NULL: none)
    CgDev* st;
    GridSlots* slots;
+   uint64_t wait;             // for a workgroup in a grid sum
    uint32_t number;           // of the first grid sum
    int32_t most;              // iterations at most
    int32_t* late;             // a grid sum was given up
@@ -790,7 +791,7 @@ __global__ void __launch_bounds__( THREADS ) grid_cg( GridCg< T, X > a )
       }
       first = false;
       cur ^= 1;
-      if( ! grid_sum< THREADS >( part, a.slots, number++, sm ) ) {
+      if( ! grid_sum< THREADS >( part, a.slots, number++, a.wait, sm ) ) {
          if( threadIdx.x == 0 )
             *a.late = 1;
          return;
@@ -812,7 +813,7 @@ __global__ void __launch_bounds__( THREADS ) grid_cg( GridCg< T, X > a )
                sums[ 1 ] += (double) r[ j ] * (double) r[ j ];
             }
          }
-         if( ! grid_sum< THREADS >( sums, a.slots, number++, sm ) ) {
+         if( ! grid_sum< THREADS >( sums, a.slots, number++, a.wait, sm ) ) {
             if( threadIdx.x == 0 )
                *a.late = 1;
             return;
@@ -1869,6 +1870,7 @@ struct GridWork
       a.p[ 1 ] = p1.ptr;
       a.z = z.ptr;
       a.slots = slots.ptr;
+      a.wait = grid_wait();
       a.number = number;
       a.most = kGridIterations;
       a.late = late.ptr;

@@ -5,13 +5,22 @@
 // iteration used to end one; a grid sum takes about 2 us.
 #pragma once
 
+#include <cstdlib>
+
 #include "common.hpp"
 
 namespace tnlmi {
 
 constexpr int kGridMax = 256;        // workgroups at most: one per CU
 constexpr int kGridValues = 32;      // values per sum at most
-constexpr uint64_t kGridWait = 200'000'000;  // 100 MHz ticks (2 s) until a wait gives up
+
+// How long a workgroup waits for the others before it gives up, in ticks of
+// 100 MHz: 2 s, or TNLMI_GRID_WAIT_US microseconds.
+inline uint64_t grid_wait()
+{
+   const char* e = std::getenv( "TNLMI_GRID_WAIT_US" );
+   return e ? 100 * std::strtoull( e, nullptr, 10 ) : 200'000'000;
+}
 
 // One value of one workgroup: two words, each with half of the value and the
 // sum's number, so that a reader sees from each word whether it belongs to
@@ -44,9 +53,12 @@ __device__ __forceinline__ void shared_stores_done()
 // v[j] = the sum over all threads of all workgroups, in a fixed order (the same
 // bits in every workgroup).  What a workgroup shared_stores before the sum is
 // seen by all after it.  sm: N * T / 64 doubles of LDS.  Returns false when a
-// workgroup did not arrive in time (then every workgroup gives up).
+// workgroup did not arrive within `wait`.  The others may have seen it arrive and
+// end normally when no sum follows: a kernel whose sum was given up says so in a
+// word that nothing else writes.
 template< int T, int N >
-__device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restrict__ slots, uint32_t number, double* sm )
+__device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restrict__ slots, uint32_t number, uint64_t wait,
+                                          double* sm )
 {
    static_assert( N <= kGridValues && T >= kGridMax, "one thread per workgroup's slot" );
    constexpr int W = T / 64;
@@ -83,6 +95,7 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
       const uint64_t begin = wall_clock64();
       uint64_t lo[ N ], hi[ N ];
       while( true ) {
+         const bool over = wall_clock64() - begin >= wait;  // (before the last look)
          bool there = true;
 #pragma unroll
          for( int j = 0; j < N; j++ ) {
@@ -94,7 +107,7 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
             there = there && (uint32_t) ( lo[ j ] >> 32 ) == number && (uint32_t) ( hi[ j ] >> 32 ) == number;
          if( there )
             break;
-         if( wall_clock64() - begin > kGridWait ) {
+         if( over ) {
             late = 1;
             break;
          }
@@ -118,18 +131,18 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
 
 // A barrier: what a workgroup shared_stores before it is seen by all after it.
 template< int T >
-__device__ __forceinline__ bool grid_barrier( GridSlots* __restrict__ slots, uint32_t number, double* sm )
+__device__ __forceinline__ bool grid_barrier( GridSlots* __restrict__ slots, uint32_t number, uint64_t wait, double* sm )
 {
    double none[ 1 ] = { 0 };
-   return grid_sum< T >( none, slots, number, sm );
+   return grid_sum< T >( none, slots, number, wait, sm );
 }
 
 // grid_sum of `count` values whose wave totals are in sm[ j * T / 64 + wave ]
 // already; the results in out[ j ] (LDS).  sm: kGridValues * T / 64 doubles.
 // Each wave polls 64 workgroups' slots of one value at a time.
 template< int T >
-__device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict__ slots, uint32_t number, double* sm,
-                                               double* out )
+__device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict__ slots, uint32_t number, uint64_t wait,
+                                               double* sm, double* out )
 {
    constexpr int W = T / 64, kAtOnce = 4;
    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, G = gridDim.x;
@@ -153,6 +166,7 @@ __device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict_
       uint64_t lo[ kAtOnce ], hi[ kAtOnce ];
       const uint64_t begin = wall_clock64();
       while( true ) {
+         const bool over = wall_clock64() - begin >= wait;
          bool there = true;
 #pragma unroll
          for( int u = 0; u < kAtOnce; u++ ) {
@@ -165,7 +179,7 @@ __device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict_
             there = there && (uint32_t) ( lo[ u ] >> 32 ) == number && (uint32_t) ( hi[ u ] >> 32 ) == number;
          if( __ballot( ! there ) == 0 )
             break;
-         if( wall_clock64() - begin > kGridWait ) {
+         if( wave_uniform( (int32_t) over ) ) {
             late = 1;
             break;
          }

@@ -31,6 +31,7 @@ public:
    DeviceArray< double > pub[ 2 ];  // vectors that every workgroup reads
    DeviceArray< GridSlots > slots;
    DeviceArray< ResidentState > state;
+   DeviceArray< int32_t > late;  // a grid sum was given up
    uint32_t number = 1;
 };
 
@@ -41,7 +42,9 @@ std::shared_ptr< Resident > resident_work( int64_t n, hipStream_t s )
    w->pub[ 1 ].allocate( n );
    w->slots.allocate( 1 );
    w->state.allocate( 1 );
+   w->late.allocate( 1 );
    TNLMI_HIP( hipMemsetAsync( w->slots.ptr, 0, sizeof( GridSlots ), s ) );
+   TNLMI_HIP( hipMemsetAsync( w->late.ptr, 0, sizeof( int32_t ), s ) );
    return w;
 }
 
@@ -60,6 +63,8 @@ struct Common
    double* pub[ 2 ];
    GridSlots* slots;
    ResidentState* st;
+   int32_t* late;
+   uint64_t wait;
    uint32_t number;
    int64_t maxit, minit;
    double tol, div;
@@ -189,12 +194,13 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
    int64_t it = a.st->it;
    uint32_t number = a.number;
    int32_t end = kResidentMore;
+   bool late = false;
    for( int32_t done = 0; done < kMost; done++ ) {
 #pragma unroll
       for( int j = 0; j < ROWS; j++ )
          R.publish( a.pub[ 0 ], own, j, p[ j ] );
-      if( ! grid_barrier< THREADS >( a.slots, number++, sm ) ) {
-         end = kResidentLate;
+      if( ! grid_barrier< THREADS >( a.slots, number++, a.wait, sm ) ) {
+         late = true;
          break;
       }
       R.product( a.pub[ 0 ], own, 1.0, Ap );
@@ -205,8 +211,8 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
             Ap[ j ] = Ap[ j ] / R.load( a.d, j, 1.0 );
          one[ 0 ] += Ap[ j ] * R.load( a.rast, j );
       }
-      if( ! grid_sum< THREADS >( one, a.slots, number++, sm ) ) {
-         end = kResidentLate;
+      if( ! grid_sum< THREADS >( one, a.slots, number++, a.wait, sm ) ) {
+         late = true;
          break;
       }
       alpha = rho / one[ 0 ];
@@ -215,8 +221,8 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          s[ j ] = r[ j ] - alpha * Ap[ j ];
          R.publish( a.pub[ 1 ], own, j, s[ j ] );
       }
-      if( ! grid_barrier< THREADS >( a.slots, number++, sm ) ) {
-         end = kResidentLate;
+      if( ! grid_barrier< THREADS >( a.slots, number++, a.wait, sm ) ) {
+         late = true;
          break;
       }
       double As[ ROWS ];
@@ -229,8 +235,8 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          two[ 0 ] += As[ j ] * s[ j ];
          two[ 1 ] += As[ j ] * As[ j ];
       }
-      if( ! grid_sum< THREADS >( two, a.slots, number++, sm ) ) {
-         end = kResidentLate;
+      if( ! grid_sum< THREADS >( two, a.slots, number++, a.wait, sm ) ) {
+         late = true;
          break;
       }
       omega = two[ 0 ] / two[ 1 ];
@@ -242,8 +248,8 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          two[ 0 ] += r[ j ] * R.load( a.rast, j );
          two[ 1 ] += r[ j ] * r[ j ];
       }
-      if( ! grid_sum< THREADS >( two, a.slots, number++, sm ) ) {
-         end = kResidentLate;
+      if( ! grid_sum< THREADS >( two, a.slots, number++, a.wait, sm ) ) {
+         late = true;
          break;
       }
       rho_old = rho;
@@ -265,9 +271,9 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          break;
       }
    }
-   if( end == kResidentLate ) {
+   if( late ) {
       if( threadIdx.x == 0 )
-         a.st->end = kResidentLate;  // (every workgroup may write the same)
+         *a.late = 1;
       return;
    }
 #pragma unroll
@@ -385,9 +391,9 @@ __global__ void __launch_bounds__( THREADS ) gmres_resident( GmresArgs a )
    for( int j = 0; j < ROWS; j++ )
       w[ j ] = R.load( a.r, j );
    bool late = false;
-   auto barrier = [ & ] { late = late || ! grid_barrier< THREADS >( a.slots, number++, sm ); };
+   auto barrier = [ & ] { late = late || ! grid_barrier< THREADS >( a.slots, number++, a.wait, sm ); };
    auto sum = [ & ]( double ( &v )[ 1 ] ) {
-      late = late || ! grid_sum< THREADS >( v, a.slots, number++, sm );
+      late = late || ! grid_sum< THREADS >( v, a.slots, number++, a.wait, sm );
       v[ 0 ] = wave_uniform( v[ 0 ] );  // (also where no sum was taken: what follows from it branches)
    };
    // sums of `count` values, value k's per-thread part in acc[ k - k0 ] for the group at k0
@@ -448,7 +454,7 @@ __global__ void __launch_bounds__( THREADS ) gmres_resident( GmresArgs a )
                own[ j * THREADS + threadIdx.x ] = w[ j ];
             for( int pass = 0; pass <= a.passes; pass++ ) {
                if( pass > 0 ) {
-                  late = late || ! grid_sum_many< THREADS >( count, a.slots, number++, sm, g.h );
+                  late = late || ! grid_sum_many< THREADS >( count, a.slots, number++, a.wait, sm, g.h );
                   if( (int) threadIdx.x < count )
                      H[ threadIdx.x ] = pass == 1 ? g.h[ threadIdx.x ] : H[ threadIdx.x ] + g.h[ threadIdx.x ];
                }
@@ -622,7 +628,7 @@ __global__ void __launch_bounds__( THREADS ) gmres_resident( GmresArgs a )
    }
    if( late ) {
       if( threadIdx.x == 0 )
-         a.st->end = kResidentLate;
+         *a.late = 1;
       return;
    }
 #pragma unroll
@@ -647,6 +653,8 @@ void fill_common( Common& c, Resident& w, const EllSlots& A, const double* d, co
    c.pub[ 1 ] = w.pub[ 1 ].ptr;
    c.slots = w.slots.ptr;
    c.st = w.state.ptr;
+   c.late = w.late.ptr;
+   c.wait = grid_wait();
    c.number = w.number;
    c.maxit = S.st->max_iterations;
    c.minit = S.st->min_iterations;
@@ -669,11 +677,16 @@ void put_state( Resident& w, const ResidentState& h, hipStream_t s )
 {
    TNLMI_HIP( hipMemcpyAsync( w.state.ptr, &h, sizeof( h ), hipMemcpyHostToDevice, s ) );
 }
+// (where any workgroup gave up: kResidentLate, whatever state the others left)
 ResidentState get_state( Resident& w, hipStream_t s )
 {
    ResidentState h;
+   int32_t late = 0;
    TNLMI_HIP( hipMemcpyAsync( &h, w.state.ptr, sizeof( h ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipMemcpyAsync( &late, w.late.ptr, sizeof( late ), hipMemcpyDeviceToHost, s ) );
    TNLMI_HIP( hipStreamSynchronize( s ) );
+   if( late )
+      h.end = kResidentLate;
    return h;
 }
 
