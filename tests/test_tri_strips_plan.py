@@ -1,8 +1,9 @@
-"""The host's plans of the strip solves (ILU(0) factors): every factor that
+"""CPU checks of the strip solves.  The host's plans of the strip solves (ILU(0) factors): every factor that
 tests/test_tri_strips_gpu.py solves is planned as it is meant to be, and the
 imports that the solving wave can wait for fit the LDS ring that holds them."""
 import ctypes
 import os
+import re
 import subprocess
 
 import numpy as np
@@ -78,3 +79,19 @@ def test_cases_are_planned_as_meant(planner, name):
         assert most <= planner.strips_imports()
         if name in gpu_cases.FULL_RING:
             assert most > 1024  # (two groups of three imports per row: 1,152)
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_strips_are_taken_in_the_order_of_starting(tmp_path):
+    """A strip waits for earlier ones, and workgroups need not start in the order of
+    their numbers (each XCD starts its own): every solve kernel takes its strip
+    from a counter, by an atomic that returns the value before."""
+    out = tmp_path / "tri_strips.s"
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "--cuda-device-only", "-S",
+                    "-o", str(out), os.path.join(CSRC, "tri_strips.hip")], check=True, capture_output=True)
+    kernels = re.findall(r"^(_Z\w*10tri_stripsI\w*):(.*?)s_endpgm", out.read_text(), re.M | re.S)
+    assert len(kernels) == 4
+    for name, body in kernels:
+        first = body.index("s_barrier")
+        assert re.search(r"global_atomic_add v\d+, .* sc0", body[:first]), name

@@ -22,11 +22,12 @@
 // multiply-adds, with everything else (record requests, flags) issued while
 // LDS answers (0.16 us when these stood in the chain).
 //
-// Waiting: a strip reads earlier strips only, workgroup j solves strip j, and
-// workgroups start in order, so the strips a running one waits for have
-// started.  Every wait is bounded all the same: an import that is not there
-// after spin_cap polls ends all waiting of its workgroup, whose values become
-// NaN.  "Not there" is a signalling NaN written before the solve, a
+// Waiting: a strip reads earlier strips only, and workgroups take the strips in
+// the order in which they start (a counter: the XCDs start their workgroups
+// independently, and other kernels may keep one of them busy), so the strips a
+// running one waits for have started.  Every wait is bounded all the same: an
+// import that is not there after spin_cap polls ends all waiting of its
+// workgroup, whose values become NaN.  "Not there" is a signalling NaN written before the solve, a
 // value that no arithmetic gives.
 #include <algorithm>
 #include <cmath>
@@ -63,6 +64,7 @@ struct Shared
    int32_t present;  // imports in LDS so far
    int32_t written;  // steps written out
    int32_t failed;
+   int32_t strip;
 };
 
 // LDS flags: accesses of one wave to LDS complete in order, so a flag written
@@ -117,14 +119,13 @@ struct Record
 template< bool UPPER, int K >
 __global__ void __launch_bounds__( 192 )
    tri_strips( const int32_t* __restrict__ table, const int32_t* __restrict__ need, const int32_t* __restrict__ src,
-               const char* __restrict__ records, double* x, int64_t spin_cap )
+               const char* __restrict__ records, double* x, int32_t* started, int64_t spin_cap )
 {
    using R = Record< UPPER, K >;
    __shared__ Shared S;
    const int wave = wave_uniform( (int32_t) ( threadIdx.x >> 6 ) ), lane = threadIdx.x & 63;
-   const int32_t step0 = table[ 4 * blockIdx.x ], steps = table[ 4 * blockIdx.x + 1 ];
-   const int32_t src0 = table[ 4 * blockIdx.x + 2 ], imports = table[ 4 * blockIdx.x + 3 ];
    if( threadIdx.x == 0 ) {
+      S.strip = atomicAdd( started, 1 );
       S.v[ kZero ] = 0.0;
       S.solved = 0;
       S.used = 0;
@@ -133,6 +134,11 @@ __global__ void __launch_bounds__( 192 )
       S.failed = 0;
    }
    __syncthreads();
+   const int32_t strip = wave_uniform( S.strip );
+   if( strip >= (int32_t) gridDim.x )
+      return;  // (not if tri_strips_load came before)
+   const int32_t step0 = table[ 4 * strip ], steps = table[ 4 * strip + 1 ];
+   const int32_t src0 = table[ 4 * strip + 2 ], imports = table[ 4 * strip + 3 ];
    // LDS waits end when another wave of the workgroup goes on; their own limit
    // only backs that up
    const int64_t lds_cap = spin_cap * 16;
@@ -312,11 +318,14 @@ __global__ void __launch_bounds__( 192 )
 // block, at: bytes of a step's records and where in them the right-hand side is
 __global__ void __launch_bounds__( 256 )
    strips_load( int64_t n, const int32_t* __restrict__ map, const double* __restrict__ src,
-                char* __restrict__ records, uint32_t block, uint32_t at, double* __restrict__ x )
+                char* __restrict__ records, uint32_t block, uint32_t at, double* __restrict__ x,
+                int32_t* __restrict__ started )
 {
    const int64_t p = (int64_t) blockIdx.x * 256 + threadIdx.x;
    if( p >= n )
       return;
+   if( p == 0 )
+      *started = 0;
    const int32_t i = map[ p ];
    // (an idle lane: not 0, which would take the division)
    *(double*) ( records + ( p >> 6 ) * block + at + ( p & 63 ) * 8 ) = i >= 0 ? src[ i ] : 1.0;
@@ -556,20 +565,21 @@ void tri_strips_upload( TriStrips& T, const TriStripsPlan& P, hipStream_t s )
    upload( T.pos, P.pos, s );
    upload( T.records, P.records, s );
    T.x.allocate( P.steps * 64 );
+   T.started.allocate( 1 );
    T.strips = P.strips;
 }
 
 void tri_strips_load( TriStrips& T, const double* src, const int32_t* map, hipStream_t s )
 {
    hipLaunchKernelGGL( strips_load, dim3( (unsigned) ceil_div( T.steps * 64, 256 ) ), dim3( 256 ), 0, s, T.steps * 64,
-                       map, src, T.records.ptr, T.block, T.b_at, T.x.ptr );
+                       map, src, T.records.ptr, T.block, T.b_at, T.x.ptr, T.started.ptr );
 }
 
 void tri_strips_solve( TriStrips& T, int64_t spin_cap, hipStream_t s )
 {
    auto go = [ & ]( auto kernel ) {
       hipLaunchKernelGGL( kernel, dim3( (unsigned) T.strips ), dim3( 192 ), 0, s, T.table.ptr, T.need.ptr, T.src.ptr,
-                          (const char*) T.records.ptr, T.x.ptr, spin_cap );
+                          (const char*) T.records.ptr, T.x.ptr, T.started.ptr, spin_cap );
    };
    if( T.upper )
       T.entries > 2 ? go( tri_strips< true, 3 > ) : go( tri_strips< true, 2 > );

@@ -33,6 +33,7 @@ struct TriStrips
    DeviceArray< char > records;   // per step: addresses, values, pivots and right-hand side of its 64 rows
    uint32_t block = 0, b_at = 0;  // bytes of a step's records; where in them the right-hand side is
    DeviceArray< double > x;       // solution by position
+   DeviceArray< int32_t > started;  // workgroups of the solve that have started
    bool used() const { return strips > 0; }
 };
 
