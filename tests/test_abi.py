@@ -62,3 +62,12 @@ def test_generators():
     assert -1 <= u.min() and u.max() < 1 and abs(u.mean()) < 0.01
     g = tnl_amd.normal(100000, seed=0)
     assert abs(g.mean()) < 0.02 and abs(g.std() - 1) < 0.02
+
+
+def test_no_cooperative_launches():
+    """Resident solves are ordinary launches (a process that made cooperative ones
+    from several threads ended in a segmentation fault)."""
+    import subprocess
+    names = subprocess.run(["nm", "-D", "--undefined-only", os.path.join(ROOT, "tnl_amd", "libtnlmi.so")], check=True,
+                           capture_output=True, text=True).stdout
+    assert "hipLaunchKernel" in names and "Cooperative" not in names

@@ -883,18 +883,15 @@ __global__ void __launch_bounds__( THREADS ) grid_cg( GridCg< T, X > a )
 constexpr int64_t kGridRows = int64_t( kGridMax ) * 1024 * 4;
 constexpr int32_t kGridIterations = 4096;  // per launch
 
-// One launch of grid_cg; false: this case is none for it (nothing was launched).
+// One launch of grid_cg, in the caller's resident_turn(); false: this case is none
+// for it (nothing was launched).
 template< typename V, typename T, typename X, typename D, bool MIXED >
 bool grid_cg_launch( const GridCg< T, X >& a, hipStream_t s )
 {
    auto go = [ & ]( auto kernel, int threads, int rows ) {
       GridCg< T, X > arg = a;
       void* args[] = { &arg };
-      const dim3 grid( (unsigned) ceil_div( a.n, (int64_t) threads * rows ) );
-      if( hipLaunchCooperativeKernel( (const void*) kernel, grid, dim3( threads ), args, 0, s ) == hipSuccess )
-         return true;
-      (void) hipGetLastError();
-      return false;
+      return resident_launch( (const void*) kernel, ceil_div( a.n, (int64_t) threads * rows ), threads, args, s );
    };
    const bool keep = a.w <= kGridWidth;
    const int64_t per_thread = ceil_div( a.n, (int64_t) kGridMax * 1024 );
@@ -1970,6 +1967,7 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
       a.st = dev.ptr;
       a.R = R;
       do {
+         const auto turn = resident_turn();
          work.fill( a, S, p.ptr );
          if( ! grid_cg_launch< double, double, double, double, false >( a, s ) )
             break;
@@ -2155,6 +2153,7 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
             a.tol = R.tol;
             a.maxit = R.maxit;
             do {
+               const auto turn = resident_turn();
                grid->fill( a, S, p.ptr );
                const bool launched = A_lo->value_type == TNLMI_F32
                                         ? grid_cg_launch< float, float, float, float, true >( a, s )

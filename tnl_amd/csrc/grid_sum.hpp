@@ -1,11 +1,12 @@
 // grid_sum.hpp -- sums over all workgroups of a running kernel, and data
 // passed between its workgroups, for kernels whose whole grid is resident
-// (cooperative launches): an iteration of a Krylov solver then needs no kernel
+// (resident_launch): an iteration of a Krylov solver then needs no kernel
 // boundary.  A launch costs about 5 us on MI355X and each reduction of an
 // iteration used to end one; a grid sum takes about 2 us.
 #pragma once
 
 #include <cstdlib>
+#include <mutex>
 
 #include "common.hpp"
 
@@ -20,6 +21,32 @@ inline uint64_t grid_wait()
 {
    const char* e = std::getenv( "TNLMI_GRID_WAIT_US" );
    return e ? 100 * std::strtoull( e, nullptr, 10 ) : 200'000'000;
+}
+
+// Launches a kernel whose workgroups wait for each other: at most one per compute
+// unit, so all are on the chip at the same time once other kernels have ended.
+// Two such kernels at a time could each hold units that the other waits for: the
+// caller holds resident_turn() from the launch until the kernel has ended.  (No
+// cooperative launch: a process with such launches from several threads' streams
+// ended in a segmentation fault at its exit.)  False: nothing was launched.
+inline bool resident_launch( const void* kernel, int64_t blocks, int threads, void** args, hipStream_t s )
+{
+   int dev = 0, cus = 0;
+   if( hipGetDevice( &dev ) == hipSuccess
+       && hipDeviceGetAttribute( &cus, hipDeviceAttributeMultiprocessorCount, dev ) == hipSuccess && blocks <= cus
+       && blocks <= kGridMax
+       && hipLaunchKernel( kernel, dim3( (unsigned) blocks ), dim3( threads ), args, 0, s ) == hipSuccess )
+      return true;
+   (void) hipGetLastError();
+   return false;
+}
+// the device's: its streams' kernels share the compute units
+inline std::unique_lock< std::mutex > resident_turn()
+{
+   static std::mutex turns[ 16 ];
+   int dev = 0;
+   (void) hipGetDevice( &dev );
+   return std::unique_lock< std::mutex >( turns[ dev & 15 ] );
 }
 
 // One value of one workgroup: two words, each with half of the value and the
@@ -94,8 +121,8 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
    if( (int) threadIdx.x < G ) {
       const uint64_t begin = wall_clock64();
       uint64_t lo[ N ], hi[ N ];
+      bool over = false;
       while( true ) {
-         const bool over = wall_clock64() - begin >= wait;  // (before the last look)
          bool there = true;
 #pragma unroll
          for( int j = 0; j < N; j++ ) {
@@ -107,10 +134,11 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
             there = there && (uint32_t) ( lo[ j ] >> 32 ) == number && (uint32_t) ( hi[ j ] >> 32 ) == number;
          if( there )
             break;
-         if( over ) {
+         if( over ) {  // (and looked once more)
             late = 1;
             break;
          }
+         over = wall_clock64() - begin >= wait;
       }
 #pragma unroll
       for( int j = 0; j < N; j++ )
@@ -165,8 +193,8 @@ __device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict_
    for( int job0 = w * kAtOnce; job0 < jobs; job0 += W * kAtOnce ) {
       uint64_t lo[ kAtOnce ], hi[ kAtOnce ];
       const uint64_t begin = wall_clock64();
+      bool over = false;
       while( true ) {
-         const bool over = wall_clock64() - begin >= wait;
          bool there = true;
 #pragma unroll
          for( int u = 0; u < kAtOnce; u++ ) {
@@ -179,10 +207,11 @@ __device__ __forceinline__ bool grid_sum_many( int count, GridSlots* __restrict_
             there = there && (uint32_t) ( lo[ u ] >> 32 ) == number && (uint32_t) ( hi[ u ] >> 32 ) == number;
          if( __ballot( ! there ) == 0 )
             break;
-         if( wave_uniform( (int32_t) over ) ) {
+         if( over ) {
             late = 1;
             break;
          }
+         over = wave_uniform( (int32_t) ( wall_clock64() - begin >= wait ) );
       }
 #pragma unroll
       for( int u = 0; u < kAtOnce; u++ ) {

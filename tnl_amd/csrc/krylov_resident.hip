@@ -194,13 +194,12 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
    int64_t it = a.st->it;
    uint32_t number = a.number;
    int32_t end = kResidentMore;
-   bool late = false;
    for( int32_t done = 0; done < kMost; done++ ) {
 #pragma unroll
       for( int j = 0; j < ROWS; j++ )
          R.publish( a.pub[ 0 ], own, j, p[ j ] );
       if( ! grid_barrier< THREADS >( a.slots, number++, a.wait, sm ) ) {
-         late = true;
+         end = kResidentLate;
          break;
       }
       R.product( a.pub[ 0 ], own, 1.0, Ap );
@@ -212,7 +211,7 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          one[ 0 ] += Ap[ j ] * R.load( a.rast, j );
       }
       if( ! grid_sum< THREADS >( one, a.slots, number++, a.wait, sm ) ) {
-         late = true;
+         end = kResidentLate;
          break;
       }
       alpha = rho / one[ 0 ];
@@ -222,7 +221,7 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          R.publish( a.pub[ 1 ], own, j, s[ j ] );
       }
       if( ! grid_barrier< THREADS >( a.slots, number++, a.wait, sm ) ) {
-         late = true;
+         end = kResidentLate;
          break;
       }
       double As[ ROWS ];
@@ -236,7 +235,7 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          two[ 1 ] += As[ j ] * As[ j ];
       }
       if( ! grid_sum< THREADS >( two, a.slots, number++, a.wait, sm ) ) {
-         late = true;
+         end = kResidentLate;
          break;
       }
       omega = two[ 0 ] / two[ 1 ];
@@ -249,7 +248,7 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          two[ 1 ] += r[ j ] * r[ j ];
       }
       if( ! grid_sum< THREADS >( two, a.slots, number++, a.wait, sm ) ) {
-         late = true;
+         end = kResidentLate;
          break;
       }
       rho_old = rho;
@@ -271,7 +270,7 @@ __global__ void __launch_bounds__( THREADS ) bicgstab_resident( BicgArgs a )
          break;
       }
    }
-   if( late ) {
+   if( end == kResidentLate ) {
       if( threadIdx.x == 0 )
          *a.late = 1;
       return;
@@ -666,11 +665,7 @@ template< typename Args >
 bool launch( const void* kernel, int threads, int rows, Args& a, hipStream_t s )
 {
    void* args[] = { &a };
-   const dim3 grid( (unsigned) ceil_div( a.n, (int64_t) threads * rows ) );
-   if( hipLaunchCooperativeKernel( kernel, grid, dim3( threads ), args, 0, s ) == hipSuccess )
-      return true;
-   (void) hipGetLastError();
-   return false;
+   return resident_launch( kernel, ceil_div( a.n, (int64_t) threads * rows ), threads, args, s );
 }
 
 void put_state( Resident& w, const ResidentState& h, hipStream_t s )
@@ -706,6 +701,7 @@ ResidentEnd resident_bicgstab( Resident& w, const ResidentBicgstab& q, Stop& S, 
    a.eps2 = q.eps2;
    ResidentState h{};
    h.it = S.it;
+   const auto turn = resident_turn();  // (until get_state)
    put_state( w, h, s );
    const bool keep = a.w <= kWidth;
    const int64_t n = a.n;
@@ -757,6 +753,7 @@ ResidentEnd resident_gmres( Resident& w, const ResidentGmres& q, Stop& S, double
    h.beta_ratio = beta_ratio;
    h.cycles = cycles;
    h.m = m;
+   const auto turn = resident_turn();  // (until get_state)
    put_state( w, h, s );
    const bool keep = a.w <= kWidth;
    const int64_t n = a.n;
