@@ -1,6 +1,8 @@
 """CG on row masks (large matrices of few distinct (column - row, value) pairs):
 the iterations of the stored matrix, for 1-byte and 2-byte masks, a diagonal
 that varies or not, and matrices that the masks must refuse."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -104,3 +106,38 @@ def test_pairs_of_signed_zero_and_nan():
     s.setMatrix(A)
     x.zero_()
     assert not s.solve(b, x)
+
+
+def _seconds(A, b, limit):
+    s = S.CG()
+    s.setMatrix(A)
+    s.setConvergenceResidue(1e-30)
+    s.setMaxIterations(limit)
+    x = torch.zeros_like(b)
+    best = np.inf
+    for _ in range(4):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        s.solve(b, x.zero_())
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+@pytest.mark.parametrize("kind", ["all_differ", "last_row"])
+def test_refusal_is_cheap(monkeypatch, kind):
+    """A matrix of many pairs is refused within the time of a few iterations (0.2 ms
+    each here), wherever its pairs begin to differ."""
+    nx, ny = 2048, 1024
+    coefficient = (lambda x, y: 1.0 + (x * 7919 + y * 104729) % 100003 / 1e5) if kind == "all_differ" else \
+        (lambda x, y: np.where(x + nx * y > nx * ny - 40, 2.0 + x / nx, 1.0))
+    off, cols, vals = _stencil(nx, ny, coefficient)
+    n = nx * ny
+    A = tnl.SparseMatrix.from_csr(n, n, off, cols, vals, fmt=tnl.ELLPACK)
+    b = torch.ones(n, dtype=torch.float64, device="cuda")
+    t = {}
+    for codes in ("1", "0"):
+        monkeypatch.setenv("TNLMI_COLUMN_CODES", codes)
+        t[codes] = _seconds(A, b, 20)
+    print(kind, t, flush=True)
+    assert t["1"] <= t["0"] + 1e-3

@@ -962,16 +962,21 @@ __device__ __forceinline__ uint64_t pair_mix( int32_t off, uint64_t bits )
    return z == kEmpty ? 0 : z;
 }
 
+// The pairs of the first `rows` rows into the table.  A matrix of many pairs has to
+// be refused at once: with half a million threads probing a full table a refusal took
+// 48 ms on 128^3 rows.  So no thread probes past kPairs occupied entries or
+// after the refusal, and a first launch over few rows refuses before most threads
+// start (0.1 ms; 0.15 ms where only the last rows differ).
 template< typename V >
 __global__ void __launch_bounds__( kFT ) pairs_collect( SegView v, const int32_t* __restrict__ cols,
-                                                        const V* __restrict__ vals, PairTable* table )
+                                                        const V* __restrict__ vals, PairTable* table, int64_t rows )
 {
    __shared__ unsigned long long seen[ kFT ];  // by the key's low bits: pairs that are in the table
    seen[ threadIdx.x ] = kEmpty;
    __syncthreads();
    constexpr int kEntries = 8;  // loaded together
-   for( int64_t r = (int64_t) blockIdx.x * kFT + threadIdx.x; r < v.n; r += (int64_t) gridDim.x * kFT ) {
-      const int32_t reject = *(volatile int32_t*) &table->reject;
+   for( int64_t r = (int64_t) blockIdx.x * kFT + threadIdx.x; r < rows; r += (int64_t) gridDim.x * kFT ) {
+      const int32_t reject = shared_load( &table->reject );
       int32_t w = 0;
       ell_slot( v, r, 0, &w );
       for( int32_t k0 = 0; k0 < w; k0 += kEntries ) {
@@ -999,12 +1004,14 @@ __global__ void __launch_bounds__( kFT ) pairs_collect( SegView v, const int32_t
          for( int u = 0; u < kEntries; u++ ) {  // (rarely)
             if( ! ( fresh >> u & 1 ) )
                continue;
+            if( shared_load( &table->reject ) )
+               return;
             const int64_t g = ell_slot( v, r, min( k0 + u, w - 1 ), &w );
             const int32_t off = cols[ g ] - (int32_t) r;
             const uint64_t bit = value_bits( vals, g );
             const unsigned long long key = pair_mix( off, bit );
             bool placed = false;
-            for( int probe = 0, h = (int) ( key >> 40 ) & ( kPairHash - 1 ); probe < kPairHash && ! placed;
+            for( int probe = 0, h = (int) ( key >> 40 ) & ( kPairHash - 1 ); probe <= kPairs && ! placed;
                  probe++, h = ( h + 1 ) & ( kPairHash - 1 ) ) {
                // (a read first: one atomic by every thread at the same pair would queue up)
                unsigned long long prev = shared_load( &table->key[ h ] );
@@ -1014,12 +1021,12 @@ __global__ void __launch_bounds__( kFT ) pairs_collect( SegView v, const int32_t
                   table->val[ h ] = bit;
                   table->off[ h ] = off;
                   if( atomicAdd( &table->count, 1 ) >= kPairs )
-                     atomicExch( &table->reject, 1 );
+                     shared_store( &table->reject, 1 );
                }
                placed = prev == kEmpty || prev == key;
             }
             if( ! placed )
-               atomicExch( &table->reject, 1 );
+               shared_store( &table->reject, 1 );
             __hip_atomic_store( seen + ( key & ( kFT - 1 ) ), key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
          }
       }
@@ -1430,7 +1437,9 @@ void make_masks_v( Stage& S, hipStream_t s )
    PairTable ht;
    TNLMI_HIP( hipMemsetAsync( table.ptr, 0xff, offsetof( PairTable, val ), s ) );
    TNLMI_HIP( hipMemsetAsync( &table.ptr->count, 0, 2 * sizeof( int32_t ), s ) );
-   hipLaunchKernelGGL( pairs_collect< V >, dim3( 2048 ), dim3( kFT ), 0, s, S.v, S.cols, (const V*) S.vals, table.ptr );
+   for( const unsigned grid : { 8u, 2048u } )
+      hipLaunchKernelGGL( pairs_collect< V >, dim3( grid ), dim3( kFT ), 0, s, S.v, S.cols, (const V*) S.vals, table.ptr,
+                          grid == 8 ? std::min< int64_t >( S.v.n, 8 * kFT ) : S.v.n );
    TNLMI_HIP( hipGetLastError() );
    TNLMI_HIP( hipMemcpyAsync( &ht, table.ptr, sizeof( ht ), hipMemcpyDeviceToHost, s ) );
    TNLMI_HIP( hipStreamSynchronize( s ) );
@@ -1496,8 +1505,12 @@ void make_masks( Stage& S, hipStream_t s )
 }
 
 // One iteration by row masks, T: the vectors' type.  p has S.reach + kMaskRoom
-// values of room at both ends, r kMaskRoom at its end.
+// values of room at both ends, r mask_rows_room( n ) values.
 constexpr int64_t kMaskRoom = kFT * 4;
+inline int64_t mask_rows_room( int64_t n )  // (whole groups of 2 or 4 rows)
+{
+   return ceil_div( n, 4 ) * 4;
+}
 template< typename T, typename X, typename DT, bool MIXED >
 void mask_iteration( const Stage& S, T* r, T* p, X* x, const DT* d, T d0, double* part1, double* part2, double* part3,
                      const CgDev* cur, CgDev* nxt, const StopRule& R, double delta2, hipStream_t s )
@@ -1894,7 +1907,7 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
    const double* d = precond_diagonal( M );
    DeviceArray< double > r, p, Ap, sc;
    DeviceArray< CgDev > dev;
-   r.allocate( n + kMaskRoom );
+   r.allocate( mask_rows_room( n ) );
    p.allocate( n );
    Ap.allocate( n );
    sc.allocate( 4 );
@@ -2062,8 +2075,9 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
       DeviceArray< CgDev > dev;
       for( auto* v : { &r64, &d64 } )
          v->allocate( n );
-      for( auto* v : { &r, &p, &Ap, &xc, &d32 } )
-         v->allocate( n + kMaskRoom );
+      r.allocate( mask_rows_room( n ) );
+      for( auto* v : { &p, &Ap, &xc, &d32 } )
+         v->allocate( n );
       sc.allocate( 4 );
       dev.allocate( 2 );
       TNLMI_HIP( hipMemsetAsync( p.ptr, 0, sizeof( float ) * n, s ) );
