@@ -880,6 +880,56 @@ __global__ void __launch_bounds__( THREADS ) grid_cg( GridCg< T, X > a )
    }
 }
 
+// ---- which matrices a resident launch takes.  What a workgroup reads of another's
+// rows goes past the L2, so columns spread over the whole matrix cost more there
+// than in the launches, the more the larger the vectors: CG on uniformly random
+// columns, resident against launch by launch, per iteration: 100,000 rows of 24
+// 35.5 / 43.5 us, 200,000 of 12 39.1 / 39.6, 400,000 of 4 36.4 / 37.4, 524,288 of 3
+// 39.7 / 38.3, 1,000,000 of 2 50.7 / 47.9 and of 12 279 / 123 us.  What counts is the lines
+// that a wave's lanes ask for (neighbouring rows' neighbouring columns share
+// one) beyond the next workgroups' rows: the 27-point grid of 80^3 has 0.76 M and takes
+// 48.7 / 61.5 us, of 100^3 1.58 M and 103 / 92 us.  The next workgroups' rows are mostly
+// found in the L2 all the same: 1,000,000 rows of 12 columns within 3,000 rows 59.9 /
+// 92.3 us, within 30,000 (16 columns) 339 / 131 us.  The line is lines * rows = 4.5e11 in FP64, in the FP32 iteration
+// 9e11 (7e11 against the launches on BF16 values, whose columns are codes): rows
+// of 4, random, 524,288 26.1 / 31.3, 1,000,000 66.5 / 50.6 us; 27-point 100^3 56.2 / 61.5 us
+// in FP32, 72.5 / 57.9 in BF16.  Below 131,073 rows the launches are never faster.
+constexpr double kFar64 = 4.5e11, kFar32 = 9e11, kFarBf16 = 7e11;
+constexpr int kFarGroups = 64;  // groups of 64 rows looked at
+
+// The lines of LINE entries of a vector that one product over the slots asks
+// from rows beyond the next `block` rows' on either side, from kFarGroups of the groups.
+template< int LINE >
+__global__ void __launch_bounds__( 1024 ) far_lines( int64_t n, int64_t stride, int32_t w, const int32_t* __restrict__ cols,
+                                                     int32_t block, double* __restrict__ out )
+{
+   __shared__ int32_t sm[ 16 ];
+   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+   const int64_t groups = ( n + 63 ) / 64;
+   const int32_t every = ( w + 31 ) / 32;  // slots
+   int32_t count = 0, slots = 0;
+   for( int g = wave; g < kFarGroups; g += 16 ) {
+      const int64_t r = groups * g / kFarGroups * 64 + lane;
+      slots = 0;
+      for( int32_t k = 0; k < w; k += every, slots++ ) {
+         const int32_t c = r < n ? cols[ k * stride + r ] : -1;
+         const int32_t line = c >= 0 && abs( c / block - (int32_t) r / block ) > 1 ? c / LINE : -1;
+         const int32_t before = __shfl_up( line, 1, 64 );
+         count += line >= 0 && ( lane == 0 || line != before ) ? 1 : 0;
+      }
+   }
+   count = group_sum< 64 >( count );
+   if( lane == 0 )
+      sm[ wave ] = count;
+   __syncthreads();
+   if( threadIdx.x == 0 ) {
+      double t = 0;
+      for( int i = 0; i < 16; i++ )
+         t += sm[ i ];
+      *out = t * ( (double) groups / kFarGroups ) * ( (double) w / max( slots, 1 ) );
+   }
+}
+
 constexpr int64_t kGridRows = int64_t( kGridMax ) * 1024 * 4;
 constexpr int32_t kGridIterations = 4096;  // per launch
 
@@ -1888,11 +1938,24 @@ struct GridWork
    }
 };
 
-// which matrices grid_cg takes: Ellpack slots (the matrix's own or the copy of
-// a CSR matrix with short rows) of at most kGridRows rows
-bool grid_cg_takes( const Stage& S )
+// Which matrices a resident launch takes: Ellpack slots (the matrix's own or the
+// copy of a CSR matrix with short rows) of at most kGridRows rows, with few
+// enough far lines for vectors of LINE entries per 128 bytes (kFar64 and so on).
+template< int LINE >
+bool grid_takes( const Stage& S, double far, hipStream_t s )
 {
-   return S.kind == 1 && S.v.format == TNLMI_ELLPACK && S.v.n > 0 && S.v.n <= kGridRows;
+   const int64_t n = S.v.n;
+   if( S.kind != 1 || S.v.format != TNLMI_ELLPACK || n <= 0 || n > kGridRows )
+      return false;
+   if( n <= (int64_t) kGridMax * 512 || (double) n * n * S.v.ell_width <= far )
+      return true;
+   const int32_t block = n <= (int64_t) kGridMax * 1024 ? 1024 : n <= (int64_t) kGridMax * 2048 ? 2048 : 4096;
+   double lines = 0;
+   hipLaunchKernelGGL( far_lines< LINE >, dim3( 1 ), dim3( 1024 ), 0, s, n, (int64_t) S.v.ell_aligned, S.v.ell_width, S.cols,
+                       block, S.part->ptr );
+   TNLMI_HIP( hipMemcpyAsync( &lines, S.part->ptr, sizeof( lines ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipStreamSynchronize( s ) );
+   return lines * n <= far;
 }
 
 }  // namespace
@@ -1944,7 +2007,7 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
    hipLaunchKernelGGL( cg_start, dim3( 1 ), dim3( 1 ), 0, s, dev.ptr, sc.ptr + 0, sc.ptr + 1, sc.ptr + 2, R );
    TNLMI_HIP( hipGetLastError() );
    Stage S = make_stage( A.A, A.plan, s );
-   const bool resident = grid && S.A->value_type == TNLMI_F64 && grid_cg_takes( S );
+   const bool resident = grid && S.A->value_type == TNLMI_F64 && grid_takes< 16 >( S, kFar64, s );
    if( ! resident ) {
       make_masks( S, s );
       if( column_codes && S.kind == 1 && ! S.pairs )
@@ -2022,12 +2085,12 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
 
 }  // namespace
 
-bool ell_slots( const Operator& A, EllSlots& out, hipStream_t s )
+bool ell_slots( const Operator& A, double far, EllSlots& out, hipStream_t s )
 {
    if( A.plan || A.A->value_type != TNLMI_F64 || A.rows > kGridRows )
       return false;
    const Stage S = make_stage( A.A, nullptr, s );
-   if( ! grid_cg_takes( S ) )
+   if( ! grid_takes< 16 >( S, far, s ) )
       return false;
    out.n = S.v.n;
    out.stride = S.v.ell_aligned;
@@ -2111,7 +2174,8 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
          return;
       }
       Stage S = make_stage( A_lo, nullptr, s );
-      if( S.kind == 1 && ! grid_cg_takes( S ) ) {
+      const bool resident = grid_takes< 32 >( S, A_lo->value_type == TNLMI_BF16 ? kFarBf16 : kFar32, s );
+      if( S.kind == 1 && ! resident ) {
          make_masks( S, s );
          if( ! S.pairs )
             make_codes( S, s );
@@ -2131,7 +2195,7 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
       bool first = true;
       int par = 0;  // the state is double-buffered by iteration parity
       std::unique_ptr< GridWork< float > > grid;
-      if( grid_cg_takes( S ) )
+      if( resident )
          grid = std::make_unique< GridWork< float > >( n, s );
       while( true ) {
          // reliable update: r = b - A x in FP64 and the true residual

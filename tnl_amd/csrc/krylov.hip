@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cmath>
 #include <future>
+#include <limits>
 #include <vector>
 
 #include "blas1.hpp"
@@ -1522,7 +1523,8 @@ void gmres_solve( const Operator& A, const tnlmi_preconditioner* M, const double
    };
    // whole cycles in one resident launch, where the matrix and preconditioner allow
    ResidentGmres q{};
-   if( ! cwy && ! inner && ( ! pre || M->kind == TNLMI_PRECOND_DIAGONAL ) && S.check() && ell_slots( A, q.A, s ) ) {
+   if( ! cwy && ! inner && ( ! pre || M->kind == TNLMI_PRECOND_DIAGONAL ) && S.check()
+       && ell_slots( A, std::numeric_limits< double >::infinity(), q.A, s ) ) {
       auto work = resident_work( n, s );
       q.d = precond_diagonal( M );
       q.b = b;

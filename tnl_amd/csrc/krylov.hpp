@@ -101,8 +101,9 @@ struct EllSlots
    const double* vals = nullptr;
    std::shared_ptr< void > own_cols, own_vals;
 };
-// false: the matrix has no such slots, or more rows than a resident launch takes
-bool ell_slots( const Operator& A, EllSlots& out, hipStream_t s );
+// false: the matrix has no such slots, more rows than a resident launch takes, or
+// more lines * rows of far columns than `far` (fused_cg.hip)
+bool ell_slots( const Operator& A, double far, EllSlots& out, hipStream_t s );
 
 // BiCGStab's iterations from an admitted one on (sc: the solver's scalars).
 // Returns what ended them, or kResidentNot when nothing was launched.
