@@ -306,6 +306,7 @@ void chunked_host( tnlmi_segments& seg, const std::vector< int32_t >& sz, hipStr
       for( int32_t i = b; i < e; i++ )
          chunk = std::max( chunk, ( sz[ i ] + s2c[ i ] - 1 ) / s2c[ i ] );
       S[ 1 ] = chunk;
+      seg.ch_longest = std::max( seg.ch_longest, chunk );
       S[ 3 ] = elements;
       elements += C * chunk;
       for( int32_t i = b; i < e; i++ ) {
@@ -851,6 +852,8 @@ void segments_import( tnlmi_segments& seg, const SegmentsFileData& f, hipStream_
          break;
       case TNLMI_CHUNKED_ELLPACK: {
          seg.ch_nslices = f.ch_nslices;
+         for( int64_t si = 0; si < f.ch_nslices; si++ )
+            seg.ch_longest = std::max( seg.ch_longest, f.ch_slices[ 4 * si + 1 ] );
          seg.chunks_in_slice = f.chunks_in_slice;
          seg.desired_chunk_size = f.desired_chunk_size;
          upload( seg.seg_to_chunk, f.seg_to_chunk, s );

@@ -52,6 +52,7 @@ struct tnlmi_segments
    int32_t logw = 5;
 
    // ChunkedEllpack (ChunkedEllpackBase.h)
+   int32_t ch_longest = 0;  // slots of the longest chunk
    tnlmi::DeviceArray< int32_t > ch_slices, seg_to_chunk, seg_to_slice, seg_ptrs, chunks_to_seg;
    int64_t ch_nslices = 0;
    int32_t chunks_in_slice = 256, desired_chunk_size = 16;

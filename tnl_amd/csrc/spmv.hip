@@ -497,10 +497,17 @@ __global__ void __launch_bounds__( 256 ) biellpack( int64_t n, int64_t strips, i
 // kChunkTile slots of every chunk at a time, 64 bytes of columns per request,
 // their products handed to the chunk's thread through LDS: lanes that each walk
 // a chunk of their own need 64 cache lines per load.  500,000 power-law rows of
-// 16 entries on average, FP32 / FP64: 407 / 447 against 1,047 / 1,093 us.
+// 16 entries on average, FP32 / FP64: 407 / 447 against 1,047 / 1,093 us.  Chunks of at
+// most kChunkShort slots share those lines well enough for a lane each, and have
+// no use for most of a tile: 2,000,000 rows of 1, 5, 10 and 12 slots, FP32 as a tile 51, 59, 61
+// and 63 us, by lanes 10, 17, 39 and 53; FP64 56, 62, 87 and 97 against 13, 24, 71 and 100.
+// Where every chunk is short the kernel has no tile (SHORT), whose LDS and
+// registers halve the waves in flight.
 constexpr int kChunkTile = 16;
+constexpr int kChunkShort = 10;
+enum ChunkWalk { CHUNK_COL_MAJOR, CHUNK_SHORT, CHUNK_TILE };
 
-template< typename V, typename X, typename C, bool COL_MAJOR >
+template< typename V, typename X, typename C, ChunkWalk WALK >
 __global__ void __launch_bounds__( 256 ) chunked( int32_t chunks_in_slice, const int32_t* __restrict__ slices,
                                                   const int32_t* __restrict__ seg_to_chunk, Args< V, X, C > a )
 {
@@ -510,11 +517,15 @@ __global__ void __launch_bounds__( 256 ) chunked( int32_t chunks_in_slice, const
                  ptr = slices[ 4 * si + 3 ];
    const int q = threadIdx.x;
    C acc = 0;
-   if constexpr( COL_MAJOR ) {
+   if constexpr( WALK == CHUNK_COL_MAJOR ) {
       if( q < chunks_in_slice )
          acc = strided_sum< V, X, C >( a.cols, a.vals, a.x, ptr + q, chunks_in_slice, cs );
    }
-   else {
+   else if( WALK == CHUNK_SHORT || cs <= kChunkShort ) {
+      if( q < chunks_in_slice )
+         acc = strided_sum< V, X, C, true >( a.cols, a.vals, a.x, ptr + (int64_t) q * cs, 1, cs );
+   }
+   else if constexpr( WALK == CHUNK_TILE ) {
       constexpr int T = kChunkTile;
       __shared__ C tile[ 256 * ( T + 1 ) ];
       const int32_t* __restrict__ cp = a.cols + ptr;
@@ -716,7 +727,9 @@ void spmv_typed( const tnlmi_matrix& A, const void* x, void* y, double alpha, do
          break;
       case TNLMI_CHUNKED_ELLPACK:
          if( seg.ch_nslices )
-            hipLaunchKernelGGL( ( seg.org == TNLMI_COLUMN_MAJOR ? chunked< V, X, C, true > : chunked< V, X, C, false > ),
+            hipLaunchKernelGGL( ( seg.org == TNLMI_COLUMN_MAJOR        ? chunked< V, X, C, CHUNK_COL_MAJOR >
+                                  : seg.ch_longest <= kChunkShort ? chunked< V, X, C, CHUNK_SHORT >
+                                                                  : chunked< V, X, C, CHUNK_TILE > ),
                                 dim3( (unsigned) seg.ch_nslices ), dim3( 256 ), 0, s, seg.chunks_in_slice,
                                 seg.ch_slices.ptr, seg.seg_to_chunk.ptr, a );
          break;
