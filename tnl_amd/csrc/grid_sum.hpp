@@ -121,9 +121,9 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
    if( (int) threadIdx.x < G ) {
       const uint64_t begin = wall_clock64();
       uint64_t lo[ N ], hi[ N ];
-      bool over = false;
+      bool there = true, over = false;
       while( true ) {
-         bool there = true;
+         there = true;
 #pragma unroll
          for( int j = 0; j < N; j++ ) {
             lo[ j ] = shared_load( &buf[ j ][ threadIdx.x ][ 0 ] );
@@ -132,14 +132,11 @@ __device__ __forceinline__ bool grid_sum( double ( &v )[ N ], GridSlots* __restr
 #pragma unroll
          for( int j = 0; j < N; j++ )
             there = there && (uint32_t) ( lo[ j ] >> 32 ) == number && (uint32_t) ( hi[ j ] >> 32 ) == number;
-         if( there )
+         if( __ballot( ! there ) == 0 || over )  // (looked once more after the time)
             break;
-         if( over ) {  // (and looked once more)
-            late = 1;
-            break;
-         }
-         over = wall_clock64() - begin >= wait;
+         over = wave_uniform( (int32_t) ( wall_clock64() - begin >= wait ) );
       }
+      late = there ? 0 : 1;
 #pragma unroll
       for( int j = 0; j < N; j++ )
          v[ j ] = __longlong_as_double( (long long) ( ( hi[ j ] << 32 ) | ( lo[ j ] & 0xffffffffu ) ) );
