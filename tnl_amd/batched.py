@@ -87,16 +87,49 @@ def _device_name():
     return f"{p.name}:{getattr(p, 'gcnArchName', '')}"
 
 
+# The FP64 kernel from LDS and registers takes a batch whose systems all have at
+# most LOCAL_ROWS rows and LOCAL_SLOTS slots per row (kLocalMost and kLocalWidth of
+# csrc/batched.hip).
+LOCAL_ROWS, LOCAL_SLOTS = 16384, 8
+
+
+def _sample(off, cols, vals, sys_rows, k):
+    """The first k systems as a batch of their own, and whether the FP64 solve of the
+    whole batch runs in the kernel from LDS and registers.  If it does not though
+    that of the first k would, the first system beyond its limits is added."""
+    rows_of = np.diff(sys_rows)
+    wide = np.flatnonzero(np.diff(off) > LOCAL_SLOTS)
+    beyond = np.flatnonzero(rows_of > LOCAL_ROWS)
+    first = [int(beyond[0])] if len(beyond) else []
+    if len(wide):
+        first.append(int(np.searchsorted(sys_rows, wide[0], side="right")) - 1)
+    rows = int(sys_rows[k])
+    o, c, v, s = off[: rows + 1], cols[: int(off[rows])], vals[: int(off[rows])], sys_rows[: k + 1]
+    if first and min(first) >= k:
+        r0, r1 = int(sys_rows[min(first)]), int(sys_rows[min(first) + 1])
+        e0, e1 = int(off[r0]), int(off[r1])
+        extra = cols[e0:e1]
+        o = np.concatenate([o, off[r0 + 1 : r1 + 1] - e0 + o[-1]]).astype(off.dtype)
+        c = np.concatenate([c, np.where(extra >= 0, extra - r0 + rows, extra)]).astype(cols.dtype)
+        v = np.concatenate([v, vals[e0:e1]])
+        s = np.append(s, rows + r1 - r0)
+    return o, c, v, s, not first
+
+
 def autotune(off, cols, vals, sys_rows, sample=256, candidates=CANDIDATES, blocks=BLOCKS, lanes=LANES,
              tolerance=1e-10, cache=True, log=None):
     """Times every (format, slice size, workgroup size, rows per wavefront)
     candidate on the first `sample` systems and returns the fastest as a dict.
-    The FP64 solve is timed, or the mixed one where the FP64 solve of these
-    systems runs in its own kernel, which no candidate shapes; results are cached in a JSON file keyed by the batch's shape, the device,
-    the candidate lists and the tolerance."""
+    The FP64 solve is timed, or the mixed one where the FP64 solve of the batch
+    runs in a kernel of its own, which no candidate shapes.  Results are cached in a JSON file
+    keyed by the batch's shape, the solve timed, the device, the candidate lists and the
+    tolerance."""
     import torch
     nsys = len(sys_rows) - 1
-    key = (f"batched_cg:nsys={nsys}:rows={int(sys_rows[-1])}:nnz={int(off[-1])}:sample={sample}"
+    k = min(sample, nsys)
+    o, c, v, rows_k, mixed = _sample(*(a.cpu().numpy() if hasattr(a, "cpu") else np.asarray(a)
+                                       for a in (off, cols, vals, sys_rows)), k)
+    key = (f"batched_cg:solve={'mixed' if mixed else 'fp64'}:local={LOCAL_ROWS}x{LOCAL_SLOTS}:nsys={nsys}:rows={int(sys_rows[-1])}:nnz={int(off[-1])}:sample={sample}"
            f":device={_device_name()}:candidates={sorted((int(f), int(p)) for f, p in candidates)}"
            f":blocks={sorted(int(b) for b in blocks)}:lanes={sorted(int(t) for t in lanes)}"
            f":tolerance={float(tolerance)!r}")
@@ -106,21 +139,16 @@ def autotune(off, cols, vals, sys_rows, sample=256, candidates=CANDIDATES, block
             db = json.load(f)
         if key in db:
             return db[key]
-    k = min(sample, nsys)
-    rows = int(sys_rows[k])
-    o = off[: rows + 1]
-    c, v = cols[: int(o[-1])], vals[: int(o[-1])]
+    rows = int(rows_k[-1])
     b = torch.ones(rows, dtype=torch.float64, device="cuda")
     x = torch.zeros(rows, dtype=torch.float64, device="cuda")
-    # (the limits of the kernel from LDS and registers, see BatchedCG)
-    mixed = k > 0 and int(np.diff(sys_rows[: k + 1]).max()) <= 16384 and int((o[1:] - o[:-1]).max()) <= 8
     trials = []
     for fmt, param in candidates:
         A = SparseMatrix.from_csr(rows, rows, o, c, v, fmt=fmt, param=param)
         A_lo = SparseMatrix(A.rows, A.columns, A.segments, A.values.float(), A.column_indexes) if mixed else None
         for bs in blocks:
             for lpr in lanes:
-                bc = BatchedCG(A, sys_rows[: k + 1], A_lo, block_size=bs, lanes_per_row=lpr)
+                bc = BatchedCG(A, rows_k, A_lo, block_size=bs, lanes_per_row=lpr)
                 x.zero_()
                 bc.solve(b, x, tolerance, mixed=mixed, use_graph=False)
                 torch.cuda.synchronize()
