@@ -465,8 +465,10 @@ tnlmi_status tnlmi_cg_solve( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan,
  * comparisons of FP64 and mixed-precision solves.  column_codes != 0: a
  * column-major Ellpack / SlicedEllpack A with at most 255 distinct offsets
  * column - row is read through 8-bit column codes, as the mixed solver reads
- * its inner matrix (identical results, fewer bytes).  No reference
- * counterpart. */
+ * its inner matrix (identical results, fewer bytes), where the iterations run
+ * neither in one resident launch (Ellpack slots of at most 2^20 rows) nor on
+ * row masks (more rows, at most 16 distinct pairs of offset and value), which
+ * read no columns.  No reference counterpart. */
 tnlmi_status tnlmi_cg_solve_true_residual( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan,
                                            const tnlmi_preconditioner* M, int32_t column_codes, const double* d_b,
                                            double* d_x, tnlmi_solver_state* state, tnlmi_stream stream );

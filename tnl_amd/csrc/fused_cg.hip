@@ -1663,7 +1663,7 @@ void make_codes( Stage& S, hipStream_t s )
 }
 
 // kind 1 launch shape over S.v (column-major Ellpack / SlicedEllpack)
-void ell_shape( Stage& S, hipStream_t s, bool codes )
+void ell_shape( Stage& S )
 {
    S.kind = 1;
    // 16-byte loads of the column indexes for 4-byte values, of the values for FP64
@@ -1673,8 +1673,6 @@ void ell_shape( Stage& S, hipStream_t s, bool codes )
    S.grid = ceil_div( ceil_div( S.v.n, S.rows_per_thread ), kFT );
    S.part = std::make_shared< DeviceArray< double > >();
    S.part->allocate( S.grid );
-   if( codes )
-      make_codes( S, s );
 }
 
 // CSR rows as column-major Ellpack slots: slot j of row r at j * stride + r
@@ -1764,7 +1762,7 @@ bool csr_ell_copy( Stage& S, hipStream_t s )
    return true;
 }
 
-Stage make_stage( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan, hipStream_t s, bool codes = false )
+Stage make_stage( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan, hipStream_t s )
 {
    Stage S;
    S.A = A;
@@ -1777,12 +1775,12 @@ Stage make_stage( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan, hipStream_
       return S;
    const int fmt = S.v.format;
    if( ( fmt == TNLMI_ELLPACK || fmt == TNLMI_SLICED_ELLPACK ) && S.v.col_major && A->matrix_type != TNLMI_SYMMETRIC ) {
-      ell_shape( S, s, codes );
+      ell_shape( S );
       return S;
    }
    const tnlmi_segments& seg = *A->segments;
    if( fmt == TNLMI_CSR && A->matrix_type != TNLMI_SYMMETRIC && csr_ell_copy( S, s ) ) {
-      ell_shape( S, s, codes );
+      ell_shape( S );
       return S;
    }
    if( fmt == TNLMI_CSR && A->matrix_type != TNLMI_SYMMETRIC && seg.max_size <= kWholeRowMax && seg.tiles > 0

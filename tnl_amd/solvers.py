@@ -136,7 +136,8 @@ class TrueResidualCG(IterativeSolver):
     solvers -- instead of the reference's preconditioned residue
     (tnlmi_cg_solve_true_residual).  column_codes: read a column-major
     Ellpack / SlicedEllpack matrix through 8-bit column codes, as the mixed
-    solver reads its inner matrix."""
+    solver reads its inner matrix, where neither the resident launch (at most
+    2^20 rows) nor the row masks (few distinct entries) are taken."""
 
     def __init__(self, column_codes=False):
         super().__init__()
