@@ -73,11 +73,13 @@ CASES = {
     "scattered": lambda g: _scattered(2500, g), "scattered_strips": lambda g: _scattered(12000, g),
     "far_one_strip": lambda g: _far(5000, 3, g), "far_strips": lambda g: _far(6000, 20, g),
     "band_strips": lambda g: _scattered_band(60000, 200, 300, g),
+    "band_full": lambda g: _scattered_band(100000, 64, 800, g), "band_full_small": lambda g: _scattered_band(20000, 128, 640, g),
 }
 # the strips of either factor (test_tri_strips_plan.py checks the plans): none, one or more than one
-STRIPS = {name: (1, 1) if name in ("line64", "thin", "scattered", "scattered_strips", "far_one_strip")
-          else (0, 0) if name == "rows127" else (2, 256) for name in CASES}
-FULL_RING = ("far_one_strip", "far_strips")  # more imports in two groups of steps than two per row
+STRIPS = {name: (1, 1) if name in ("line64", "thin", "scattered")
+          else (0, 0) if name in ("rows127", "scattered_strips", "far_one_strip", "far_strips")
+          else (1, 256) if name.startswith("band_full") else (2, 256) for name in CASES}
+FULL_RING = ("band_full", "band_full_small")  # one factor has almost three imports per row in two groups of steps
 
 
 @pytest.mark.parametrize("name", CASES)

@@ -690,11 +690,12 @@ void ilu0_build( tnlmi_preconditioner& P, const tnlmi_matrix& A, hipStream_t s )
    plan_runs( P.llev, P.lruns );
    plan_runs( P.ulev, P.uruns );
    // what the solves by levels take: 0.65 us per level of a narrow run, a
-   // launch (6 us) per wide level, measured on 5- and 7-point grid factors
+   // launch (5 us) per wide level, measured on 5- and 7-point grid factors and on 20
+   // levels of 6,000 rows (104 us)
    auto level_us = []( const std::vector< tnlmi_preconditioner::Run >& runs ) {
       double us = 0;
       for( const auto& R : runs )
-         us += R.narrow ? 10 + 0.65 * (double) ( R.l1 - R.l0 ) : 6.0;
+         us += R.narrow ? 10 + 0.65 * (double) ( R.l1 - R.l0 ) : 5.0;
       return us;
    };
    const char* fenv = std::getenv( "TNLMI_ILU_FLOW" );

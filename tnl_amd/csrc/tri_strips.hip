@@ -407,6 +407,8 @@ double expected_steps( const Factor& F, int64_t R, std::vector< int32_t >& slot,
             if( d >= before )
                behind = std::max( behind, slot[ d ] / 64 + 1 - slot[ t ] / 64 );
          }
+         else if( slot[ t ] / 64 - slot[ d ] / 64 >= kWin )
+            imports++;  // (not in LDS any more: by way of memory too)
       }
    // (a strip cannot go faster than its imports arrive: about kBatches * 64 per round trip to memory)
    const double rate = std::max< double >( steps, imports * kLagSteps / ( 64.0 * kBatches ) );
