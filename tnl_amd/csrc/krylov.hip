@@ -862,7 +862,7 @@ void precond_apply( const tnlmi_preconditioner* P, int64_t n, const double* b, d
       if( US.used() )
          tri_strips_load( US, LS.x.ptr, P->mid.ptr, s );
       else
-         tri_strips_store( LS, x, s );
+         tri_strips_result( LS, x, s );
    }
    else {
       if( any_ring( P->lruns ) )
@@ -897,7 +897,7 @@ void precond_apply( const tnlmi_preconditioner* P, int64_t n, const double* b, d
       if( ! LS.used() )
          tri_strips_load( US, x, US.row.ptr, s );
       tri_strips_solve( US, spin_cap, s );
-      tri_strips_store( US, x, s );
+      tri_strips_result( US, x, s );
       return;
    }
    // the upper solve's right-hand side is the lower solve's result

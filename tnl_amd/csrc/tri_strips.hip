@@ -333,7 +333,7 @@ __global__ void __launch_bounds__( 256 )
 }
 
 __global__ void __launch_bounds__( 256 )
-   strips_store( int64_t n, const int32_t* __restrict__ pos, const double* __restrict__ xp, double* __restrict__ x )
+   strips_result( int64_t n, const int32_t* __restrict__ pos, const double* __restrict__ xp, double* __restrict__ x )
 {
    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
    if( i < n )
@@ -589,9 +589,9 @@ void tri_strips_solve( TriStrips& T, int64_t spin_cap, hipStream_t s )
       T.entries > 2 ? go( tri_strips< false, 3 > ) : go( tri_strips< false, 2 > );
 }
 
-void tri_strips_store( const TriStrips& T, double* x, hipStream_t s )
+void tri_strips_result( const TriStrips& T, double* x, hipStream_t s )
 {
-   hipLaunchKernelGGL( strips_store, dim3( (unsigned) ceil_div( T.n, 256 ) ), dim3( 256 ), 0, s, T.n, T.pos.ptr,
+   hipLaunchKernelGGL( strips_result, dim3( (unsigned) ceil_div( T.n, 256 ) ), dim3( 256 ), 0, s, T.n, T.pos.ptr,
                        (const double*) T.x.ptr, x );
 }
 

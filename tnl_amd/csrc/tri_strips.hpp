@@ -63,6 +63,6 @@ void tri_strips_load( TriStrips& T, const double* src, const int32_t* map, hipSt
 // the solution by position into T.x
 void tri_strips_solve( TriStrips& T, int64_t spin_cap, hipStream_t s );
 // x[i] = the solution's row i
-void tri_strips_store( const TriStrips& T, double* x, hipStream_t s );
+void tri_strips_result( const TriStrips& T, double* x, hipStream_t s );
 
 }  // namespace tnlmi
