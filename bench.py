@@ -495,7 +495,10 @@ def wl_cg_poisson(args):
         res[label] = rec
         return rec
 
-    nvec64, nvec32 = 11 * 8 * n, 11 * 4 * n  # vector passes of one fused iteration
+    # bytes of one fused iteration: on row masks (above 2^20 rows) two reads of a byte per row
+    # and 9 vector passes, else the matrix and 11 vector passes
+    masks = n > 1 << 20
+    nvec64, nvec32 = 11 * 8 * n, 11 * 4 * n
     for fname, fmt in (("CSR", tnl_amd.CSR), ("Ellpack", tnl_amd.ELLPACK)):
         A = tnl_amd.SparseMatrix.from_csr(n, n, off, cols, vals, fmt=fmt)
         ob = 4 * (n + 1) if fmt == tnl_amd.CSR else 0
@@ -511,7 +514,7 @@ def wl_cg_poisson(args):
         cg.setPreconditioner(solvers.Diagonal(A))
         cg.setConvergenceResidue(tol)
         cg.setMaxIterations(20_000)
-        run(f"fp64_cg[{fname}]", cg, A, 12 * nnz + ob + 16 * n + nvec64)
+        run(f"fp64_cg[{fname}]", cg, A, 74 * n if masks else 12 * nnz + ob + 16 * n + nvec64)
         for lo_name, lo_dtype, sv in (("fp32", torch.float32, 4), ("bf16", torch.bfloat16, 2)):
             A_lo = tnl_amd.SparseMatrix(A.rows, A.columns, A.segments, A.values.to(lo_dtype), A.column_indexes)
             m = solvers.ReliableMixedCG()
@@ -521,7 +524,7 @@ def wl_cg_poisson(args):
             m.setConvergenceResidue(tol)
             m.setMaxIterations(20_000)
             m.solve(bd, torch.zeros(n, dtype=torch.float64, device="cuda"))  # warm-up
-            run(f"reliable_{lo_name}[{fname}]", m, A, (sv + 4) * nnz + ob + 8 * n + nvec32)
+            run(f"reliable_{lo_name}[{fname}]", m, A, 38 * n if masks else (sv + 4) * nnz + ob + 8 * n + nvec32)
             if fname == "CSR" and lo_name == "fp32":
                 ir = solvers.MixedCG()
                 ir.setMatrix(A)
@@ -552,9 +555,10 @@ def wl_cg_poisson(args):
                        "mixed_seconds": tmx, "delta": args.delta, "results": res,
                        "note": "FP64 CG = TNL's CG (stops on the preconditioned residue sqrt(r.z)/||M^-1 b||); mixed "
                                "= FP32 CG with reliable updates stopping on the FP64 true residual; GBs = bytes of "
-                               "one fused iteration (SpMV with x once + 11 vector passes) x iterations / time"})
+                               "one fused iteration (two reads of the row masks + 9 vector passes; at most 2^20 "
+                               "rows: SpMV with x once + 11 vector passes) x iterations / time"})
     out["roofline"] = roofline(mixed[best_k]["GBs_per_iteration_bytes"])
-    out["roofline"]["kernel"] = f"whole {best_k} solve (fused SpMV + vector kernels)"
+    out["roofline"]["kernel"] = f"whole {best_k} solve (fused product and vector kernels)"
     if not args.no_cpu:
         A_off, A_cols, A_vals = off, cols, vals
         per_it = _cpu_cg_per_iteration(A_off, A_cols, A_vals, b)
