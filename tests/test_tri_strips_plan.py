@@ -95,6 +95,21 @@ def test_any_plan_fits_the_ring(planner, width, lines):
         assert width < 1000 or most == 1152
 
 
+def test_no_strips_that_wait_too_long(planner):
+    """Eight chains of rows: 8 rows a step, strip after strip.  The last strip would wait
+    for all steps, longer than a wait may last by default."""
+    n = 17000000
+    row = np.arange(n, dtype=np.int64)
+    ptr = np.maximum(np.arange(n + 1) - 8, 0).astype(np.int32)
+    col = (row[8:] - 8).astype(np.int32)
+    strips = ctypes.c_int32(-1)
+    planner.strips_plan(n, ptr.ctypes.data, col.ctypes.data, 0, 1e9, ctypes.byref(strips))
+    assert strips.value == 0
+    m = 800000  # (the same, shorter)
+    planner.strips_plan(m, ptr.ctypes.data, col.ctypes.data, 0, 1e9, ctypes.byref(strips))
+    assert strips.value > 0
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
 def test_strips_are_taken_in_the_order_of_starting(tmp_path):
     """A strip waits for earlier ones, and workgroups need not start in the order of

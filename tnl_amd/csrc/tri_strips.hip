@@ -55,6 +55,9 @@ constexpr uint64_t kUnsolved = 0x7ff4dead5eed0001ull;  // a signalling NaN
 // what the model of the strip choice counts: measured on MI355X
 constexpr double kStepUs = 0.1;   // a step of the solving wave
 constexpr double kLagSteps = 22;  // a value's way to the next strip, in steps
+// The last strip may wait for its first value until all others are done, and by
+// default a wait is given up after 2^20 polls, about a second: at most 0.2 s of steps.
+constexpr double kMostSteps = 2e6;
 
 struct Shared
 {
@@ -467,7 +470,7 @@ TriStripsPlan tri_strips_plan( int64_t N, const std::vector< int32_t >& ptr, con
          rows = std::min( R, N );
       }
    }
-   if( ! rows || best * kStepUs > other_us )
+   if( ! rows || best * kStepUs > other_us || best > kMostSteps )
       return T;
    // the schedule of every strip
    const int64_t ns = ceil_div( N, rows );
