@@ -85,6 +85,36 @@ def test_near_columns_stay_resident(n):
     assert _compare(S.CG, n, _band(n, 3, np.random.default_rng(n))) <= 0.95
 
 
+@pytest.mark.parametrize("solver", ["CG", "ReliableMixedCG"])
+def test_far_stencil_runs_on_row_masks(monkeypatch, solver):
+    """Few pairs, but far ones: below 2^20 rows the masks take such a matrix too."""
+    n = 1000003
+    i = np.arange(n)
+    offs = [-300000, -250000, -200000, -150000, -100000, -50000, -20000]
+    cols = np.stack([i + o for o in offs + [0] + [-o for o in reversed(offs)]], 1)
+    keep = (cols >= 0) & (cols < n)
+    vals = np.where(cols == i[:, None], 15.0, -1.0)
+    off = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    A = tnl.SparseMatrix.from_csr(n, n, off, cols[keep].astype(np.int32), vals[keep], fmt=tnl.ELLPACK)
+    b = torch.from_numpy(np.random.default_rng(3).standard_normal(n)).cuda()
+    got = []
+    for codes in ("1", "0"):
+        monkeypatch.setenv("TNLMI_COLUMN_CODES", codes)
+        s = getattr(S, solver)()
+        if solver == "ReliableMixedCG":
+            s.setInnerMatrix(tnl.SparseMatrix(n, n, A.segments, A.values.float(), A.column_indexes))
+        else:
+            s.setPreconditioner(S.Diagonal(A))
+        s.setMatrix(A)
+        s.setConvergenceResidue(1e-10)
+        x = torch.full_like(b, 0.5)
+        assert s.solve(b, x)
+        assert S.true_residual(A, x, b) <= 1e-9
+        got.append((s.getIterations(), x))
+    assert abs(got[0][0] - got[1][0]) <= 1
+    assert float((got[0][1] - got[1][1]).norm()) <= 1e-8 * float(got[1][1].norm())
+
+
 def test_next_workgroups_columns_stay_resident():
     n = 1 << 20
     rng = np.random.default_rng(n)
