@@ -204,8 +204,10 @@ __device__ __forceinline__ void put_result( int64_t* iters, double* res, int64_t
 // solve lays out first -- column-major, so that a wave's reads are contiguous,
 // with the column as a 16-bit distance from the row.  CSR rows read in place cost a
 // wave about 20 cache lines per load, and vectors in memory an L2 round trip per
-// step.  Bound by the slots' L2 reads (10 bytes per entry) for the large systems
-// and by the workgroup's two sums (about 2 us) for the small ones.
+// step.  Bound by one CU's chain of slot reads for the large systems (16,384
+// rows: 1.2 MB an iteration, 23 us, 52 GB/s; the largest ones alone take most of a
+// batch's time, so the slots come at 4 TB/s on average over the chip) and by the
+// workgroup's two sums (about 2 us) for the small ones.
 // 1,024 diffusion systems of 256 to 16,384 rows, 1e-10: 22.4 against 77 ms (one of
 // 16,384 rows alone 23 us an iteration for its 1.2 MB); 500 of 144 to 9,216 rows
 // 8.8 against 67 ms; 1,024 of 64 to 2,304 rows 2.2 against 6.2 ms.  1,024 threads

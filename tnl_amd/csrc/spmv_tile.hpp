@@ -43,9 +43,11 @@ __device__ __forceinline__ void keep( X* __restrict__ y, int64_t r, C v, C alpha
 // loads) and stages their products after the tile's in s, so every owned row
 // is stored complete and carry is never called; every row is then summed by
 // one lane, left to right from 0.  s then holds TILE + kWholeRowMax entries.
-// Bound by memory, in fact by the three round trips of a tile (its row range,
-// its columns, values and row bounds, its x entries): all gathers of a lane, the
-// tail's too, are issued before the first product is stored.  With a wait per product, a
+// Large products are bound by memory; small ones by a tile's requests in turn, five
+// in the WHOLE form: its row range and the tail's entries, the bounds of a lane's
+// row, the end of the last row, the columns and values (which need none of these but
+// stand behind them), the x entries.  All gathers of a lane, the tail's too, are
+// issued before the first product is stored: with a wait per product, a
 // 7-point grid of 149 x 151 x 157 took 61.5 (FP32) and 78.7 us (FP64), now 51.9 and
 // 70 us (4.3 and 5.0 TB/s); 256^3 309 -> 253 and 391 -> 361 us.  The row sums' LDS
 // reads ahead of their additions, and the bounds of a lane's second row loaded
