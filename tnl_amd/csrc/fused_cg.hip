@@ -981,6 +981,12 @@ bool grid_cg_launch( const GridCg< T, X >& a, hipStream_t s )
 // row and 76 with 4.
 constexpr int kPairs = 16;
 constexpr int kPairHash = 256;
+// Below half a million rows an iteration takes the same with and without masks (5-point
+// SlicedEllpack 300^2 16.0 us either way; 900^2 19.8 against 28.4), and finding the pairs
+// costs a short solve more than it saves (0.1 of 0.29 ms).  The mixed solver would
+// collect the column codes instead, which takes longer (100 iterations on 300^2 3.9 against
+// 5.2 ms).
+constexpr int64_t kMaskRows = 1 << 19, kMaskRowsMixed = 1 << 12;
 
 template< typename T >
 struct PairDict
@@ -1480,18 +1486,16 @@ struct Stage
 // Two passes over the matrix: 0.5 + 0.6 ms for 117 M FP64 entries.
 // TNLMI_COLUMN_CODES=0 in the environment keeps the matrix as it is.
 template< typename V >
-void make_masks_v( Stage& S, hipStream_t s )
+void make_masks_v( Stage& S, PairTable* table, hipStream_t s )
 {
-   DeviceArray< PairTable > table;
-   table.allocate( 1 );
    PairTable ht;
-   TNLMI_HIP( hipMemsetAsync( table.ptr, 0xff, offsetof( PairTable, val ), s ) );
-   TNLMI_HIP( hipMemsetAsync( &table.ptr->count, 0, 2 * sizeof( int32_t ), s ) );
+   TNLMI_HIP( hipMemsetAsync( table, 0xff, offsetof( PairTable, val ), s ) );
+   TNLMI_HIP( hipMemsetAsync( &table->count, 0, 2 * sizeof( int32_t ), s ) );
    for( const unsigned grid : { 8u, 2048u } )
-      hipLaunchKernelGGL( pairs_collect< V >, dim3( grid ), dim3( kFT ), 0, s, S.v, S.cols, (const V*) S.vals, table.ptr,
+      hipLaunchKernelGGL( pairs_collect< V >, dim3( grid ), dim3( kFT ), 0, s, S.v, S.cols, (const V*) S.vals, table,
                           grid == 8 ? std::min< int64_t >( S.v.n, 8 * kFT ) : S.v.n );
    TNLMI_HIP( hipGetLastError() );
-   TNLMI_HIP( hipMemcpyAsync( &ht, table.ptr, sizeof( ht ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipMemcpyAsync( &ht, table, sizeof( ht ), hipMemcpyDeviceToHost, s ) );
    TNLMI_HIP( hipStreamSynchronize( s ) );
    if( ht.reject || ht.count > kPairs || ht.count == 0 )
       return;
@@ -1523,13 +1527,13 @@ void make_masks_v( Stage& S, hipStream_t s )
    masks->allocate( rows * ( D.count <= 8 ? 1 : 2 ) );
    if( D.count <= 8 )
       hipLaunchKernelGGL( ( pairs_encode< V, uint8_t > ), dim3( 4096 ), dim3( kFT ), 0, s, S.v, S.cols,
-                          (const V*) S.vals, D, masks->ptr, rows, &table.ptr->reject );
+                          (const V*) S.vals, D, masks->ptr, rows, &table->reject );
    else
       hipLaunchKernelGGL( ( pairs_encode< V, uint16_t > ), dim3( 4096 ), dim3( kFT ), 0, s, S.v, S.cols,
-                          (const V*) S.vals, D, (uint16_t*) masks->ptr, rows, &table.ptr->reject );
+                          (const V*) S.vals, D, (uint16_t*) masks->ptr, rows, &table->reject );
    TNLMI_HIP( hipGetLastError() );
    int32_t reject = 0;
-   TNLMI_HIP( hipMemcpyAsync( &reject, &table.ptr->reject, sizeof( reject ), hipMemcpyDeviceToHost, s ) );
+   TNLMI_HIP( hipMemcpyAsync( &reject, &table->reject, sizeof( reject ), hipMemcpyDeviceToHost, s ) );
    TNLMI_HIP( hipStreamSynchronize( s ) );
    if( reject )
       return;
@@ -1539,18 +1543,23 @@ void make_masks_v( Stage& S, hipStream_t s )
    S.evals.reset();
 }
 
-void make_masks( Stage& S, hipStream_t s )
+// scratch: a vector of the matrix's rows that the solve does not use yet
+template< typename T >
+void make_masks( Stage& S, T* scratch, hipStream_t s )
 {
+   constexpr int64_t least = sizeof( T ) == 8 ? kMaskRows : kMaskRowsMixed;
+   static_assert( least * sizeof( T ) >= sizeof( PairTable ) );
    const char* env = std::getenv( "TNLMI_COLUMN_CODES" );
-   if( S.kind != 1 || S.v.n == 0 || ( env && std::string( env ) == "0" ) )
+   if( S.kind != 1 || S.v.n < least || ( env && std::string( env ) == "0" ) )
       return;
+   PairTable* table = (PairTable*) scratch;
    switch( S.A->value_type ) {
       case TNLMI_F64:
-         return make_masks_v< double >( S, s );
+         return make_masks_v< double >( S, table, s );
       case TNLMI_F32:
-         return make_masks_v< float >( S, s );
+         return make_masks_v< float >( S, table, s );
       case TNLMI_BF16:
-         return make_masks_v< bf16 >( S, s );
+         return make_masks_v< bf16 >( S, table, s );
    }
 }
 
@@ -2004,10 +2013,12 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
       dot( n, r.ptr, r.ptr, sc.ptr + 2, w, s );
    hipLaunchKernelGGL( cg_start, dim3( 1 ), dim3( 1 ), 0, s, dev.ptr, sc.ptr + 0, sc.ptr + 1, sc.ptr + 2, R );
    TNLMI_HIP( hipGetLastError() );
+   const CgDev* h = &hs.read( dev.ptr, s );
    Stage S = make_stage( A.A, A.plan, s );
    const bool resident = grid && S.A->value_type == TNLMI_F64 && grid_takes< 16 >( S, kFar64, s );
    if( ! resident ) {
-      make_masks( S, s );
+      if( h->active )
+         make_masks( S, Ap.ptr, s );
       if( column_codes && S.kind == 1 && ! S.pairs )
          make_codes( S, s );
    }
@@ -2031,7 +2042,6 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
    // the state is double-buffered by iteration parity: iteration k reads
    // dev[k & 1] and its last kernel writes dev[(k + 1) & 1]
    int par = 0;
-   const CgDev* h = &hs.read( dev.ptr, s );
    if( resident && h->active ) {
       GridWork< double > work( n, s );
       GridCg< double, double > a{};
@@ -2174,7 +2184,7 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
       Stage S = make_stage( A_lo, nullptr, s );
       const bool resident = grid_takes< 32 >( S, A_lo->value_type == TNLMI_BF16 ? kFarBf16 : kFar32, s );
       if( S.kind == 1 && ! resident ) {
-         make_masks( S, s );
+         make_masks( S, Ap.ptr, s );
          if( ! S.pairs )
             make_codes( S, s );
       }
