@@ -1714,47 +1714,61 @@ __global__ void csr_to_ell( int64_t n, int64_t stride, int32_t w, const int32_t*
 // Ellpack kernels on the same matrix stored as Ellpack.  TNLMI_CG_CSR_COPY=0
 // in the environment keeps the one-launch CSR kernel instead, and so does a
 // device without room for the copy.
-bool csr_ell_copy( Stage& S, hipStream_t s )
+// room: memory of csr_copy_slots( A ) slots for it, or NULL (the copy has its own).
+int64_t csr_copy_slots( const tnlmi_matrix& A )  // 0: no copy is made
 {
    const char* env = std::getenv( "TNLMI_CG_CSR_COPY" );
-   if( env && std::string( env ) == "0" )
-      return false;
+   const tnlmi_segments& seg = *A.segments;
+   if( seg.format != TNLMI_CSR || A.matrix_type == TNLMI_SYMMETRIC || ( env && std::string( env ) == "0" ) )
+      return 0;
+   const int64_t n = make_view( seg ).n, slots = ceil_div( n, 64 ) * 64 * std::max( 1, seg.max_size );
+   return seg.max_size > kWholeRowMax || slots > seg.elements + seg.elements / 8 ? 0 : slots;
+}
+
+bool csr_ell_copy( Stage& S, void* room, hipStream_t s )
+{
    const tnlmi_matrix& A = *S.A;
    const tnlmi_segments& seg = *A.segments;
-   const int64_t n = S.v.n;
+   const int64_t n = S.v.n, slots = csr_copy_slots( A );
+   if( slots == 0 )
+      return false;
    const int32_t w = std::max( 1, seg.max_size );
-   const int64_t stride = ceil_div( std::max< int64_t >( n, 1 ), 64 ) * 64;
-   if( seg.max_size > kWholeRowMax || n == 0 || stride * w > seg.elements + seg.elements / 8 )
-      return false;
+   const int64_t stride = slots / w;
    const size_t vs = A.value_type == TNLMI_F64 ? 8 : A.value_type == TNLMI_F32 ? 4 : 2;
-   S.ecols = std::make_shared< DeviceArray< int32_t > >();
-   S.evals = std::make_shared< DeviceArray< char > >();
-   try {
-      S.ecols->allocate( stride * w );
-      S.evals->allocate( stride * w * (int64_t) vs );
-   }
-   catch( const Error& e ) {
-      // no room for the copy: the one-launch CSR kernel on the matrix itself
-      if( e.status != TNLMI_BAD_ALLOC )
-         throw;
-      (void) hipGetLastError();
-      S.ecols.reset();
-      S.evals.reset();
-      return false;
+   void* evals = room;
+   int32_t* ecols = (int32_t*) ( (char*) room + slots * vs );
+   if( ! room ) {
+      S.ecols = std::make_shared< DeviceArray< int32_t > >();
+      S.evals = std::make_shared< DeviceArray< char > >();
+      try {
+         S.ecols->allocate( slots );
+         S.evals->allocate( slots * (int64_t) vs );
+      }
+      catch( const Error& e ) {
+         // no room for the copy: the one-launch CSR kernel on the matrix itself
+         if( e.status != TNLMI_BAD_ALLOC )
+            throw;
+         (void) hipGetLastError();
+         S.ecols.reset();
+         S.evals.reset();
+         return false;
+      }
+      ecols = S.ecols->ptr;
+      evals = S.evals->ptr;
    }
    const dim3 grid( (unsigned) ceil_div( stride, 256 ) ), block( 256 );
    switch( A.value_type ) {
       case TNLMI_F64:
          hipLaunchKernelGGL( csr_to_ell< double >, grid, block, 0, s, n, stride, w, seg.offsets.ptr, A.column_indexes,
-                             (const double*) A.values, S.ecols->ptr, (double*) S.evals->ptr );
+                             (const double*) A.values, ecols, (double*) evals );
          break;
       case TNLMI_F32:
          hipLaunchKernelGGL( csr_to_ell< float >, grid, block, 0, s, n, stride, w, seg.offsets.ptr, A.column_indexes,
-                             (const float*) A.values, S.ecols->ptr, (float*) S.evals->ptr );
+                             (const float*) A.values, ecols, (float*) evals );
          break;
       default:
          hipLaunchKernelGGL( csr_to_ell< bf16 >, grid, block, 0, s, n, stride, w, seg.offsets.ptr, A.column_indexes,
-                             (const bf16*) A.values, S.ecols->ptr, (bf16*) S.evals->ptr );
+                             (const bf16*) A.values, ecols, (bf16*) evals );
          break;
    }
    TNLMI_HIP( hipGetLastError() );
@@ -1765,13 +1779,13 @@ bool csr_ell_copy( Stage& S, hipStream_t s )
    v.ell_width = w;
    v.ell_aligned = (int32_t) stride;
    S.v = v;
-   S.cols = S.ecols->ptr;
-   S.vals = S.evals->ptr;
-   S.storage = stride * w;
+   S.cols = ecols;
+   S.vals = evals;
+   S.storage = slots;
    return true;
 }
 
-Stage make_stage( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan, hipStream_t s )
+Stage make_stage( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan, hipStream_t s, void* room = nullptr )
 {
    Stage S;
    S.A = A;
@@ -1788,7 +1802,7 @@ Stage make_stage( const tnlmi_matrix* A, const tnlmi_spmv_plan* plan, hipStream_
       return S;
    }
    const tnlmi_segments& seg = *A->segments;
-   if( fmt == TNLMI_CSR && A->matrix_type != TNLMI_SYMMETRIC && csr_ell_copy( S, s ) ) {
+   if( fmt == TNLMI_CSR && A->matrix_type != TNLMI_SYMMETRIC && csr_ell_copy( S, room, s ) ) {
       ell_shape( S );
       return S;
    }
@@ -1909,33 +1923,32 @@ struct HostState
 namespace {
 
 // What a solve by grid_cg needs besides the solve's own arrays.
+// z goes where the residual was: a launch holds that in registers, and no
+// workgroup reads another's z after the last sum, when it is stored again.
 template< typename T >
 struct GridWork
 {
-   DeviceArray< T > z, p1;
    DeviceArray< GridSlots > slots;
    DeviceArray< int32_t > late;
    uint32_t number = 1;
-   GridWork( int64_t n, hipStream_t s )
+   explicit GridWork( hipStream_t s )
    {
-      z.allocate( n );
-      p1.allocate( n );
       slots.allocate( 1 );
       late.allocate( 1 );
       TNLMI_HIP( hipMemsetAsync( slots.ptr, 0, sizeof( GridSlots ), s ) );
       TNLMI_HIP( hipMemsetAsync( late.ptr, 0, sizeof( int32_t ), s ) );
    }
    template< typename X >
-   void fill( GridCg< T, X >& a, const Stage& S, T* p )
+   void fill( GridCg< T, X >& a, const Stage& S, T* r, T* p, T* p1 )
    {
       a.n = S.v.n;
       a.stride = S.v.ell_aligned;
       a.w = S.v.ell_width;
       a.cols = S.cols;
       a.vals = S.vals;
+      a.r = a.z = r;
       a.p[ 0 ] = p;
-      a.p[ 1 ] = p1.ptr;
-      a.z = z.ptr;
+      a.p[ 1 ] = p1;
       a.slots = slots.ptr;
       a.wait = grid_wait();
       a.number = number;
@@ -2043,16 +2056,15 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
    // dev[k & 1] and its last kernel writes dev[(k + 1) & 1]
    int par = 0;
    if( resident && h->active ) {
-      GridWork< double > work( n, s );
+      GridWork< double > work( s );
       GridCg< double, double > a{};
-      a.r = r.ptr;
       a.x = x;
       a.d = d;
       a.st = dev.ptr;
       a.R = R;
       do {
          const auto turn = resident_turn();
-         work.fill( a, S, p.ptr );
+         work.fill( a, S, r.ptr, p.ptr, Ap.ptr );
          if( ! grid_cg_launch< double, double, double, double, false >( a, s ) )
             break;
          int32_t late = 0;
@@ -2093,11 +2105,16 @@ bool fused_cg_run( const Operator& A, const tnlmi_preconditioner* M, const doubl
 
 }  // namespace
 
-bool ell_slots( const Operator& A, double far, EllSlots& out, hipStream_t s )
+int64_t ell_copy_values( const Operator& A )
 {
-   if( A.plan || A.A->value_type != TNLMI_F64 || A.rows > kGridRows )
+   return A.plan || A.A->value_type != TNLMI_F64 || A.rows > kGridRows ? 0 : ceil_div( 3 * csr_copy_slots( *A.A ), 2 );
+}
+
+bool ell_slots( const Operator& A, double far, double* room, EllSlots& out, hipStream_t s )
+{
+   if( A.plan || A.A->value_type != TNLMI_F64 || A.rows > kGridRows || ( ! room && ell_copy_values( A ) > 0 ) )
       return false;
-   const Stage S = make_stage( A.A, nullptr, s );
+   const Stage S = make_stage( A.A, nullptr, s, room );
    if( ! grid_takes< 16 >( S, far, s ) )
       return false;
    out.n = S.v.n;
@@ -2105,8 +2122,6 @@ bool ell_slots( const Operator& A, double far, EllSlots& out, hipStream_t s )
    out.w = S.v.ell_width;
    out.cols = S.cols;
    out.vals = (const double*) S.vals;
-   out.own_cols = S.ecols;
-   out.own_vals = S.evals;
    return true;
 }
 
@@ -2204,7 +2219,7 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
       int par = 0;  // the state is double-buffered by iteration parity
       std::unique_ptr< GridWork< float > > grid;
       if( resident )
-         grid = std::make_unique< GridWork< float > >( n, s );
+         grid = std::make_unique< GridWork< float > >( s );
       while( true ) {
          // reliable update: r = b - A x in FP64 and the true residual
          op.apply( d_x, r64.ptr, s );
@@ -2230,7 +2245,6 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
          int32_t late = 0;
          if( grid ) {
             GridCg< float, float > a{};
-            a.r = r.ptr;
             a.x = xc.ptr;
             a.d = d32.ptr;
             a.st = cur;
@@ -2240,7 +2254,7 @@ tnlmi_status tnlmi_mixed_cg_solve( const tnlmi_matrix* A, const tnlmi_matrix* A_
             a.maxit = R.maxit;
             do {
                const auto turn = resident_turn();
-               grid->fill( a, S, p.ptr );
+               grid->fill( a, S, r.ptr, p.ptr, Ap.ptr );
                const bool launched = A_lo->value_type == TNLMI_F32
                                         ? grid_cg_launch< float, float, float, float, true >( a, s )
                                         : grid_cg_launch< bf16, float, float, float, true >( a, s );

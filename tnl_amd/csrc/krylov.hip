@@ -1446,7 +1446,19 @@ void gmres_solve( const Operator& A, const tnlmi_preconditioner* M, const double
    const bool pre = M && M->kind != TNLMI_PRECOND_NONE;
    GLayout L( rmax );
    DeviceArray< double > V, r, wv, tmp, g;
-   V.allocate( ld * ( rmax + 1 ) );
+   // (V also has room for a copy of the matrix, where one is made)
+   const bool resident = variant != 4 && ! inner && ( ! pre || M->kind == TNLMI_PRECOND_DIAGONAL );
+   int64_t copied = resident ? ell_copy_values( A ) : 0;
+   try {
+      V.allocate( ld * ( rmax + 1 ) + copied );
+   }
+   catch( const Error& ) {
+      if( copied == 0 )
+         throw;
+      (void) hipGetLastError();
+      copied = 0;
+      V.allocate( ld * ( rmax + 1 ) );
+   }
    r.allocate( n );
    wv.allocate( n );
    tmp.allocate( n );
@@ -1524,9 +1536,9 @@ void gmres_solve( const Operator& A, const tnlmi_preconditioner* M, const double
    };
    // whole cycles in one resident launch, where the matrix and preconditioner allow
    ResidentGmres q{};
-   if( ! cwy && ! inner && ( ! pre || M->kind == TNLMI_PRECOND_DIAGONAL ) && S.check()
-       && ell_slots( A, std::numeric_limits< double >::infinity(), q.A, s ) ) {
-      auto work = resident_work( n, s );
+   if( resident && S.check()
+       && ell_slots( A, std::numeric_limits< double >::infinity(), copied ? V.ptr + ld * ( rmax + 1 ) : nullptr, q.A, s ) ) {
+      auto work = resident_work( wv.ptr, tmp.ptr, s );
       q.d = precond_diagonal( M );
       q.b = b;
       q.r = r.ptr;

@@ -100,11 +100,14 @@ struct EllSlots
    int32_t w = 0;
    const int32_t* cols = nullptr;
    const double* vals = nullptr;
-   std::shared_ptr< void > own_cols, own_vals;
 };
+// how many doubles the copy takes (0: none is made).  It has a place in a work array
+// of the solve: an allocation of its own, of more than 64 MB, would take 0.3 ms
+int64_t ell_copy_values( const Operator& A );
 // false: the matrix has no such slots, more rows than a resident launch takes, or
 // more lines * rows of far columns than `far` (fused_cg.hip)
-bool ell_slots( const Operator& A, double far, EllSlots& out, hipStream_t s );
+// room: ell_copy_values( A ) doubles, or NULL (then no copy is made)
+bool ell_slots( const Operator& A, double far, double* room, EllSlots& out, hipStream_t s );
 
 // BiCGStab's iterations from an admitted one on (sc: the solver's scalars).
 // Returns what ended them, or kResidentNot when nothing was launched.
@@ -125,7 +128,8 @@ struct ResidentBicgstab
    double b_norm, eps2;
 };
 class Resident;  // work space of a solve
-std::shared_ptr< Resident > resident_work( int64_t n, hipStream_t s );
+// pub0, pub1: n values each that the solve does not use otherwise
+std::shared_ptr< Resident > resident_work( double* pub0, double* pub1, hipStream_t s );
 ResidentEnd resident_bicgstab( Resident& w, const ResidentBicgstab& a, Stop& S, hipStream_t s );
 
 struct ResidentGmres

@@ -136,14 +136,35 @@ void bicgstab_solve( const Operator& A, const tnlmi_preconditioner* M, bool exac
                      tnlmi_solver_state* st, hipStream_t s )
 {
    const int64_t n = A.rows;
-   DeviceArray< double > r, rast, p, pn, s_, Ap, As, tmp, sc;
-   for( auto* a : { &r, &rast, &p, &pn, &s_, &Ap, &As, &tmp } )
-      a->allocate( std::max< int64_t >( 1, n ) );
+   const bool pre = M && precond_kind( M ) != TNLMI_PRECOND_NONE;
+   const bool resident = ! exact && ( ! pre || precond_kind( M ) == TNLMI_PRECOND_DIAGONAL );
+   DeviceArray< double > all, sc;
+   struct Vector
+   {
+      double* ptr;
+   } r, rast, p, pn, s_, Ap, As, tmp;
+   // one array for all, with room for a copy of the matrix where one is made
+   const int64_t ld = ceil_div( std::max< int64_t >( 1, n ), 32 ) * 32;
+   int64_t copied = resident ? ell_copy_values( A ) : 0;
+   try {
+      all.allocate( 8 * ld + copied );
+   }
+   catch( const Error& ) {
+      if( copied == 0 )
+         throw;
+      (void) hipGetLastError();
+      copied = 0;
+      all.allocate( 8 * ld );
+   }
+   double* next = all.ptr;
+   for( auto* v : { &r, &rast, &p, &pn, &s_, &Ap, &As, &tmp } ) {
+      v->ptr = next;
+      next += ld;
+   }
    sc.allocate( kBsSlots );
    RedWork w;
    HostScalars hs;
    Stop S{ st };
-   const bool pre = M && precond_kind( M ) != TNLMI_PRECOND_NONE;
    // the norm of the preconditioned right-hand side (BICGStab.hpp:47-53)
    if( pre ) {
       precond_apply( M, n, b, tmp.ptr, s );
@@ -175,13 +196,12 @@ void bicgstab_solve( const Operator& A, const tnlmi_preconditioner* M, bool exac
       hipLaunchKernelGGL( bs_restart, dim3( 1 ), dim3( 1 ), 0, s, sc.ptr );
       hipLaunchKernelGGL( bs_dir, vg( n ), dim3( 256 ), 0, s, n, r.ptr, p.ptr, Ap.ptr, pn.ptr, sc.ptr );
    };
-   const bool jacobi = pre && precond_kind( M ) == TNLMI_PRECOND_DIAGONAL;
    ResidentBicgstab q{};
    // far columns: 1,000,000 rows of 6 random ones 212 us an iteration, launch by launch 210;
    // of 12 337 and 318; 524,288 rows are faster in the resident launch at any width
    const double far = n > ( 1 << 19 ) ? 4e12 : std::numeric_limits< double >::infinity();
-   if( ! exact && ( ! pre || jacobi ) && ell_slots( A, far, q.A, s ) ) {
-      auto work = resident_work( n, s );
+   if( resident && S.check() && ell_slots( A, far, copied ? next : nullptr, q.A, s ) ) {
+      auto work = resident_work( s_.ptr, As.ptr, s );
       q.d = precond_diagonal( M );
       q.rast = rast.ptr;
       q.r = r.ptr;

@@ -28,18 +28,18 @@ namespace tnlmi {
 class Resident
 {
 public:
-   DeviceArray< double > pub[ 2 ];  // vectors that every workgroup reads
+   double* pub[ 2 ];  // vectors that every workgroup reads
    DeviceArray< GridSlots > slots;
    DeviceArray< ResidentState > state;
    DeviceArray< int32_t > late;  // a grid sum was given up
    uint32_t number = 1;
 };
 
-std::shared_ptr< Resident > resident_work( int64_t n, hipStream_t s )
+std::shared_ptr< Resident > resident_work( double* pub0, double* pub1, hipStream_t s )
 {
    auto w = std::make_shared< Resident >();
-   w->pub[ 0 ].allocate( n );
-   w->pub[ 1 ].allocate( n );
+   w->pub[ 0 ] = pub0;
+   w->pub[ 1 ] = pub1;
    w->slots.allocate( 1 );
    w->state.allocate( 1 );
    w->late.allocate( 1 );
@@ -648,8 +648,8 @@ void fill_common( Common& c, Resident& w, const EllSlots& A, const double* d, co
    c.cols = A.cols;
    c.vals = A.vals;
    c.d = d;
-   c.pub[ 0 ] = w.pub[ 0 ].ptr;
-   c.pub[ 1 ] = w.pub[ 1 ].ptr;
+   c.pub[ 0 ] = w.pub[ 0 ];
+   c.pub[ 1 ] = w.pub[ 1 ];
    c.slots = w.slots.ptr;
    c.st = w.state.ptr;
    c.late = w.late.ptr;
