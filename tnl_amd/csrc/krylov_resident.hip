@@ -14,7 +14,7 @@
 // against 339 us; GMRES(30) with classical Gram-Schmidt twice on 120^2 27 against
 // 84 us, on 1024^2 111 against 173 us (the basis read three times, 390 MB on
 // average, is most of it); BiCGStab on 100^2 15 against 98 us, 500^2 30 against
-// 98 us, 1024^2 74 against 125 us.  Small systems: 2 grid sums per basis vector of
+// 98 us, 1024^2 66 against 125 us.  Small systems: 2 grid sums per basis vector of
 // modified Gram-Schmidt, 5 per BiCGStab iteration, 2.2 us each.
 #include <algorithm>
 #include <type_traits>
@@ -688,11 +688,11 @@ ResidentState get_state( Resident& w, hipStream_t s )
 }  // namespace
 
 // Threads and rows per thread.  60 iterations on 450^2, 700^2 and 1000^2 grids with
-// 1,024 threads (1, 2 and 4 rows) against 512 (2, 4 and 8): BiCGStab 2.00 / 1.90, 2.82 /
-// 2.76, 4.68 / 4.44 ms; GMRES(20) CGSR 3.64 / 2.39, 4.91 / 3.83, 7.29 / 5.56 ms (the 32
-// sums of a pass spill 131 registers of 128), GMRES(10) MGSR 3.63 / 3.25, 4.12 / 3.96,
-// 5.31 / 5.32 ms.  Past 2^20 rows, launch by launch: BiCGStab 78 -> 131 us an iteration at
-// 1025^2, GMRES(20) CGSR 94 -> 157, GMRES(10) MGSR 89 -> 205.
+// 1,024 threads (1, 2 and 4 rows) against 512 (2, 4 and 8): BiCGStab 1.94 / 1.88, 2.56 /
+// 2.56, 3.98 / 3.72 ms; GMRES(20) CGSR 3.66 / 2.38, 4.87 / 3.78, 7.26 / 5.54 ms (with 128
+// registers the 32 sums of a pass spill 131), GMRES(10) MGSR 3.63 / 3.25, 4.17 / 4.03,
+// 5.39 / 5.38 ms.  Past 2^20 rows, launch by launch: BiCGStab 67 -> 123 us an iteration at
+// 1025^2, GMRES(20) CGSR 93 -> 158, GMRES(10) MGSR 91 -> 200.
 ResidentEnd resident_bicgstab( Resident& w, const ResidentBicgstab& q, Stop& S, hipStream_t s )
 {
    BicgArgs a{};
