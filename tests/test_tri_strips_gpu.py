@@ -124,3 +124,27 @@ def test_strip_solve_pivots_at_the_ends_of_the_range(monkeypatch, scale):
         monkeypatch.setenv("TNLMI_ILU_FLOW", "0")
         want = S.ILU0(A).solve(dev(rhs), torch.zeros(n, dtype=torch.float64, device="cuda")).cpu().numpy()
         np.testing.assert_array_equal(got, want)
+
+
+def test_strip_solve_in_a_graph():
+    """A captured apply, replayed with other right-hand sides and eager applies between: the
+    counter of the started strips is cleared in the graph."""
+    rng = np.random.default_rng(63)
+    off, cols, vals = _grid(65, 130, 1, rng)
+    n = len(off) - 1
+    P = S.ILU0(tnl.SparseMatrix.from_csr(n, n, off, cols, vals))
+    b, x = dev(rng.standard_normal(n)), torch.zeros(n, dtype=torch.float64, device="cuda")
+    P.solve(b, x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        P.solve(b, x)
+    for _ in range(4):
+        b.copy_(dev(rng.standard_normal(n)))
+        x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = x.clone()
+        want = P.solve(b, torch.zeros_like(x))
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
