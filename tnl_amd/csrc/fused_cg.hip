@@ -907,15 +907,21 @@ __global__ void __launch_bounds__( 1024 ) far_lines( int64_t n, int64_t stride, 
    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
    const int64_t groups = ( n + 63 ) / 64;
    const int32_t every = ( w + 31 ) / 32;  // slots
-   int32_t count = 0, slots = 0;
+   const int32_t slots = ( w + every - 1 ) / every;
+   int32_t count = 0;
    for( int g = wave; g < kFarGroups; g += 16 ) {
       const int64_t r = groups * g / kFarGroups * 64 + lane;
-      slots = 0;
-      for( int32_t k = 0; k < w; k += every, slots++ ) {
-         const int32_t c = r < n ? cols[ k * stride + r ] : -1;
-         const int32_t line = c >= 0 && abs( c / block - (int32_t) r / block ) > 1 ? c / LINE : -1;
-         const int32_t before = __shfl_up( line, 1, 64 );
-         count += line >= 0 && ( lane == 0 || line != before ) ? 1 : 0;
+      for( int32_t k0 = 0; k0 < slots; k0 += 8 ) {
+         int32_t c[ 8 ];
+#pragma unroll
+         for( int u = 0; u < 8; u++ )
+            c[ u ] = r < n && k0 + u < slots ? cols[ (int64_t) ( k0 + u ) * every * stride + r ] : -1;
+#pragma unroll
+         for( int u = 0; u < 8; u++ ) {
+            const int32_t line = c[ u ] >= 0 && abs( c[ u ] / block - (int32_t) r / block ) > 1 ? c[ u ] / LINE : -1;
+            const int32_t before = __shfl_up( line, 1, 64 );
+            count += line >= 0 && ( lane == 0 || line != before ) ? 1 : 0;
+         }
       }
    }
    count = group_sum< 64 >( count );
@@ -926,7 +932,7 @@ __global__ void __launch_bounds__( 1024 ) far_lines( int64_t n, int64_t stride, 
       double t = 0;
       for( int i = 0; i < 16; i++ )
          t += sm[ i ];
-      *out = t * ( (double) groups / kFarGroups ) * ( (double) w / max( slots, 1 ) );
+      *out = t * ( (double) groups / kFarGroups ) * ( (double) w / slots );
    }
 }
 

@@ -52,6 +52,8 @@ __device__ __forceinline__ C fetch_nt( const int32_t* __restrict__ cols, const V
 // slots and vectors); with the remainder in one batch it takes 38.7
 // us.  500,000 power-law rows of 16 entries on average in FP32: 32-row slices 570 ->
 // 288 us, BiEllpack 133 -> 95 us, ChunkedEllpack 563 -> 290 us.
+// (FP64 rows of random columns over 1,000,000 rows take 3 to 10 % longer than slot by
+// slot, 8 entries 78.3 against 70.8 us; FP32 rows and 4,000,000 rows do not.)
 // KEEP (a lane's slots are neighbours): the lines stay for the lane's next slots.
 constexpr int kSU = 8;
 
