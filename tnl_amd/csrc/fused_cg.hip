@@ -1692,24 +1692,59 @@ void ell_shape( Stage& S )
 
 // CSR rows as column-major Ellpack slots: slot j of row r at j * stride + r
 // (padding: column -1, value 0); rows [n, stride) are all padding
-template< typename V >
-__global__ void csr_to_ell( int64_t n, int64_t stride, int32_t w, const int32_t* __restrict__ off,
-                            const int32_t* __restrict__ cols, const V* __restrict__ vals, int32_t* __restrict__ ec,
-                            V* __restrict__ ev )
+//
+// Bound: both layouts' bytes.  A workgroup takes ROWS rows, whose entries are
+// contiguous in CSR, through LDS, so that the loads and the stores are both
+// coalesced.  One lane per row without LDS: a wave's loads of a slot lie w
+// entries apart, and with long rows their lines leave L1 before the next slot
+// wants them.  10^6 rows in FP64, us before -> now: of 27 entries 898 -> 116
+// (5.6 TB/s), 16: 431 -> 67, 9: 113 -> 46, 8: 88 -> 40, 5: 32 -> 26, 1: 8 -> 8;
+// Poisson 256^3 907 -> 502.  With 64 rows of up to eight entries, too, 1: 17,
+// 5: 31, Poisson 256^3 569: a short row's workgroup has more rows.
+constexpr int kCopySlots = 2048;  // of a workgroup: 24 KB of LDS in FP64
+constexpr int kCopyRows = kCopySlots / kWholeRowMax, kCopyShortRows = 256;  // kCopyShortRows: w <= kCopyShort
+constexpr int kCopyShort = kCopySlots / kCopyShortRows;
+
+// one word of padding per 32 keeps rows of 8, 16 and 32 entries off one bank
+__host__ __device__ constexpr int copy_slot( int i ) { return i + ( i >> 5 ); }
+
+template< int ROWS, typename V >
+__global__ __launch_bounds__( 256 ) void csr_to_ell( int64_t n, int64_t stride, int32_t w,
+                                                     const int32_t* __restrict__ off,
+                                                     const int32_t* __restrict__ cols, const V* __restrict__ vals,
+                                                     int32_t* __restrict__ ec, V* __restrict__ ev )
 {
-   const int64_t r = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+   __shared__ V sv[ copy_slot( kCopySlots ) ];
+   __shared__ int32_t sc[ copy_slot( kCopySlots ) ];
+   const int64_t r0 = (int64_t) blockIdx.x * ROWS, r = r0 + threadIdx.x % ROWS;
+   const int32_t first = off[ r0 < n ? r0 : n ], last = off[ r0 + ROWS < n ? r0 + ROWS : n ];
+   const int32_t b = off[ r < n ? r : n ] - first, e = off[ r < n ? r + 1 : n ] - first;
+   for( int32_t i = threadIdx.x; i < last - first; i += 256 ) {  // at most ROWS * w <= kCopySlots
+      sc[ copy_slot( i ) ] = cols[ first + i ];
+      sv[ copy_slot( i ) ] = vals[ first + i ];
+   }
+   __syncthreads();
    if( r >= stride )
       return;
-   int32_t b = 0, e = 0;
-   if( r < n ) {
-      b = off[ r ];
-      e = off[ r + 1 ];
-   }
-   for( int32_t j = 0; j < w; j++ ) {
+   for( int32_t j = threadIdx.x / ROWS; j < w; j += 256 / ROWS ) {
       const bool in = b + j < e;
-      ec[ j * stride + r ] = in ? cols[ b + j ] : -1;
-      ev[ j * stride + r ] = in ? vals[ b + j ] : V{};
+      ec[ j * stride + r ] = in ? sc[ copy_slot( b + j ) ] : -1;
+      ev[ j * stride + r ] = in ? sv[ copy_slot( b + j ) ] : V{};
    }
+}
+
+template< typename V >
+void csr_to_ell_launch( int64_t n, int64_t stride, int32_t w, const tnlmi_matrix& A, int32_t* ec, void* ev,
+                        hipStream_t s )
+{
+   if( w <= kCopyShort )
+      hipLaunchKernelGGL( ( csr_to_ell< kCopyShortRows, V > ), dim3( (unsigned) ceil_div( stride, kCopyShortRows ) ),
+                          dim3( 256 ), 0, s, n, stride, w, A.segments->offsets.ptr, A.column_indexes,
+                          (const V*) A.values, ec, (V*) ev );
+   else
+      hipLaunchKernelGGL( ( csr_to_ell< kCopyRows, V > ), dim3( (unsigned) ceil_div( stride, kCopyRows ) ),
+                          dim3( 256 ), 0, s, n, stride, w, A.segments->offsets.ptr, A.column_indexes,
+                          (const V*) A.values, ec, (V*) ev );
 }
 
 // A CSR matrix whose rows are all short (at most kWholeRowMax entries) and
@@ -1762,20 +1797,10 @@ bool csr_ell_copy( Stage& S, void* room, hipStream_t s )
       ecols = S.ecols->ptr;
       evals = S.evals->ptr;
    }
-   const dim3 grid( (unsigned) ceil_div( stride, 256 ) ), block( 256 );
    switch( A.value_type ) {
-      case TNLMI_F64:
-         hipLaunchKernelGGL( csr_to_ell< double >, grid, block, 0, s, n, stride, w, seg.offsets.ptr, A.column_indexes,
-                             (const double*) A.values, ecols, (double*) evals );
-         break;
-      case TNLMI_F32:
-         hipLaunchKernelGGL( csr_to_ell< float >, grid, block, 0, s, n, stride, w, seg.offsets.ptr, A.column_indexes,
-                             (const float*) A.values, ecols, (float*) evals );
-         break;
-      default:
-         hipLaunchKernelGGL( csr_to_ell< bf16 >, grid, block, 0, s, n, stride, w, seg.offsets.ptr, A.column_indexes,
-                             (const bf16*) A.values, ecols, (bf16*) evals );
-         break;
+      case TNLMI_F64: csr_to_ell_launch< double >( n, stride, w, A, ecols, evals, s ); break;
+      case TNLMI_F32: csr_to_ell_launch< float >( n, stride, w, A, ecols, evals, s ); break;
+      default: csr_to_ell_launch< bf16 >( n, stride, w, A, ecols, evals, s ); break;
    }
    TNLMI_HIP( hipGetLastError() );
    SegView v{};
